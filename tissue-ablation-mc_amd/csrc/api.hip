@@ -117,6 +117,8 @@ McArgs mc_args(tam_ctx* c, int64_t npackets, uint64_t seed, uint32_t stream)
     a.n_zlo = (float)c->p.n_ext_zlo;
     a.n_zhi = (float)c->p.n_ext_zhi;
     a.mut = c->mut; a.mat = c->mat; a.mtab = c->mtab;
+    a.nmat = c->nmat + 1;                  // and air
+    a.mut_by_mat = c->mut_by_mat ? 1 : 0;
     a.tally = c->tally; a.counters = c->counters;
     a.p0 = 0; a.npk = (uint64_t)npackets;
     a.key0 = (uint32_t)seed; a.key1 = (uint32_t)(seed >> 32); a.stream = stream;
@@ -683,7 +685,7 @@ int tam_set_optics(tam_ctx* c, const uint8_t* mat, const tam_material* table, in
         tab[m].albedo = mt > 0 ? (float)(t.mus / mt) : 0.f;
         tab[m].g = (float)t.g;
         tab[m].n = (float)t.n;
-        tab[m].mua = (float)t.mua;
+        tab[m].mut = (float)mt;
         tab[m].omg2 = (float)(1.0 - t.g * t.g);
         tab[m].opg2 = (float)(1.0 + t.g * t.g);
         tab[m].inv2g = t.g != 0.0 ? (float)(1.0 / (2.0 * t.g)) : 0.f;
@@ -691,7 +693,7 @@ int tam_set_optics(tam_ctx* c, const uint8_t* mat, const tam_material* table, in
         c->host_tab[m] = t;
     }
     c->air_id = nmat;                     // removed voxels: no absorption, no scattering, n = 1
-    tab[nmat].albedo = 0.f; tab[nmat].g = 0.f; tab[nmat].n = 1.f; tab[nmat].mua = 0.f;
+    tab[nmat].albedo = 0.f; tab[nmat].g = 0.f; tab[nmat].n = 1.f; tab[nmat].mut = 0.f;
     tab[nmat].omg2 = 1.f; tab[nmat].opg2 = 1.f; tab[nmat].inv2g = 0.f;
     frac[nmat] = 0.0;
     for (int m = 0; m <= nmat; ++m) {     // normal-incidence specular reflectance at the top face
@@ -713,12 +715,17 @@ int tam_set_optics(tam_ctx* c, const uint8_t* mat, const tam_material* table, in
         rhokap = rk.data();
     }
     std::vector<float> mut((size_t)V);
+    // the table model keeps mu_t per material (removed voxels become air, mu_t
+    // 0); the water model's rebuild writes its own per voxel
+    bool by_mat = c->p.thermal_mode == TAM_THERMAL_TABLE;
     for (int k = 1; k <= c->p.nz; ++k)
         for (int j = 1; j <= c->p.ny; ++j)
             for (int i = 1; i <= c->p.nx; ++i) {
                 const long v = (i - 1) + (long)c->p.nx * ((j - 1) + (long)c->p.ny * (k - 1));
                 mut[(size_t)v] = (float)rhokap[i + c->px * j + c->pxy * k];
+                by_mat &= mut[(size_t)v] == tab[mat[v]].mut;
             }
+    c->mut_by_mat = by_mat;
     HIPCHK(c, hipMemcpyAsync(c->mat, mat, (size_t)V, hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipMemcpyAsync(c->mtab, tab, sizeof(tab), hipMemcpyHostToDevice, c->stream));
     HIPCHK(c, hipMemcpyAsync(c->mua_frac, frac, sizeof(frac), hipMemcpyHostToDevice, c->stream));
@@ -1130,6 +1137,7 @@ int tam_upload(tam_ctx* c, int32_t field, const double* in)
                 for (int i = 1; i <= c->p.nx; ++i)
                     mut[(size_t)((i - 1) + (long)c->p.nx * ((j - 1) + (long)c->p.ny * (k - 1)))] =
                         (float)in[i + c->px * j + c->pxy * k];
+        c->mut_by_mat = false;                       // mu_t per voxel from here on
         HIPCHK(c, hipMemcpyAsync(c->mut, mut.data(), sizeof(float) * (size_t)V, hipMemcpyHostToDevice, c->stream));
         HIPCHK(c, hipMemcpyAsync(c->rhokap, in, sizeof(double) * (size_t)H, hipMemcpyHostToDevice, c->stream));
         HIPCHK(c, hipStreamSynchronize(c->stream));

@@ -5,11 +5,12 @@
 // inttau2.f90:7-239; HG scattering in place of stokes, stokes.f90:6-153).
 //
 // Design:
-//  * Each lane owns one packet at a time.  Packets are handed out from a
-//    queue head in device memory, a chunk per wave at a time, so waves that
-//    draw short histories take more packets and the grid drains together.
-//    The random stream of a packet depends only on its index, never on the
-//    lane or the order in which packets are taken.
+//  * Each lane owns one packet at a time.  A wave starts on its own first
+//    packets; the rest are handed out from a queue head in device memory, a
+//    chunk per wave at a time, so waves that draw short histories take more
+//    packets and the grid drains together.  The random stream of a packet
+//    depends only on its index, never on the lane or the order in which
+//    packets are taken.
 //  * Random numbers: Philox4x32-10, key = seed, counter = (packet id, event,
 //    stream).  One 4-word block per event: launch (radius, azimuth, specular
 //    test, first tau), interaction (albedo test, HG cos, HG azimuth, next
@@ -28,7 +29,18 @@
 //    takes the smallest T, adds one voxel's span on that axis to it, and
 //    steps the cell and the linear voxel index.  Scattering or a reflection
 //    starts a new segment.  Voxels with mu_t = 0 (ablated) are crossed in
-//    free flight.
+//    free flight.  Where mu_t follows from the material (the table model), a
+//    crossing loads the material's byte and takes mu_t from the table in LDS,
+//    and an event loads nothing: 8 MB instead of 40 MB of grid at 200^3, of
+//    which each XCD's 4 MB L2 holds the part under the beam.
+//  * What bounds it: issue and latency of the loop itself (with its device
+//    adds left out it takes 6-7% less); a short run, the chain of events of
+//    its longest packets.  The pass as straight code with selects, the
+//    absorbed packets' tally merged into the pass, LDS counts of rare ends,
+//    the byte loads, and no draws from a drained queue took 1e8 packets on the
+//    cratered 200^3 skin from 187 to 164-173 ms (31 device adds a packet,
+//    1.9e10/s), 3e7 on the fresh skin from 27.5 to 19.8, 1e6 at 100^3 from 7.1
+//    to 5.4 (one 1024-lane block a CU, random-phase batch 32).
 //  * Tally: path length is summed in a register while the packet stays in a
 //    voxel and written with one FP64 atomic add per voxel visit (at exit or
 //    absorption).  The absorbed fraction per voxel is mu_a * L.  Voxels with
@@ -100,13 +112,12 @@ __device__ __forceinline__ float face_dist(float o, float lo, float d, float u, 
 }
 
 constexpr uint32_t kMaxEvents = 1u << 24;   // walk steps + random events of one packet
-constexpr uint32_t kChunk = 256;            // packets a wave takes from the queue at once
 constexpr int kBoxUnitBits = 13;            // fixed-point box unit: 2^-13 of dx + dy + dz
 
-enum : int { PEND_NONE = 0, PEND_LAUNCH = 1, PEND_INTERACT = 2, PEND_FRESNEL = 3 };
+constexpr long kLdsOwn = 1024;              // LDS per block kept for the kernel's own use (counts, material table)
+constexpr int kTabMax = 64;                 // materials in the LDS of a kernel without the box
+constexpr int kBatchTab = 4;                // materials per wave in a batched block's own LDS
 
-// The transport of one instance by the calling wave's lanes, until its
-// packet queue is drained; the fate counters go to a.counters.
 // The LDS tally box of a launch: voxels [o, o + n).
 struct BoxGeom {
     int o[3], n[3];
@@ -185,43 +196,78 @@ __device__ __forceinline__ void box_carry(const McArgs& a, BT* box, BoxAdd& pa)
 __device__ __forceinline__ double box_path(uint16_t s, const McArgs& a) { return (double)s * a.box_quantum; }
 __device__ __forceinline__ double box_path(double s, const McArgs&) { return s; }
 
-template <bool BOX, class BT>
-__device__ __forceinline__ void transport(const McArgs& a, BT* box, const BoxGeom& g)
+// A packet's state in its lane.  The first two take walk passes, the next
+// three wait for the random phase.
+enum : int { ST_WALK = 0, ST_DEAD = 1, ST_LAUNCH = 2, ST_INTERACT = 3, ST_FRESNEL = 4, ST_IDLE = 5 };
+
+// Product and difference that keep their own rounding: a walk must take the
+// same steps in every kernel, so what the compiler may contract is not left
+// to the code around it.
+__device__ __forceinline__ float mul_r(float x, float y)
 {
-    unsigned long long* head = a.counters + TAM_CNT_N;     // queue head, packets taken
+#pragma clang fp contract(off)
+    return x * y;
+}
+__device__ __forceinline__ float sub_r(float x, float y)
+{
+#pragma clang fp contract(off)
+    return x - y;
+}
+
+// The transport of one instance by the calling wave's lanes, until its
+// packet queue is drained; the fate counters go to sums (TAM_CNT_N words of
+// LDS).
+// nw > 0: the launch's nw waves all start on this queue, wave `wid` with its
+// own first share of the packets; the queue head counts what is drawn after
+// those.
+// TAB: mu_t is a function of the material (McArgs.mut_by_mat) and tab is the
+// material table in LDS: a crossing then loads one byte per lane, which keeps
+// a 200^3 grid's transport in the XCDs' L2, and an event loads nothing.
+// Otherwise tab is the table in device memory and a crossing loads mu_t.
+template <bool BOX, class BT, bool TAB>
+__device__ __forceinline__ void transport(const McArgs& a, BT* box, const BoxGeom& g, const MatEntry* tab,
+                                          unsigned long long* sums, uint32_t wid, uint32_t nw)
+{
+    unsigned long long* head = a.counters + TAM_CNT_N;     // queue head, packets drawn
     const uint32_t nxy = (uint32_t)a.nx * (uint32_t)a.ny;
     const float idx_ = rcp(a.dx), idy_ = rcp(a.dy);
     const float ztop = a.dz * (float)a.nz;
     const uint32_t batch = (uint32_t)a.rng_batch;
     const uint64_t npk = a.dyn_npk ? (uint64_t)*a.dyn_npk : a.npk;
     const uint32_t stream = a.dyn_stream ? *a.dyn_stream : a.stream;
+    auto count = [&](int i) { atomicAdd(&sums[i], 1ull); };     // escapes and other rare ends
 
-    uint32_t c_abs = 0, c_spec = 0, c_miss = 0, c_cross = 0, c_inter = 0, c_kill = 0, c_tally = 0, c_box = 0;
-    uint32_t c_esc[6] = {0, 0, 0, 0, 0, 0};
+    uint32_t c_cross = 0, c_inter = 0, c_tally = 0, c_box = 0, c_abs = 0, c_spec = 0;
     BoxAdd pa{-1, 0u, 0u, 0u};
 
-    // wave-uniform queue state: packets [pool, pool_end) are this wave's
-    uint64_t pool = 0, pool_end = 0;
+    // wave-uniform queue state: packets [pool, pool_end) are this wave's.
+    // The first share, at most a packet per lane, needs no draw, and with
+    // fewer packets than lanes it spreads them over all waves.
+    const uint64_t share = nw ? (npk >= (uint64_t)nw * 64u ? 64u : (npk + nw - 1) / nw) : 0u;
+    const uint64_t queue0 = share * nw;                    // first packet the head hands out
+    const uint32_t chunk = npk >= (uint64_t)nw * 4096u ? 256u : 64u;   // packets drawn at once
+    bool dry = queue0 >= npk;                              // nothing left to draw
+    uint64_t pool = share * wid, pool_end = pool + share;
+    if (pool_end > npk) pool_end = npk > pool ? npk : pool;
 
-    bool have = false;                         // the lane holds a packet
-    int pend = PEND_NONE;
+    int st = ST_IDLE;
     uint64_t pid = 0;
     uint32_t ev = 0, nev = 0;                  // Philox event counter; steps of this packet
     int ci = 0, cj = 0, ck = 0;
     uint32_t v = 0;                            // linear voxel index of (ci, cj, ck)
     float mu = 0.f;                            // mu_t of voxel v
-    int mat = 0;                               // material of v, loaded when an event is pending
+    int mat = 0;                               // material of v (TAB; otherwise loaded when an event is pending)
     float ox = 0.f, oy = 0.f, oz = 0.f;        // segment origin, cm
     float t = 0.f;                             // distance travelled from the origin
     float Tx = 0.f, Ty = 0.f, Tz = 0.f;        // distance from the origin to the next face per axis
     float ux = 0.f, uy = 0.f, uz = -1.f;
-    float iux = 0.f, iuy = 0.f, iuz = -1.f;    // reciprocals (unused where u == 0)
+    float sx = 0.f, sy = 0.f, sz = 0.f;        // path across one voxel per axis (0 where u == 0)
     float tau = 0.f, lacc = 0.f;               // optical depth left; path in this voxel
     float nin = 1.f, nout = 1.f;               // indices at a pending Fresnel test
 
     for (;;) {
         // ---- lanes without a packet take the next ones from the queue
-        const uint64_t wm = ballot(!have);
+        const uint64_t wm = ballot(st == ST_IDLE);
         if (wm) {
             const uint32_t cnt = (uint32_t)__popcll(wm);
             const uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(wm >> 32),
@@ -229,24 +275,28 @@ __device__ __forceinline__ void transport(const McArgs& a, BT* box, const BoxGeo
             const uint64_t avail = pool_end - pool;
             uint64_t mine = pool + rank;
             if (avail < cnt) {
-                uint64_t nb = 0;
-                if (rank == 0 && !have) nb = atomicAdd(head, (unsigned long long)kChunk);
-                // the lowest lane wanting a packet is not always the lowest
-                // active lane: pass the chunk base through the wave
-                nb = __shfl(nb, (int)(__ffsll((long long)wm) - 1), 64);
-                nb = bcast_first(nb);
+                uint64_t nb = npk;
+                if (!dry) {
+                    if (rank == 0 && st == ST_IDLE) nb = queue0 + atomicAdd(head, (unsigned long long)chunk);
+                    // the lowest lane wanting a packet is not always the lowest
+                    // active lane: pass the chunk base through the wave
+                    nb = __shfl(nb, (int)(__ffsll((long long)wm) - 1), 64);
+                    nb = bcast_first(nb);
+                    // a wave's last lanes end one by one: each would draw again,
+                    // and the returning adds of all waves to the head queue up
+                    dry = nb + chunk >= npk;
+                }
                 if (rank >= avail) mine = nb + (rank - avail);
                 pool = nb + (cnt - avail);
-                pool_end = nb + kChunk;
+                pool_end = nb + chunk;
                 if (pool_end > npk) pool_end = npk > nb ? npk : nb;
                 if (pool > pool_end) pool = pool_end;
             } else {
                 pool += cnt;
             }
-            if (!have) {
+            if (st == ST_IDLE) {
                 if (mine >= npk) break;            // queue drained: this lane is done
-                have = true;
-                pend = PEND_LAUNCH;
+                st = ST_LAUNCH;
                 pid = a.p0 + mine;
                 ev = 0;
                 nev = 0;
@@ -254,16 +304,19 @@ __device__ __forceinline__ void transport(const McArgs& a, BT* box, const BoxGeo
         }
 
         const uint64_t am = ballot(true);
-        const uint64_t pm = ballot(pend != PEND_NONE);
-        if ((uint32_t)__popcll(pm) >= batch || pm == am) {
+        // `batch` of 64 lanes, in proportion where fewer are left: the wave of
+        // a draining queue does not wait for all of its last lanes
+        const uint32_t need = max(1u, ((uint32_t)__popcll(am) * batch + 32u) >> 6);
+        const uint64_t pm = ballot(st >= ST_LAUNCH);
+        if ((uint32_t)__popcll(pm) >= need || pm == am) {
             // ================= random phase: lanes with a pending event ====
-            if (pend != PEND_NONE) {
+            if (st >= ST_LAUNCH) {
                 const uint4 r = philox4x32_10(make_uint4((uint32_t)pid, (uint32_t)(pid >> 32), ev, stream),
                                               a.key0, a.key1);
                 ++ev;
-                const int kind = pend;
-                pend = PEND_NONE;
-                if (kind == PEND_LAUNCH) {
+                const int kind = st;
+                st = ST_WALK;
+                if (kind == ST_LAUNCH) {
                     // sourcephCO2 with a beam profile (sourceph.f90:7-49)
                     const float u0 = u01(r.x), u1 = u01(r.y), u2 = u01(r.z), u3 = u01(r.w);
                     const float rad = (a.beam == TAM_BEAM_TOPHAT) ? a.radius * fsqrt(u0)
@@ -280,23 +333,26 @@ __device__ __forceinline__ void transport(const McArgs& a, BT* box, const BoxGeo
                     // state is never read (voxel 0 stands in for its loads).
                     // One straight path keeps the state in its registers.
                     v = inside ? (uint32_t)ci + (uint32_t)a.nx * (uint32_t)cj + nxy * (uint32_t)ck : 0u;
-                    mu = a.mut[v];
-                    const bool spec = inside && u2 < a.mtab[a.mat[v]].rsp_top;
-                    c_miss += inside ? 0u : 1u;
+                    mat = a.mat[v];
+                    if (!TAB) mu = a.mut[v];
+                    const bool spec = inside && u2 < tab[mat].rsp_top;
                     c_spec += spec ? 1u : 0u;
-                    have = inside && !spec;
+                    if (!inside) count(TAM_CNT_MISSED);
+                    if (!inside || spec) st = ST_IDLE;
                     const float xl = (float)ci * a.dx, yl = (float)cj * a.dy;
                     ox = fminf(fmaxf(x, xl), xl + a.dx);
                     oy = fminf(fmaxf(y, yl), yl + a.dy);
                     oz = ztop;
                     ux = 0.f; uy = 0.f; uz = -1.f;
-                    iux = 0.f; iuy = 0.f; iuz = -1.f;
+                    sx = 0.f; sy = 0.f; sz = a.dz;
                     t = 0.f;
                     Tx = 3.0e38f; Ty = 3.0e38f; Tz = a.dz;
                     tau = neg_ln(u3);
                     lacc = 0.f;
                 }
-                if (kind == PEND_INTERACT) {
+                if (kind == ST_INTERACT) {
+                    const MatEntry me = tab[mat];
+                    if (TAB) mu = me.mut;
                     // interaction inside voxel v, tau / mu beyond the current point
                     const float s = tau * rcp(mu);
                     lacc += s;
@@ -306,14 +362,11 @@ __device__ __forceinline__ void transport(const McArgs& a, BT* box, const BoxGeo
                     oy = fminf(fmaxf(oy + tt * uy, yl), yl + a.dy);
                     oz = fminf(fmaxf(oz + tt * uz, zl), zl + a.dz);
                     ++c_inter;
-                    const MatEntry me = a.mtab[mat];
                     if (!(u01(r.x) < me.albedo)) {
-                        c_box += tally_add<BOX, BT>(a, box, g, v, ci, cj, ck, lacc, pa);
-                        box_carry<BT>(a, box, pa);
-                        ++c_tally;
-                        lacc = 0.f;
+                        // absorbed: the next walk pass leaves its path in the
+                        // tally and ends the packet
                         ++c_abs;
-                        have = false;
+                        st = ST_DEAD;
                     } else {
                         // Henyey-Greenstein deflection, MCML direction-cosine update
                         float ct;
@@ -324,24 +377,27 @@ __device__ __forceinline__ void transport(const McArgs& a, BT* box, const BoxGeo
                             ct = (me.opg2 - q * q) * me.inv2g;
                         }
                         ct = fminf(fmaxf(ct, -1.f), 1.f);
-                        const float st = fsqrt(1.f - ct * ct);
+                        const float st_ = fsqrt(1.f - ct * ct);
                         float sp, cp;
                         sincos_rev(u01(r.z), &sp, &cp);
                         float nx_, ny_, nz_;
                         if (fabsf(uz) > 0.99999f) {
-                            nx_ = st * cp;
-                            ny_ = st * sp;
+                            nx_ = st_ * cp;
+                            ny_ = st_ * sp;
                             nz_ = uz >= 0.f ? ct : -ct;
                         } else {
                             const float w2 = 1.f - uz * uz;
                             const float rt = __builtin_amdgcn_rsqf(w2);    // 1/sqrt(1-uz^2)
-                            nx_ = st * (ux * uz * cp - uy * sp) * rt + ux * ct;
-                            ny_ = st * (uy * uz * cp + ux * sp) * rt + uy * ct;
-                            nz_ = -st * cp * (w2 * rt) + uz * ct;
+                            nx_ = st_ * (ux * uz * cp - uy * sp) * rt + ux * ct;
+                            ny_ = st_ * (uy * uz * cp + ux * sp) * rt + uy * ct;
+                            nz_ = -st_ * cp * (w2 * rt) + uz * ct;
                         }
                         const float inv = __builtin_amdgcn_rsqf(nx_ * nx_ + ny_ * ny_ + nz_ * nz_);
                         ux = nx_ * inv; uy = ny_ * inv; uz = nz_ * inv;
-                        iux = rcp(ux); iuy = rcp(uy); iuz = rcp(uz);
+                        const float iux = rcp(ux), iuy = rcp(uy), iuz = rcp(uz);
+                        sx = mul_r(a.dx, fabsf(iux));
+                        sy = mul_r(a.dy, fabsf(iuy));
+                        sz = mul_r(a.dz, fabsf(iuz));
                         t = 0.f;
                         Tx = face_dist(ox, xl, a.dx, ux, iux);
                         Ty = face_dist(oy, yl, a.dy, uy, iuy);
@@ -349,7 +405,7 @@ __device__ __forceinline__ void transport(const McArgs& a, BT* box, const BoxGeo
                         tau = neg_ln(u01(r.w));
                     }
                 }
-                if (kind == PEND_FRESNEL) {
+                if (kind == ST_FRESNEL) {
                     // Fresnel test at a z face of the grid (the crossing is tallied)
                     const bool top = uz > 0.f;
                     if (u01(r.x) < fresnel(nin, nout, fabsf(uz))) {
@@ -362,105 +418,138 @@ __device__ __forceinline__ void transport(const McArgs& a, BT* box, const BoxGeo
                         Ty -= t;
                         t = 0.f;
                         uz = -uz;
-                        iuz = -iuz;
-                        Tz = a.dz * fabsf(iuz);
+                        Tz = sz;
                     } else {
-                        ++c_esc[top ? TAM_FACE_ZHI : TAM_FACE_ZLO];
-                        have = false;
+                        count(TAM_CNT_ESC0 + (top ? TAM_FACE_ZHI : TAM_FACE_ZLO));
+                        st = ST_IDLE;
                     }
                 }
             }
         }
         // ================= walk phase: face crossings, one per lane and
-        // pass, until `batch` lanes wait for a random event or a packet (or
+        // pass, until `need` lanes wait for a random event or a packet (or
         // every lane does).  Staying in this loop keeps the walk state in
-        // place between crossings.
+        // place between crossings.  A pass is nearly straight code: the three
+        // axes' steps are selects, and only tallies and grid faces branch.
         {
-            uint64_t sm = ballot(pend != PEND_NONE || !have);
-            while ((uint32_t)__popcll(sm) < batch && sm != am) {
-                if (pend == PEND_NONE && have) {
-                    if (++nev > kMaxEvents) {
+            uint64_t sm = ballot(st >= ST_LAUNCH);
+            while ((uint32_t)__popcll(sm) < need && sm != am) {
+                if (st < ST_LAUNCH) {
+                    if (TAB) mu = tab[mat].mut;
+                    const bool by = Ty < Tx;
+                    const float txy = by ? Ty : Tx;
+                    const bool bz = Tz < txy;
+                    const float tn = bz ? Tz : txy;
+                    const bool live = st == ST_WALK;
+                    const float s = live ? fmaxf(tn - t, 0.f) : 0.f;
+                    const float ms = mul_r(mu, s);
+                    if (nev >= kMaxEvents && live) {
                         // a packet that neither escapes nor is absorbed within
                         // kMaxEvents steps (e.g. total internal reflection in a
                         // non-absorbing slab) is abandoned, so every lane's loop ends
-                        ++c_kill;
-                        have = false;
-                    } else {
-                        int axis = 0;
-                        float tn = Tx;
-                        if (Ty < tn) { tn = Ty; axis = 1; }
-                        if (Tz < tn) { tn = Tz; axis = 2; }
-                        const float s = fmaxf(tn - t, 0.f);
-                        if (mu * s < tau) {
-                            tau -= mu * s;
-                            lacc += s;
-                            ++c_cross;
-                            // mu_t = 0 (ablated): nothing is absorbed, and the atomic
-                            // unit's throughput is what bounds this kernel
-                            if (mu > 0.f) {
-                                c_box += tally_add<BOX, BT>(a, box, g, v, ci, cj, ck, lacc, pa);
-                                ++c_tally;
-                            }
-                            lacc = 0.f;
+                        count(TAM_CNT_KILLED);
+                        st = ST_IDLE;
+                    } else if (ms < tau || !live) {
+                        // crossing (or a dead packet's last tally)
+                        ++nev;
+                        lacc += s;
+                        // mu_t = 0 (ablated): nothing is absorbed, and the atomic
+                        // unit's throughput is what bounds this kernel
+                        if (mu > 0.f) {
+                            c_box += tally_add<BOX, BT>(a, box, g, v, ci, cj, ck, lacc, pa);
+                            ++c_tally;
+                        }
+                        lacc = 0.f;
+                        if (!live) {
+                            st = ST_IDLE;
+                        } else {
+                            tau = sub_r(tau, ms);
                             t = tn;
-                            bool out = false;
-                            int face = 0;
-                            if (axis == 0) {
-                                Tx += a.dx * fabsf(iux);
-                                if (ux > 0.f) { ++ci; ++v; out = ci >= a.nx; face = TAM_FACE_XHI; }
-                                else          { --ci; --v; out = ci < 0;     face = TAM_FACE_XLO; }
-                            } else if (axis == 1) {
-                                Ty += a.dy * fabsf(iuy);
-                                if (uy > 0.f) { ++cj; v += a.nx; out = cj >= a.ny; face = TAM_FACE_YHI; }
-                                else          { --cj; v -= a.nx; out = cj < 0;     face = TAM_FACE_YLO; }
-                            } else {
-                                const bool top = uz > 0.f;
-                                if (top ? (ck == a.nz - 1) : (ck == 0)) {
+                            ++c_cross;
+                            const bool ay = by && !bz, ax = !by && !bz;
+                            const int kx = ux > 0.f ? 1 : -1, ky = uy > 0.f ? 1 : -1, kz = uz > 0.f ? 1 : -1;
+                            const bool zface = bz && (unsigned)(ck + kz) >= (unsigned)a.nz;
+                            const bool az = bz && !zface;
+                            Tx += ax ? sx : 0.f;
+                            Ty += ay ? sy : 0.f;
+                            Tz += az ? sz : 0.f;
+                            ci += ax ? kx : 0;
+                            cj += ay ? ky : 0;
+                            ck += az ? kz : 0;
+                            v += (uint32_t)(ax ? kx : (ay ? (ky > 0 ? a.nx : -a.nx) : (az ? (kz > 0 ? (int)nxy : -(int)nxy) : 0)));
+                            if (zface || (unsigned)ci >= (unsigned)a.nx || (unsigned)cj >= (unsigned)a.ny) {
+                                int face = ax ? (kx > 0 ? TAM_FACE_XHI : TAM_FACE_XLO)
+                                              : (ky > 0 ? TAM_FACE_YHI : TAM_FACE_YLO);
+                                st = ST_IDLE;
+                                if (zface) {
                                     // z face of the grid: Fresnel test where the index changes
-                                    nout = top ? a.n_zhi : a.n_zlo;
-                                    nin = a.mtab[a.mat[v]].n;
-                                    if (nout > 0.f && nout != nin) pend = PEND_FRESNEL;
-                                    else { out = true; face = top ? TAM_FACE_ZHI : TAM_FACE_ZLO; }
-                                } else {
-                                    Tz += a.dz * fabsf(iuz);
-                                    if (top) { ++ck; v += nxy; } else { --ck; v -= nxy; }
+                                    nout = kz > 0 ? a.n_zhi : a.n_zlo;
+                                    nin = tab[TAB ? mat : (int)a.mat[v]].n;
+                                    if (nout > 0.f && nout != nin) st = ST_FRESNEL;
+                                    face = kz > 0 ? TAM_FACE_ZHI : TAM_FACE_ZLO;
                                 }
-                            }
-                            if (out) {
-                                ++c_esc[face];
-                                have = false;
-                            } else if (pend == PEND_NONE) {
+                                if (st == ST_IDLE) count(TAM_CNT_ESC0 + face);
+                            } else if (TAB) {
+                                mat = a.mat[v];
+                            } else {
                                 mu = a.mut[v];
                             }
-                            box_carry<BT>(a, box, pa);
-                        } else {
-                            pend = PEND_INTERACT;
-                            mat = a.mat[v];
                         }
+                        box_carry<BT>(a, box, pa);
+                    } else {
+                        ++nev;
+                        st = ST_INTERACT;
+                        if (!TAB) mat = a.mat[v];
                     }
                 }
-                sm = ballot(pend != PEND_NONE || !have);
+                sm = ballot(st >= ST_LAUNCH);
             }
         }
     }
 
-    // ---- per-wave reduction of the fate and work counters ----------------
+    // ---- the wave's work counters ------------------------------------------
     // (lanes leave the loop one by one as the queue drains; the reduction
     // runs once every lane of the wave has left)
-    const uint32_t vals[TAM_CNT_N] = {c_abs, c_spec, c_esc[0], c_esc[1], c_esc[2], c_esc[3],
-                                      c_esc[4], c_esc[5], c_miss, c_cross, c_inter, c_kill,
-                                      c_tally, c_box};
+    const uint32_t vals[6] = {c_abs, c_spec, c_cross, c_inter, c_tally, c_box};
+    const int slot[6] = {TAM_CNT_ABSORBED, TAM_CNT_SPECULAR, TAM_CNT_CROSS, TAM_CNT_INTER, TAM_CNT_TALLY, TAM_CNT_BOX};
     const bool leader = (threadIdx.x & 63) == 0;
 #pragma unroll
-    for (int i = 0; i < TAM_CNT_N; ++i) {
+    for (int i = 0; i < 6; ++i) {
         const uint32_t w = wave_sum(vals[i]);
-        if (leader && w) atomicAdd(&a.counters[i], (unsigned long long)w);
+        if (leader && w) atomicAdd(&sums[slot[i]], (unsigned long long)w);
     }
 }
 
+// A block's counts (LDS) reach the device counters as one add each:
+// thousands of waves adding to the same few addresses would take as long as a
+// short run.
+__device__ __forceinline__ void add_counts(const McArgs& a, const unsigned long long* sums, int i)
+{
+    if (i < TAM_CNT_N && sums[i]) atomicAdd(&a.counters[i], sums[i]);
+}
+
+// the material table's first `ntab` entries into LDS, by the block's threads
+__device__ __forceinline__ void stage_table(const McArgs& a, MatEntry* tab, int ntab, int i, int n)
+{
+    const float* src = reinterpret_cast<const float*>(a.mtab);
+    float* dst = reinterpret_cast<float*>(tab);
+    for (int q = i; q < ntab * (int)(sizeof(MatEntry) / 4); q += n) dst[q] = src[q];
+}
+
+// a.ntab > 0: the launch's dynamic LDS holds that many table entries
+template <bool TAB>
 __global__ __launch_bounds__(256) void mc_kernel(McArgs a)
 {
-    transport<false, double>(a, nullptr, BoxGeom{});
+    extern __shared__ __attribute__((aligned(16))) unsigned char mc_lds[];
+    __shared__ unsigned long long sums[TAM_CNT_N];
+    MatEntry* tab = reinterpret_cast<MatEntry*>(mc_lds);
+    if (threadIdx.x < TAM_CNT_N) sums[threadIdx.x] = 0ull;
+    if (TAB) stage_table(a, tab, a.ntab, threadIdx.x, 256);
+    __syncthreads();
+    transport<false, double, TAB>(a, nullptr, BoxGeom{}, TAB ? tab : a.mtab, sums,
+                                  blockIdx.x * 4u + (threadIdx.x >> 6), gridDim.x * 4u);
+    __syncthreads();
+    add_counts(a, sums, threadIdx.x);
 }
 
 // The same with the block-private LDS tally box: cleared first, added to the
@@ -468,7 +557,8 @@ __global__ __launch_bounds__(256) void mc_kernel(McArgs a)
 // has drained the queue.  NT = 256, or 1024: one block of 16 waves per CU
 // holds one box of the CU's whole LDS instead of four quarter-size copies.
 // BT = uint16_t (16-bit fixed point, the default box) or double.
-template <int NT, class BT>
+// The material table (TAB) follows the box in the dynamic LDS.
+template <int NT, class BT, bool TAB>
 __global__ __launch_bounds__(NT) void mc_box_kernel(McArgs a)
 {
     extern __shared__ __attribute__((aligned(16))) unsigned char box_lds[];
@@ -483,11 +573,22 @@ __global__ __launch_bounds__(NT) void mc_box_kernel(McArgs a)
     }
     const int nbox = g.n[0] * g.n[1] * g.n[2];
     for (int i = threadIdx.x; i < nbox; i += NT) box[i] = (BT)0;
+    __shared__ unsigned long long sums[TAM_CNT_N];
+    MatEntry* tab = reinterpret_cast<MatEntry*>(box_lds + a.tab_off);
+    if (threadIdx.x < TAM_CNT_N) sums[threadIdx.x] = 0ull;
+    if (TAB) stage_table(a, tab, a.ntab, threadIdx.x, NT);
     __syncthreads();
-    transport<true, BT>(a, box, g);
+    transport<true, BT, TAB>(a, box, g, TAB ? tab : a.mtab, sums, blockIdx.x * (NT / 64) + (threadIdx.x >> 6),
+                             gridDim.x * (NT / 64));
     __syncthreads();
+    add_counts(a, sums, threadIdx.x);
+    // Each block starts its adds at another place of the box: blocks end
+    // together, and all of them walking the box from its start meet on the
+    // same few memory channels.
     const uint32_t nxy = (uint32_t)a.nx * (uint32_t)a.ny;
-    for (int i = threadIdx.x; i < nbox; i += NT) {
+    const int start = (int)((uint64_t)blockIdx.x * (uint32_t)nbox / gridDim.x) & ~63;
+    for (int q = threadIdx.x; q < nbox; q += NT) {
+        const int i = q + start < nbox ? q + start : q + start - nbox;
         const double s = box_path(box[i], a);
         if (s != 0.0) {
             const int bx = i % g.n[0], by = (i / g.n[0]) % g.n[1], bz = i / (g.n[0] * g.n[1]);
@@ -592,12 +693,20 @@ __global__ __launch_bounds__(256) void mc_batch_kernel(const McArgs* __restrict_
     extern __shared__ __attribute__((aligned(16))) unsigned char lds_slices[];
     // wbox is a multiple of 8, so every slice starts on a 16-byte boundary
     uint16_t* box = reinterpret_cast<uint16_t*>(lds_slices) + (size_t)(threadIdx.x >> 6) * (size_t)wbox;
+    // per wave: counts of the current instance and its material table
+    __shared__ unsigned long long wsums[4][TAM_CNT_N];
+    __shared__ __attribute__((aligned(16))) MatEntry wtab[4][kBatchTab];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
+    unsigned long long* sums = wsums[threadIdx.x >> 6];
+    MatEntry* mtl = wtab[threadIdx.x >> 6];
     for (int k = 0; k < n; ++k) {
         const int i = (wave + k) % n;
         const McArgs a = tab[i];
-        if (a.npk == 0) continue;
+        // an instance that the other waves have drained costs no box either
+        if (a.npk == 0 || __hip_atomic_load(a.counters + TAM_CNT_N, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >=
+                              a.npk)
+            continue;
         BoxGeom g{};
         if (wbox > 0 && a.box_enable) {
             // a cube of at most wbox voxels inside the grid (sd <= nx, ny; d <= nz)
@@ -614,16 +723,21 @@ __global__ __launch_bounds__(256) void mc_batch_kernel(const McArgs* __restrict_
             g.o[2] = a.nz - d;
         }
         const int nb = g.n[0] * g.n[1] * g.n[2];
-        if (nb < 8) {
-            transport<false, double>(a, nullptr, g);
-            continue;
-        }
-        for (int q = lane; q < nb; q += 64) box[q] = 0;
+        const bool small = nb < 8;                         // no box worth its clearing
+        const bool tabbed = a.mut_by_mat && a.nmat <= kBatchTab;
+        if (lane < TAM_CNT_N) sums[lane] = 0ull;
+        if (tabbed) stage_table(a, mtl, a.nmat, lane, 64);
+        if (!small)
+            for (int q = lane; q < nb; q += 64) box[q] = 0;
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");   // the zeros land before any add
         __builtin_amdgcn_wave_barrier();
-        transport<true, uint16_t>(a, box, g);
+        if (small) transport<false, double, false>(a, nullptr, g, a.mtab, sums, 0u, 0u);
+        else if (tabbed) transport<true, uint16_t, true>(a, box, g, mtl, sums, 0u, 0u);
+        else transport<true, uint16_t, false>(a, box, g, a.mtab, sums, 0u, 0u);
         __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");   // every lane's adds land before the flush
         __builtin_amdgcn_wave_barrier();
+        add_counts(a, sums, lane);
+        if (small) continue;
         const uint32_t nxy = (uint32_t)a.nx * (uint32_t)a.ny;
         for (int q = lane; q < nb; q += 64) {
             const double s = box_path(box[q], a);
@@ -684,7 +798,7 @@ hipError_t launch_mc_batch(const McArgs* dtab, int n, long total_npk, int blocks
     if (hipDeviceGetAttribute(&lds_blk, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess ||
         lds_blk <= 0)
         lds_blk = 64 * 1024;
-    const long per_block = std::min((long)lds_blk - 1024L, (long)lds_cu / bpc - 1024L);
+    const long per_block = std::min((long)lds_blk - kLdsOwn, (long)lds_cu / bpc - kLdsOwn);
     // 16-bit slots, a multiple of 8 per wave
     const int wbox = per_block > 0 ? (int)(per_block / 4 / 2) & ~7 : 0;
     const size_t lds = sizeof(uint16_t) * 4 * (size_t)wbox;
@@ -703,9 +817,14 @@ hipError_t mc_prepare(int dev)
     int lds_blk = 0;
     hipError_t e = hipDeviceGetAttribute(&lds_blk, hipDeviceAttributeMaxSharedMemoryPerBlock, dev);
     if (e != hipSuccess || lds_blk <= 64 * 1024) return e;
-    // allow the box kernels the device's whole per-block LDS (outside any graph capture)
-    const void* box_kernels[] = {(const void*)mc_box_kernel<256, uint16_t>, (const void*)mc_box_kernel<1024, uint16_t>,
-                                 (const void*)mc_box_kernel<256, double>, (const void*)mc_box_kernel<1024, double>};
+    // allow the box kernels the device's whole per-block LDS, less 1 KiB for
+    // their own use (outside any graph capture)
+    lds_blk -= kLdsOwn;
+    const void* box_kernels[] = {
+        (const void*)mc_box_kernel<256, uint16_t, false>, (const void*)mc_box_kernel<1024, uint16_t, false>,
+        (const void*)mc_box_kernel<256, double, false>,   (const void*)mc_box_kernel<1024, double, false>,
+        (const void*)mc_box_kernel<256, uint16_t, true>,  (const void*)mc_box_kernel<1024, uint16_t, true>,
+        (const void*)mc_box_kernel<256, double, true>,    (const void*)mc_box_kernel<1024, double, true>};
     for (const void* k : box_kernels) {
         e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, lds_blk);
         if (e != hipSuccess) return e;
@@ -728,17 +847,13 @@ hipError_t launch_mc(const McArgs& a, hipStream_t s)
     if (hipDeviceGetAttribute(&lds_blk, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess ||
         lds_blk <= 0)
         lds_blk = 64 * 1024;
-    // blocks_per_cu 256-lane blocks per CU (autotuned); every lane takes
-    // packets from the queue until it is empty, so more blocks than packets
-    // only idle
+    // blocks_per_cu 256-lane blocks per CU (autotuned) set the LDS box and the
+    // most blocks; runs of fewer packets launch fewer (below)
     const int bpc = a.blocks_per_cu > 0 ? a.blocks_per_cu : 8;
     // with the box on, a multiple of 4 runs as bpc / 4 blocks of 1024 lanes:
     // the same waves per CU, one box per 16 waves
     const bool wide = a.box_enable && bpc % 4 == 0;
     const int lanes = wide ? 1024 : 256, bpc_l = wide ? bpc / 4 : bpc;
-    long blocks = (long)ncu * bpc_l;
-    const long need = (long)((a.npk + lanes - 1) / lanes);
-    if (need < blocks) blocks = need;
     // LDS tally box: the resident blocks of a CU share its LDS (160 KiB on
     // MI355X, also the most one block may take), 1 KiB per block kept for
     // the kernel's own use: with 16-bit sums 42^2 x 46 voxels at 1 block per CU
@@ -760,7 +875,7 @@ hipError_t launch_mc(const McArgs& a, hipStream_t s)
     mc_box_units(b);
     b.box_n[0] = b.box_n[1] = b.box_n[2] = 0;
     b.box_geom = nullptr;
-    const long vox = std::min((long)lds_blk - 1024L, (long)lds_cu / bpc_l - 1024L) / esz;
+    const long vox = std::min((long)lds_blk - kLdsOwn, (long)lds_cu / bpc_l - kLdsOwn) / esz;
     BoxPlace bp{};
     bp.sd = std::min((int)std::cbrt((double)vox), std::min(a.nx, a.ny));
     if (fx && bp.sd > 1) bp.sd &= ~1;
@@ -777,6 +892,17 @@ hipError_t launch_mc(const McArgs& a, hipStream_t s)
         b.box_o[2] = a.nz - bp.d;
         b.box_n[0] = b.box_n[1] = bp.sd;
         b.box_n[2] = bp.d;
+        // A block's box costs a clearing and a device add per touched voxel,
+        // and waves that share a SIMD slow each other's longest packets: a
+        // block per CU from 16 packets a wave on, the further blocks of the
+        // launch shape from 1024 a wave on (100^3 cube, 8 blocks of 256 lanes a
+        // CU: 3e6 packets 12.7 ms on 256 blocks of 1024 lanes, 13.9 on 512;
+        // 1e7 39.3 on both.  Down to 16 a wave instead of 256: 140 000 packets
+        // 2.4 against 3.9 ms, 400 000 3.3 against 3.9, 1e6 5.4 on both).
+        const long wpb = lanes / 64;
+        long blocks = std::max((long)(a.npk / (uint64_t)(wpb * 1024)),
+                               std::min((long)ncu, (long)(a.npk / (uint64_t)(wpb * 16))));
+        blocks = std::max(1L, std::min(blocks, (long)ncu * bpc_l));
         const size_t lds = (size_t)esz * (size_t)bp.sd * (size_t)bp.sd * (size_t)bp.d;
         if (a.box_psum && a.box_geom) {
             hipLaunchKernelGGL(box_plane_kernel, dim3((unsigned)a.nz), dim3(256), 0, s, a.tally, a.mut, a.nx, a.ny,
@@ -788,19 +914,49 @@ hipError_t launch_mc(const McArgs& a, hipStream_t s)
             const hipError_t ef = launch_fill_f64(a.tally, nvox, 0.0, s);
             if (ef != hipSuccess) return ef;
         }
+        // the material table goes behind the box where that keeps the resident
+        // blocks: LDS is given out in steps of lds_cu / 128
+        const size_t tab_off = (lds + 15) & ~(size_t)15, tab_lds = tab_off + sizeof(MatEntry) * (size_t)a.nmat;
+        const size_t step = (size_t)lds_cu / 128;
+        const bool tab = a.mut_by_mat && tab_lds + sizeof(unsigned long long) * TAM_CNT_N <= lds + (size_t)kLdsOwn &&
+                         (tab_lds + sizeof(unsigned long long) * TAM_CNT_N + step - 1) / step * step * (size_t)bpc_l <=
+                             (size_t)lds_cu;
+        b.ntab = tab ? a.nmat : 0;
+        b.tab_off = (int)tab_off;
+#define TAM_BOX(NT_, BT_)                                                                                          \
+    do {                                                                                                           \
+        if (tab)                                                                                                   \
+            hipLaunchKernelGGL((mc_box_kernel<NT_, BT_, true>), dim3((unsigned)blocks), dim3(NT_), tab_lds, s, b); \
+        else hipLaunchKernelGGL((mc_box_kernel<NT_, BT_, false>), dim3((unsigned)blocks), dim3(NT_), lds, s, b);   \
+    } while (0)
         if (fx) {
-            if (wide) hipLaunchKernelGGL((mc_box_kernel<1024, uint16_t>), dim3((unsigned)blocks), dim3(1024), lds, s, b);
-            else hipLaunchKernelGGL((mc_box_kernel<256, uint16_t>), dim3((unsigned)blocks), dim3(256), lds, s, b);
+            if (wide) TAM_BOX(1024, uint16_t);
+            else TAM_BOX(256, uint16_t);
         } else {
-            if (wide) hipLaunchKernelGGL((mc_box_kernel<1024, double>), dim3((unsigned)blocks), dim3(1024), lds, s, b);
-            else hipLaunchKernelGGL((mc_box_kernel<256, double>), dim3((unsigned)blocks), dim3(256), lds, s, b);
+            if (wide) TAM_BOX(1024, double);
+            else TAM_BOX(256, double);
         }
+#undef TAM_BOX
     } else {
         if (a.clear_tally) {
             const hipError_t ef = launch_fill_f64(a.tally, nvox, 0.0, s);
             if (ef != hipSuccess) return ef;
         }
-        hipLaunchKernelGGL(mc_kernel, dim3((unsigned)blocks), dim3(256), 0, s, b);
+        // A short run takes as long as its longest packet's chain of events,
+        // and a wave's pass costs the same for 4 lanes as for 64: up to 8
+        // waves a CU (2 per SIMD) share fewer than 64 packets each, down to
+        // 4; past that every wave starts with a full set of lanes.  20 000
+        // packets at 64^3: 1.35 ms, against 2.7 ms on full waves alone
+        // (1.6 at 4 waves a CU, 1.35 at 16); 125 000 packets of a pure
+        // absorber: 40 us, against 68 (44 at 16 waves a CU).
+        const long waves = std::max((long)((a.npk + 63) / 64), std::min(8L * ncu, (long)((a.npk + 3) / 4)));
+        const long blocks = std::min((long)ncu * bpc, (waves + 3) / 4);
+        const bool tab = a.mut_by_mat && a.nmat <= kTabMax;
+        b.ntab = tab ? a.nmat : 0;
+        if (tab)
+            hipLaunchKernelGGL((mc_kernel<true>), dim3((unsigned)blocks), dim3(256), sizeof(MatEntry) * (size_t)a.nmat,
+                               s, b);
+        else hipLaunchKernelGGL((mc_kernel<false>), dim3((unsigned)blocks), dim3(256), 0, s, b);
     }
     return hipGetLastError();
 }

@@ -81,7 +81,7 @@ __device__ __forceinline__ unsigned thres_chain(double* thres, uint8_t* tmask, l
 
 
 struct MatEntry {          // per material, in device memory
-    float albedo, g, n, mua;
+    float albedo, g, n, mut;
     // Henyey-Greenstein constants and the specular reflectance of the top face
     float omg2;            // 1 - g^2
     float opg2;            // 1 + g^2
@@ -99,6 +99,9 @@ struct McArgs {
     const float* mut;          // interior mu_t, cm^-1
     const uint8_t* mat;        // interior material ids
     const MatEntry* mtab;
+    int nmat;                  // entries of mtab in use, air included
+    int mut_by_mat;            // every voxel's mu_t is its material's mtab[].mut
+    int ntab, tab_off;         // material table in LDS: entries and byte offset (set by launch_mc)
     double* tally;             // interior path length, cm
     unsigned long long* counters;   // TAM_CNT_*
     uint64_t p0, npk;
@@ -258,6 +261,7 @@ struct tam_ctx {
     long nvox, nhalo, px, pxy;
     int nmat, air_id;
     bool optics_set, thermal_set, src_valid;
+    bool mut_by_mat;            // mut[v] == mtab[mat[v]].mut for every voxel
     // device arrays
     float *dT0, *dT1, *gx, *gy, *gz, *src;
     float *cur, *nxt;           // current / next temperature buffer (ping-pong)
