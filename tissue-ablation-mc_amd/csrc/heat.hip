@@ -26,6 +26,8 @@
 // the owned tile, handed to the second through LDS.
 #include "tam_internal.h"
 
+#include <type_traits>
+
 namespace {
 
 __device__ __forceinline__ double wave_sum_d(double v)
@@ -507,56 +509,105 @@ __global__ __launch_bounds__(TX* TY) void stencil_direct_kernel(const HeatArgs a
     direct_body<TX, TY, LUT>(a, Tin, Tout, lon, t_after, kz, flags, xcd_tile(), (int)gridDim.x, (int)gridDim.y);
 }
 
+// What the two-step kernels' damage integral reads, in LDS: as kernel arguments
+// these stay in scalar registers through the whole march, which spill.
+struct DamageConst {
+    double t_ref, Tlo, Thi, lnA, dE, Rg, delt, thr_min, thr0, thr1, thr2, t_after[2];
+    float lo_test, hi_test;
+};
+
 // One step's damage at interior voxel v, dT = tn after the step
 // (3dFD.f90:450-461, the same arithmetic as the one-step kernels).  Omega and
-// the threshold mask are loaded on first use (from the prefetch when pom)
-// and kept in registers across the two steps of a launch; `dirty` says that
-// Omega changed and must be stored.  Outside the window the chain runs only
-// where a time is due (`due`: from the class byte for the launch's first
-// step, from the first step's chain for the second).  Returns whether a time
-// is still due after the step.
-__device__ __forceinline__ bool damage_step(const HeatArgs& a, long v, long nv, float tn, double t_after, bool due,
-                                            bool pom, double om_pf, unsigned tm_pf, double& om, bool& have,
-                                            bool& dirty, unsigned& m, bool& have_m)
+// the threshold mask stay in om and m across the two steps of a launch;
+// `dirty` says that Omega changed and must be stored.  Outside the window the
+// chain runs only where a time is due (`due`: from the class byte for the
+// launch's first step, from the first step's chain for the second).  Returns
+// whether a time is still due after the step.
+__device__ __forceinline__ bool damage_step(const DamageConst& d, double* thres, uint8_t* tmask, long v, long nv,
+                                            float tn, double t_after, bool due, double& om, bool& dirty, unsigned& m)
 {
     bool chain = due;                      // outside the window: only where a time is due
-    if (tn >= a.dT_lo_test && tn < a.dT_hi_test) {
-        const double T = a.t_ref + (double)tn;
-        if (T >= a.arr_Tlo && T < a.arr_Thi) {
-            const float arg = (float)(a.lnA - a.arr_dE / (a.arr_R * T));
-            if (!have) {
-                om = pom ? om_pf : a.omega[v];
-                have = true;
-            }
-            om = om + a.delt * (double)expf(arg);
+    if (tn >= d.lo_test && tn < d.hi_test) {
+        const double T = d.t_ref + (double)tn;
+        if (T >= d.Tlo && T < d.Thi) {
+            const float arg = (float)(d.lnA - d.dE / (d.Rg * T));
+            om = om + d.delt * (double)expf(arg);
             dirty = true;
-            chain = om >= a.thr_min;
+            chain = om >= d.thr_min;
         }
     }
     if (!chain) return false;
-    if (!have) {
-        om = pom ? om_pf : a.omega[v];
-        have = true;
-    }
-    if (!have_m) {
-        m = pom ? tm_pf : a.tmask[v];
-        have_m = true;
-    }
-    m = thres_chain(a.thres, a.tmask, v, nv, om, a.thr0, a.thr1, a.thr2, t_after, m);
+    m = thres_chain(thres, tmask, v, nv, om, d.thr0, d.thr1, d.thr2, t_after, m);
     return (m & TAM_TMASK_DUE) != 0u;
+}
+
+// A plane's base address, opaque to the optimiser: it stays a scalar, and the
+// loads take it with a 32-bit lane offset (strength reduction would make it a
+// 64-bit pointer per lane, advanced by vector adds).  The address space is
+// named because the optimiser cannot see through the barrier: a flat access
+// would also count as an LDS access, and every LDS wait would wait for it.
+template <class T>
+using Global = T __attribute__((address_space(1)))*;
+template <class T>
+__device__ __forceinline__ Global<T> plane(T* base, long cells)
+{
+    Global<T> q = (Global<T>)(base + cells);
+    asm volatile("" : "+s"(q));
+    return q;
+}
+template <class T>
+__device__ __forceinline__ T ld(Global<const T> base, unsigned index)
+{
+    return *(Global<const T>)((Global<const char>)base + index * (unsigned)sizeof(T));
+}
+template <class T>
+__device__ __forceinline__ void st(Global<T> base, unsigned index, T value)
+{
+    *(Global<T>)((Global<char>)base + index * (unsigned)sizeof(T)) = value;
+}
+
+// a value that every lane holds alike, as a scalar (an instance's arguments
+// come from device memory in the batched kernels)
+__device__ __forceinline__ int uni(int x) { return __builtin_amdgcn_readfirstlane(x); }
+template <class T>
+__device__ __forceinline__ T* uni(T* q)
+{
+    const uint64_t b = (uint64_t)q;
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)b), hi = __builtin_amdgcn_readfirstlane((uint32_t)(b >> 32));
+    return (T*)(((uint64_t)hi << 32) | lo);
 }
 
 // Two steps per launch (temporal blocking), class mode without boiling.
 //
 // A TX x TY block covers a footprint of TX x TY columns and owns the inner
 // (TX-2) x (TY-2) of them.  Marching up z, it computes the first step on
-// every footprint column (x-y neighbours loaded directly, as in direct_body),
-// hands each first-step plane to the second step through a double-buffered
-// LDS plane (one barrier per plane), and computes the second step one plane
-// behind on the owned columns.  The intermediate field never reaches HBM:
-// per two steps a voxel's dT is read and written once, its class and source
-// read once, Omega read and written at most once.  The footprint ring
-// repeats first-step work: TX*TY / ((TX-2)*(TY-2)) in x-y, (kz+2)/kz in z.
+// every footprint column, hands each first-step plane to the second step
+// through a double-buffered LDS plane (one barrier per plane), and computes
+// the second step one plane behind on the owned columns.  The intermediate
+// field never reaches HBM: per two steps a voxel's dT is read and written
+// once, its class and source read once, Omega read and written at most once.
+// The footprint ring repeats first-step work: TX*TY / ((TX-2)*(TY-2)) in x-y,
+// (kz+2)/kz in z.
+//
+// What bounds it is not HBM (about 1.9 TB/s of 5.2) but the instructions and
+// the L1 accesses that a wave has between two barriers, so both are kept few:
+// - dT before the first step goes through LDS too: a lane loads its own column
+//   and, on the footprint's edge, the one outside it; four loads per lane and
+//   plane from rows that straddle cache lines were 40 % of the L1 accesses.
+// - A plane's address is a scalar and a lane adds a 32-bit offset; the loads
+//   are global ones (a flat load also counts as an LDS access).
+// - The face coefficients of the first step at a plane are kept for the second.
+//   Where a wave is inside one class they are one 16-byte LDS read.
+// - Both steps share one test of the damage window on the larger and the
+//   smaller dT; the exact tests follow inside.  Loads of the next plane go out
+//   after the class loads of mixed waves, which would otherwise wait for them
+//   (loads return in order).
+// us a step, before and after: 200^3 skin, late state, 32x16 kz 8: 39.4, 34.3
+// (without damage 31.0, 25.7); 256^3 kz 16: 80.3, 69.6; 113x97x101 kz 4: 7.6,
+// 6.7.  VALU instructions per wave and plane 157, 110; L1 accesses 12.8e6,
+// 8.4e6 a launch at 200^3.  At most 64 VGPRs (8 waves a SIMD) gave 66.9 at 256^3
+// but 35.6 and 7.2 at the other two; two copies of the loop body with the
+// registers renamed instead of moved gave nothing.
 //
 // Both steps use the one-step kernels' face coefficients (they only change in
 // the rebuild) and arithmetic, in the same order, so the field, Omega and
@@ -573,173 +624,214 @@ __device__ __forceinline__ void t2_body(const HeatArgs& a, const float* __restri
     constexpr int OX = TX - 2, OY = TY - 2;
     __shared__ float sLut[3 * 256 + 16];
     __shared__ float2 sRob[16];
-    __shared__ float sT1[2][TY][TX];            // first-step plane, buffer = plane parity
-    const uint8_t* __restrict__ cla = a.cls;
-    const float* __restrict__ srca = a.src;
-    const long px = a.px, pxy = a.pxy;
-    const int nx = a.nx, ny = a.ny, nz = a.nz;
+    __shared__ DamageConst sDmg;
+    // dT before the first step (with one ring of columns around the footprint)
+    // and after it, buffer = plane parity
+    constexpr int P = TX + 2, PLANE = P * (TY + 2);
+    __shared__ float sT0[2 * PLANE], sT1[2 * PLANE];
+    __shared__ float4 sHom[16];                  // face coefficients between voxels of one class
+    const int nx = uni(a.nx), ny = uni(a.ny), nz = uni(a.nz);
+    const int px = nx + 2;
+    const long pxy = (long)px * (ny + 2);
+    Tin = uni(Tin);
+    Tout = uni(Tout);
+    const float* src = uni(a.src);
+    uint8_t* cls = uni(a.cls);
+    double* omega = uni(a.omega);
+    uint8_t* tmask = uni(a.tmask);
     const int tx = threadIdx.x % TX, ty = threadIdx.x / TX;
     const int i = tl.x * OX + tx, j = tl.y * OY + ty;            // footprint column; 0 and n+1 are halo
     const bool real = i >= 1 && i <= nx && j >= 1 && j <= ny;    // the first step updates this column
     const bool own = real && tx >= 1 && tx <= TX - 2 && ty >= 1 && ty <= TY - 2;
-    const bool bnd_ij = i == 1 || i == nx || j == 1 || j == ny;
-    // dT and class of the lane's own column (a halo column for lanes outside the grid)
-    const long ch = (long)min(i, nx + 1) + px * min(j, ny + 1);
-    // x-y neighbours and source: the nearest interior column, so every address
-    // is valid; lanes that are not `real` discard what they compute from them
-    const long ci = (long)min(max(i, 1), nx) + px * min(max(j, 1), ny);
+    // dT, class and source of the lane's own column (a halo column for lanes outside the grid)
+    unsigned ch = (unsigned)(min(i, nx + 1) + px * min(j, ny + 1));
+    // lanes on the footprint's edge also fetch the column outside it
+    const bool ring = tx == 0 || tx == TX - 1 || ty == 0 || ty == TY - 1;
+    const int ox = tx == 0 ? -1 : tx == TX - 1 ? 1 : 0;
+    const int oy = ox != 0 ? 0 : ty == 0 ? -1 : ty == TY - 1 ? 1 : 0;
+    unsigned co = (unsigned)(max(min(i + ox, nx + 1), 0) + px * max(min(j + oy, ny + 1), 0));
+    // the nearest interior column, for the classes around it
+    const unsigned ci = (unsigned)(min(max(i, 1), nx) + px * min(max(j, 1), ny));
+    // Omega and the threshold mask have no halo
+    const long nxy = (long)nx * ny;
+    unsigned vc = (unsigned)(max(min(i, nx), 1) - 1 + nx * (max(min(j, ny), 1) - 1));
     const int k0 = tl.z * kz + 1;
     const int k1 = min(k0 + kz, nz + 1);
     const bool robin = flags & F_ROBIN, damage = flags & F_DAMAGE;
     const bool energy = (flags & F_ENERGY) &&
                         (tl.x == 0 || tl.x == gx - 1 || tl.y == 0 || tl.y == gy - 1 || k0 == 1 || k1 == nz + 1);
+    const bool bnd_ij = i == 1 || i == nx || j == 1 || j == ny;
     for (int t = threadIdx.x; t < 3 * 256 + 16; t += TX * TY) sLut[t] = a.glut[t];
-    if (threadIdx.x < 16) sRob[threadIdx.x] = a.robin_lut[threadIdx.x];
-    __syncthreads();
-
-    const long nxy = (long)nx * ny, nv = nxy * nz;
-    const long vcol = (long)(i - 1) + (long)nx * (j - 1);        // interior index of the column (own lanes)
+    if (threadIdx.x < 16) {
+        sRob[threadIdx.x] = a.robin_lut[threadIdx.x];
+        const int d = threadIdx.x * 17;
+        sHom[threadIdx.x] = float4{a.glut[d], a.glut[256 + d], a.glut[512 + d], 0.f};
+    }
+    if (threadIdx.x == 0)
+        sDmg = DamageConst{a.t_ref, a.arr_Tlo, a.arr_Thi, a.lnA, a.arr_dE, a.arr_R, a.delt, a.thr_min, a.thr0, a.thr1,
+                           a.thr2, {ta0, ta1}, a.dT_lo_test, a.dT_hi_test};
+    // where Omega and the mask are fetched ahead: the damage window, wider by
+    // what a step may change dT
     const float wlo = a.dT_lo_test - a.dT_win_pad, whi = a.dT_hi_test + a.dT_win_pad;
-    // first step at plane p: dT0 at p-1, p (z0m, z0c), classes at p-1, p
+    // the laser states as VGPRs: a scalar operand halves the rate of an FP32 instruction
+    asm volatile("" : "+v"(lon0), "+v"(lon1));
+
+    // first step at plane p: dT0 at p-1, p (z0m, z0c), class byte at p
     int p = k0 - 1;
-    float z0m = p >= 1 ? Tin[ch + pxy * (p - 1)] : 0.f;
-    float z0c = Tin[ch + pxy * p];
-    int cm = p >= 1 ? cla[ch + pxy * (p - 1)] & TAM_CLASS_MASK : 0;
-    unsigned ccr = cla[ch + pxy * p];
-    // second step at plane k = p-1: dT1 at k-1, k (u1m, u1c) and the first
-    // step's face coefficients, source and class at k
-    float u1m = 0.f, u1c = 0.f;
-    float Gxm = 0.f, Gxp = 0.f, Gym = 0.f, Gyp = 0.f, Gzm = 0.f, Gzp = 0.f, Sk = 0.f;
-    int Ck = 0;
-    unsigned Ckr = 0;                                         // raw class byte at k (TAM_CLASS_DUE)
-    float e_acc = 0.f;
-    // loads of plane q (x-y neighbours, source) and of the column at q+1,
-    // issued one iteration ahead of their use
-    float n_z0p = 0.f, n_txm = 0.f, n_txp = 0.f, n_tym = 0.f, n_typ = 0.f, n_s = 0.f;
-    unsigned n_cpr = 0;
+    float z0m = ld<float>(plane(Tin, pxy * max(p - 1, 0)), ch);
+    float z0c = ld<float>(plane(Tin, pxy * p), ch);
+    unsigned ccr = ld<uint8_t>(plane((const uint8_t*)cls, pxy * p), ch);
+    // second step at plane k = p-1: dT1 at k-1, k (u1m, u1c), k's source, class
+    // byte and face coefficients
+    float u1m = 0.f, u1c = 0.f, Sk = 0.f;
+    float G[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    unsigned Ckr = 0;
+    float e_acc = 0.f, tmin = 3.4e38f;
+    const int slot = (ty + 1) * P + tx + 1;                     // the lane's place in a plane
+    const int oslot = slot + ox + P * oy;                        // and the outside column's
+    int odd = (p & 1) * PLANE;                                   // plane p's buffers
+    sT0[odd + slot] = z0c;
+    if (ring) sT0[odd + oslot] = ld<float>(plane(Tin, pxy * p), co);
+    __syncthreads();
+    // Loads of plane q's source and of dT and class at q+1, issued one iteration
+    // ahead of their use (plane nz + 2 does not exist: plane nz + 1 stands in, unused)
+    float n_z0p, n_o = 0.f, n_s;
+    unsigned n_cpr;
+    long aq = pxy * p, up = pxy * (p + 1);                       // planes q and q+1
     auto issue = [&](int q) {
-        if (q <= nz) {                                        // plane q+1 <= nz+1 exists
-            n_z0p = Tin[ch + pxy * (q + 1)];
-            n_cpr = cla[ch + pxy * (q + 1)];
-        }
-        if (q >= 1 && q <= nz) {
-            const long c = ci + pxy * q;
-            n_txm = Tin[c - 1];
-            n_txp = Tin[c + 1];
-            n_tym = Tin[c - px];
-            n_typ = Tin[c + px];
-            n_s = srca[c];
-        }
+        const Global<const float> t = plane(Tin, up);
+        n_z0p = ld<float>(t, ch);
+        if (ring) n_o = ld<float>(t, co);
+        n_cpr = ld<uint8_t>(plane((const uint8_t*)cls, up), ch);
+        n_s = ld<float>(plane(src, aq), ch);
+        aq = up;
+        up += q < nz ? pxy : 0;
+    };
+    // increment of a step at (plane q, column) with mixed classes around it;
+    // g: the face coefficients
+    auto mixed = [&](int q, unsigned c, float* g) {
+        const Global<const uint8_t> cq = plane((const uint8_t*)cls, pxy * q);
+        const int cc = c & TAM_CLASS_MASK;
+        const unsigned xm = ld<uint8_t>(cq - 1, ci), xp = ld<uint8_t>(cq + 1, ci), ym = ld<uint8_t>(cq - px, ci), yp = ld<uint8_t>(cq + px, ci),
+                       zm = ld<uint8_t>(cq - pxy, ci), zp = ld<uint8_t>(cq + pxy, ci);
+        g[0] = sLut[(xm & TAM_CLASS_MASK) * 16 + cc];
+        g[1] = sLut[cc * 16 + (xp & TAM_CLASS_MASK)];
+        g[2] = sLut[256 + (ym & TAM_CLASS_MASK) * 16 + cc];
+        g[3] = sLut[256 + cc * 16 + (yp & TAM_CLASS_MASK)];
+        g[4] = sLut[512 + (zm & TAM_CLASS_MASK) * 16 + cc];
+        g[5] = sLut[512 + cc * 16 + (zp & TAM_CLASS_MASK)];
+    };
+    // energy through the grid's faces at a boundary voxel
+    auto faces = [&](int q, unsigned c, const float* g, float tc, float xm, float xp, float ym, float yp, float zm,
+                     float zp) {
+        float e = 0.f;
+        if (i == 1) e += g[0] * (xm - tc);
+        if (i == nx) e += g[1] * (xp - tc);
+        if (j == 1) e += g[2] * (ym - tc);
+        if (j == ny) e += g[3] * (yp - tc);
+        if (q == 1) e += g[4] * (zm - tc);
+        if (q == nz) e += g[5] * (zp - tc);
+        e_acc -= sLut[768 + (c & TAM_CLASS_MASK)] * e;
     };
     issue(p);
-    for (; p <= k1; ++p) {
-        const bool interior = p >= 1 && p <= nz;              // else a halo plane: dT fixed
+    const int top = robin ? nz : -1;                             // the plane under the convective face
+    long ok = pxy * (p - 1), vk = nxy * (p - 2);                 // plane k in dT and in Omega
+    for (; p <= k1; ++p, ok += pxy, vk += nxy) {
+        // opaque, so that the 32-bit lane offsets are not widened outside the loop
+        asm volatile("" : "+v"(ch), "+v"(co), "+v"(vc));
         const int k = p - 1;
-        const bool step2 = p > k0;                            // second step at k in this iteration
-        // ---- plane p's values (loaded last iteration); plane p+1's loads go out now
-        const float z0p = n_z0p, txm = n_txm, txp = n_txp, tym = n_tym, typ = n_typ, s_p = n_s;
+        const float z0p = n_z0p, s_p = n_s;
         const unsigned cpr = n_cpr;
-        if (p < k1) issue(p + 1);
-        const long v = vcol + nxy * (k - 1);
-        const bool pom = step2 && damage && own && u1c >= wlo && u1c < whi;
-        double om_pf = 0.0;
-        unsigned tm_pf = 0;
-        if (pom) {
-            om_pf = a.omega[v];
-            tm_pf = a.tmask[v];
-        }
         // ---- first step at plane p
-        float t1p = z0c;                                      // halo planes and columns keep dT
-        float gxm = 0.f, gxp = 0.f, gym = 0.f, gyp = 0.f, gzm = 0.f, gzp = 0.f;
-        const int cc = ccr & TAM_CLASS_MASK;
-        if (interior) {
-            const int cp = cpr & TAM_CLASS_MASK;
-            if (__all((ccr & TAM_CLASS_HOM) != 0)) {
-                gxm = gxp = sLut[cc * 17];
-                gym = gyp = sLut[256 + cc * 17];
-                gzm = gzp = sLut[512 + cc * 17];
-            } else {
-                const long c = ci + pxy * p;
-                const int cxm = cla[c - 1] & TAM_CLASS_MASK, cxp = cla[c + 1] & TAM_CLASS_MASK;
-                const int cym = cla[c - px] & TAM_CLASS_MASK, cyp = cla[c + px] & TAM_CLASS_MASK;
-                gxm = sLut[cxm * 16 + cc];
-                gxp = sLut[cc * 16 + cxp];
-                gym = sLut[256 + cym * 16 + cc];
-                gyp = sLut[256 + cc * 16 + cyp];
-                gzp = sLut[512 + cc * 16 + cp];
-                gzm = sLut[512 + cm * 16 + cc];
+        const float* t0 = sT0 + odd + slot;
+        const float xm0 = t0[-1], xp0 = t0[1], ym0 = t0[-P], yp0 = t0[P];
+        float g[6];
+        if (__builtin_amdgcn_ballot_w64((ccr & TAM_CLASS_HOM) == 0 && real) == 0) {
+            const float4 h = sHom[ccr & TAM_CLASS_MASK];
+            g[0] = g[1] = h.x;
+            g[2] = g[3] = h.y;
+            g[4] = g[5] = h.z;
+        } else {
+            mixed(min(max(p, 1), nz), ccr, g);
+        }
+        float tp = z0p;
+        if (p == top) {
+            const float2 rb = sRob[ccr & TAM_CLASS_MASK];
+            tp = fmaf(rb.x, z0c, rb.y);
+        }
+        const float inc = face_sum(z0c, g[0], xm0, g[1], xp0, g[2], ym0, g[3], yp0, g[4], z0m, g[5], tp);
+        const float t1 = step_update(z0c, inc, lon0, s_p);
+        const float t1p = real && p >= 1 && p <= nz ? t1 : z0c;   // halo planes and columns keep dT
+        if (energy) {
+            asm volatile("");                                    // a scalar branch of its own
+            if (p >= k0 && p < k1 && own && (bnd_ij || p == 1 || p == nz))
+                faces(p, ccr, g, z0c, xm0, xp0, ym0, yp0, z0m, tp);
+        }
+        // what the next iteration reads of plane p+1; the buffers last held
+        // planes p-1 and p-2, whose readers passed the previous barrier
+        sT0[PLANE - odd + slot] = z0p;
+        if (ring) sT0[PLANE - odd + oslot] = n_o;
+        sT1[odd + slot] = t1p;
+        // ---- loads of the next plane, and of Omega and the mask where this
+        // plane's second step may need them
+        if (p < k1) issue(p + 1);
+        if (p > k0) {
+            double om = 0.0;
+            unsigned m = 0;
+            const bool pom = damage && own && u1c >= wlo && u1c < whi;
+            if (pom) {
+                om = ld<double>(plane((const double*)omega, vk), vc);
+                m = ld<uint8_t>(plane((const uint8_t*)tmask, vk), vc);
             }
-            float tp = z0p;
-            if (robin && p == nz) {
-                const float2 rb = sRob[cc];
-                tp = fmaf(rb.x, z0c, rb.y);
+            // ---- second step at plane k = p-1 (dT1 of plane k is in the other buffer)
+            const float* t = sT1 + (PLANE - odd) + slot;
+            const float xm = t[-1], xp = t[1], ym = t[-P], yp = t[P];
+            float tq = t1p;
+            if (k == top) {
+                const float2 rb = sRob[Ckr & TAM_CLASS_MASK];
+                tq = fmaf(rb.x, u1c, rb.y);
             }
-            const float inc = face_sum(z0c, gxm, txm, gxp, txp, gym, tym, gyp, typ, gzm, z0m, gzp, tp);
-            if (real) t1p = step_update(z0c, inc, lon0, s_p);
-            if (own && p >= k0 && p < k1) {
-                if (z0c < a.dT_neg) a.flags[0] = 1;             // 3dFD.f90:179-182
-                if (energy && (bnd_ij || p == 1 || p == nz)) {
-                    float e = 0.f;
-                    if (i == 1) e += gxm * (txm - z0c);
-                    if (i == nx) e += gxp * (txp - z0c);
-                    if (j == 1) e += gym * (tym - z0c);
-                    if (j == ny) e += gyp * (typ - z0c);
-                    if (p == 1) e += gzm * (z0m - z0c);
-                    if (p == nz) e += gzp * (tp - z0c);
-                    e_acc -= sLut[768 + cc] * e;
+            const float inc2 = face_sum(u1c, G[0], xm, G[1], xp, G[2], ym, G[3], yp, G[4], u1m, G[5], tq);
+            const float tn = step_update(u1c, inc2, lon1, Sk);
+            if (energy) {
+                asm volatile("");
+                if (own && (bnd_ij || k == 1 || k == nz)) faces(k, Ckr, G, u1c, xm, xp, ym, yp, u1m, tq);
+            }
+            tmin = fminf(tmin, fminf(z0m, u1c));              // dT at k before either step
+            if (own) {
+                st(plane(Tout, ok), ch, tn);
+                if (damage) {                                   // step 1, then step 2
+                    const bool din = (Ckr & TAM_CLASS_DUE) != 0u;
+                    // true wherever either step's dT is inside; the exact tests follow
+                    if (din || (fmaxf(u1c, tn) >= a.dT_lo_test && fminf(u1c, tn) < a.dT_hi_test)) {
+                        if (!pom) {
+                            om = ld<double>(plane((const double*)omega, vk), vc);
+                            m = ld<uint8_t>(plane((const uint8_t*)tmask, vk), vc);
+                        }
+                        const long v = vk + vc, nv = nxy * nz;
+                        bool dirty = false;
+                        bool due = damage_step(sDmg, a.thres, tmask, v, nv, u1c, sDmg.t_after[0], din, om, dirty, m);
+                        due = damage_step(sDmg, a.thres, tmask, v, nv, tn, sDmg.t_after[1], due, om, dirty, m);
+                        if (dirty) st(plane(omega, vk), vc, om);
+                        if (due != din)
+                            st(plane(cls, ok), ch, (uint8_t)((Ckr & ~TAM_CLASS_DUE) | (due ? TAM_CLASS_DUE : 0u)));
+                    }
                 }
             }
         }
-        // ---- second step at plane k = p-1 (dT1 of plane k is in sT1[k & 1])
-        if (step2 && own) {
-            const float xm = sT1[k & 1][ty][tx - 1], xp = sT1[k & 1][ty][tx + 1];
-            const float ym = sT1[k & 1][ty - 1][tx], yp = sT1[k & 1][ty + 1][tx];
-            float tp = t1p;
-            if (robin && k == nz) {
-                const float2 rb = sRob[Ck];
-                tp = fmaf(rb.x, u1c, rb.y);
-            }
-            const float inc = face_sum(u1c, Gxm, xm, Gxp, xp, Gym, ym, Gyp, yp, Gzm, u1m, Gzp, tp);
-            const float tn = step_update(u1c, inc, lon1, Sk);
-            if (u1c < a.dT_neg) a.flags[0] = 1;
-            Tout[ch + pxy * k] = tn;
-            if (damage) {                                       // step 1, then step 2
-                double om = 0.0;
-                unsigned m = 0;
-                bool have = false, dirty = false, have_m = false;
-                const bool din = (Ckr & TAM_CLASS_DUE) != 0u;
-                bool due = damage_step(a, v, nv, u1c, ta0, din, pom, om_pf, tm_pf, om, have, dirty, m, have_m);
-                due = damage_step(a, v, nv, tn, ta1, due, pom, om_pf, tm_pf, om, have, dirty, m, have_m);
-                if (dirty) a.omega[v] = om;
-                if (due != din)
-                    a.cls[ch + pxy * k] = (uint8_t)((Ckr & ~TAM_CLASS_DUE) | (due ? TAM_CLASS_DUE : 0u));
-            }
-            if (energy && (bnd_ij || k == 1 || k == nz)) {
-                float e = 0.f;
-                if (i == 1) e += Gxm * (xm - u1c);
-                if (i == nx) e += Gxp * (xp - u1c);
-                if (j == 1) e += Gym * (ym - u1c);
-                if (j == ny) e += Gyp * (yp - u1c);
-                if (k == 1) e += Gzm * (u1m - u1c);
-                if (k == nz) e += Gzp * (tp - u1c);
-                e_acc -= sLut[768 + Ck] * e;
-            }
-        }
-        // plane p's buffer last held plane p-2, whose readers passed the
-        // previous iteration's barrier
-        sT1[p & 1][ty][tx] = t1p;
         __syncthreads();
+        odd = PLANE - odd;
         u1m = u1c;
         u1c = t1p;
         z0m = z0c;
         z0c = z0p;
-        cm = cc;
         Ckr = ccr;                                            // plane p's byte, before the rotation
         ccr = cpr;
-        Gxm = gxm; Gxp = gxp; Gym = gym; Gyp = gyp; Gzm = gzm; Gzp = gzp;
         Sk = s_p;
-        Ck = cc;
+#pragma unroll
+        for (int f = 0; f < 6; ++f) G[f] = g[f];
     }
+    if (own && tmin < a.dT_neg) a.flags[0] = 1;                // 3dFD.f90:179-182
     if (energy) {
         __shared__ double sE[TX * TY / 64];
         const double w = wave_sum_d((double)e_acc);
@@ -783,13 +875,14 @@ __device__ __forceinline__ int batch_tile(const HeatBatchEntry* __restrict__ tab
         if (tile_start[mid] <= b) lo = mid;
         else hi = mid - 1;
     }
+    lo = __builtin_amdgcn_readfirstlane(lo);      // the block's, so the instance's arguments stay scalar
     const HeatBatchEntry& e = tab[lo];
     gx = (e.a.nx + ox - 1) / ox;
     gy = (e.a.ny + oy - 1) / oy;
     const int local = b - tile_start[lo];
-    tl.x = local % gx;
-    tl.y = (local / gx) % gy;
-    tl.z = local / (gx * gy);
+    tl.x = __builtin_amdgcn_readfirstlane(local % gx);
+    tl.y = __builtin_amdgcn_readfirstlane((local / gx) % gy);
+    tl.z = __builtin_amdgcn_readfirstlane(local / (gx * gy));
     tl.id = local;
     return lo;
 }
