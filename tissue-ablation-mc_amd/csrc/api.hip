@@ -147,7 +147,7 @@ HeatArgs heat_args(tam_ctx* c)
     a.arr_A = c->p.arr_A; a.arr_dE = c->p.arr_dE; a.arr_R = c->p.arr_R;
     a.arr_Tlo = c->p.arr_Tlo; a.arr_Thi = c->p.arr_Thi;
     a.thr0 = c->p.arr_thr[0]; a.thr1 = c->p.arr_thr[1]; a.thr2 = c->p.arr_thr[2];
-    a.energy = c->energy; a.flags = c->flags;
+    a.flags = c->flags;
     a.cls = c->cls; a.glut = c->glut; a.robin_lut = c->robin_lut;
     a.eblk = c->eblk;
     a.lnA = std::log(c->p.arr_A);
@@ -277,7 +277,7 @@ Heat64Args heat64_args(tam_ctx* c)
     a.arr_A = c->p.arr_A; a.arr_dE = c->p.arr_dE; a.arr_R = c->p.arr_R;
     a.arr_Tlo = c->p.arr_Tlo; a.arr_Thi = c->p.arr_Thi;
     a.thr0 = c->p.arr_thr[0]; a.thr1 = c->p.arr_thr[1]; a.thr2 = c->p.arr_thr[2];
-    a.energy = c->energy; a.flags = c->flags;
+    a.eblk = c->eblk; a.flags = c->flags;
     return a;
 }
 
@@ -578,7 +578,7 @@ int tam_create(const tam_params* p, tam_ctx** out)
     if (e == hipSuccess) e = dalloc(&c->box_psum, nz);
     if (e == hipSuccess) e = dalloc(&c->box_geom, 6);
     if (e == hipSuccess) e = hipMemsetAsync(c->box_geom, 0, 6 * sizeof(int), c->stream);
-    if (e == hipSuccess) e = dalloc(&c->energy, 4);
+    if (e == hipSuccess) e = dalloc(&c->energy, 1);
     if (e == hipSuccess) e = dalloc(&c->flags, 4);
     if (e == hipSuccess) e = dalloc(&c->counters, TAM_CNT_SLOTS);
     if (c->fp64) {
@@ -609,7 +609,6 @@ int tam_create(const tam_params* p, tam_ctx** out)
     launch_fill_f64(c->omega, V, 0.0, s);
     launch_fill_f64(c->thres, 3 * V, 0.0, s);
     launch_tmask(c->thres, c->omega, p->arr_thr[0], p->arr_thr[1], p->arr_thr[2], c->tmask, V, s);
-    launch_fill_f64(c->energy, 4, 0.0, s);
     launch_fill_f64(c->eblk, c->neblk, 0.0, s);
     launch_fill_f32((float*)c->flags, 4, 0.f, s);
     launch_fill_f32(c->mut, V, 0.f, s);
@@ -777,7 +776,6 @@ int tam_set_thermal(tam_ctx* c, const double* temp, const double* kappa, const d
     else HIPCHK(c, launch_fill_f64(c->Q, V, 0.0, c->stream));
     if (W) HIPCHK(c, hipMemcpyAsync(c->W, W, sizeof(double) * (size_t)V, hipMemcpyHostToDevice, c->stream));
     else HIPCHK(c, launch_fill_f64(c->W, V, 0.75, c->stream));
-    HIPCHK(c, launch_fill_f64(c->energy, 4, 0.0, c->stream));
     HIPCHK(c, launch_fill_f64(c->eblk, c->neblk, 0.0, c->stream));
     HIPCHK(c, launch_fill_f32((float*)c->flags, 4, 0.f, c->stream));
     c->cur = c->dT0;
@@ -1176,17 +1174,17 @@ int tam_energy(tam_ctx* c, double* heat_content, double* boundary_out)
 {
     if (!c) return TAM_ERR_ARG;
     Dev d(c->dev);
-    HIPCHK(c, launch_fill_f64(c->energy + 1, 1, 0.0, c->stream));
+    HIPCHK(c, launch_fill_f64(c->energy, 1, 0.0, c->stream));
     HIPCHK(c, launch_energy(c->p.nx, c->p.ny, c->p.nz, c->px, c->pxy, c->cur, c->fp64 ? c->cur64 : nullptr,
-                            c->p.t_ref, c->heatcap, c->p.mass_voxel, c->energy + 1, c->stream));
-    double e[2];
+                            c->p.t_ref, c->heatcap, c->p.mass_voxel, c->energy, c->stream));
+    double content = 0.0, out = 0.0;
     std::vector<double> blk((size_t)c->neblk);
-    HIPCHK(c, hipMemcpyAsync(e, c->energy, sizeof(e), hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, hipMemcpyAsync(&content, c->energy, sizeof(content), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipMemcpyAsync(blk.data(), c->eblk, sizeof(double) * blk.size(), hipMemcpyDeviceToHost, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
-    for (double b : blk) e[0] += b;
-    if (boundary_out) *boundary_out = e[0];
-    if (heat_content) *heat_content = e[1];
+    for (double b : blk) out += b;
+    if (boundary_out) *boundary_out = out;
+    if (heat_content) *heat_content = content;
     return TAM_OK;
 }
 

@@ -25,6 +25,11 @@ __device__ __forceinline__ double wave_sum_d(double v)
     return v;
 }
 
+// One thread per voxel; bound by the FP64 fields it streams (dT, three face
+// coefficients, coeff, jmean: about 40 MB at 80^3).  The energy through the
+// grid's faces goes to the block's own slot, which only this block writes in a
+// launch: on a grid of 80^3 nearly every wave holds a boundary voxel, and 8000
+// FP64 adds to one address took 95 us of the step's 102 us at 12 ns each.
 template <bool BOIL, bool ROBIN, bool DAMAGE, bool ENERGY>
 __global__ __launch_bounds__(256) void heat64_kernel(Heat64Args a, const double* __restrict__ Tin,
                                                      double* __restrict__ Tout, double lon, double time_after)
@@ -33,14 +38,14 @@ __global__ __launch_bounds__(256) void heat64_kernel(Heat64Args a, const double*
         lon = (double)*a.dyn_lon;
         time_after = *a.dyn_tafter;
     }
-    const long nv = (long)a.nx * a.ny * a.nz;
-    const long v = (long)blockIdx.x * 256 + threadIdx.x;
+    const unsigned nv = (unsigned)a.nx * a.ny * a.nz;          // fewer than 2^32 voxels
+    const unsigned v = blockIdx.x * 256 + threadIdx.x;
     double e_out = 0.0;
     if (v < nv) {
-        const int i = (int)(v % a.nx) + 1;
-        const long r = v / a.nx;
-        const int j = (int)(r % a.ny) + 1;
-        const int k = (int)(r / a.ny) + 1;
+        const unsigned r = v / (unsigned)a.nx;
+        const int i = (int)(v - r * a.nx) + 1;
+        const int k = (int)(r / (unsigned)a.ny) + 1;
+        const int j = (int)(r - (unsigned)(k - 1) * a.ny) + 1;
         const long px = a.px, pxy = a.pxy;
         const long c = i + px * j + pxy * k;
         const double Tc = Tin[c];
@@ -99,8 +104,11 @@ __global__ __launch_bounds__(256) void heat64_kernel(Heat64Args a, const double*
         }
     }
     if (ENERGY) {
+        __shared__ double sE[4];
         const double w = wave_sum_d(e_out);
-        if ((threadIdx.x & 63) == 0 && w != 0.0) unsafeAtomicAdd(&a.energy[0], w);
+        if ((threadIdx.x & 63) == 0) sE[threadIdx.x >> 6] = w;
+        __syncthreads();
+        if (threadIdx.x == 0) a.eblk[blockIdx.x] += (sE[0] + sE[1]) + (sE[2] + sE[3]);
     }
 }
 

@@ -169,19 +169,20 @@ __global__ __launch_bounds__(256) void normalise_kernel(int nx, int ny, int nz, 
     src[c] = (float)(coeff[c] * jm);
 }
 
+// A grid-stride sum: one add per block to the one result, at 12 ns each, so the
+// grid is held to 2048 blocks (a block per 256 voxels took 0.4 ms at 200^3).
 __global__ __launch_bounds__(256) void energy_kernel(int nx, int ny, int nz, long px, long pxy,
                                                      const float* dT, const double* T64, double t_ref,
                                                      const double* heatcap, double mass, double* out)
 {
     __shared__ double red[4];
     const long nv = (long)nx * ny * nz;
-    const long v = (long)blockIdx.x * 256 + threadIdx.x;
     double e = 0.0;
-    if (v < nv) {
+    for (long v = (long)blockIdx.x * 256 + threadIdx.x; v < nv; v += (long)gridDim.x * 256) {
         int i, j, k;
         vox_ijk(v, nx, ny, i, j, k);
         const long c = i + px * j + pxy * k;
-        e = heatcap[c] * mass * (T64 ? T64[c] - t_ref : (double)dT[c]);
+        e += heatcap[c] * mass * (T64 ? T64[c] - t_ref : (double)dT[c]);
     }
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) e += __shfl_xor(e, o, 64);
@@ -284,7 +285,8 @@ hipError_t launch_block_sums(const double* f, int nx, int ny, int nz, int k, dou
 hipError_t launch_energy(int nx, int ny, int nz, long px, long pxy, const float* dT, const double* T64,
                          double t_ref, const double* heatcap, double mass_voxel, double* out, hipStream_t s)
 {
-    hipLaunchKernelGGL(energy_kernel, dim3(grid_for((long)nx * ny * nz)), dim3(256), 0, s, nx, ny, nz, px, pxy,
+    const unsigned blocks = grid_for((long)nx * ny * nz);
+    hipLaunchKernelGGL(energy_kernel, dim3(blocks < 2048 ? blocks : 2048), dim3(256), 0, s, nx, ny, nz, px, pxy,
                        dT, T64, t_ref, heatcap, mass_voxel, out);
     return hipGetLastError();
 }

@@ -157,8 +157,7 @@ struct HeatArgs {
     double thr_min;            // smallest threshold of the chain
     float dT_win_pad;          // extra margin of the Omega prefetch predicate, K
     // energy accounting
-    double* energy;            // [0] boundary outflow, J
-    double* eblk;              // per-block boundary outflow slots (FP32 stencil)
+    double* eblk;              // per-block boundary outflow slots
     int* flags;                // [0] negative temperature seen
     // class mode (see heat.hip)
     uint8_t* cls;              // halo: thermal class per cell (the step keeps TAM_CLASS_DUE)
@@ -208,7 +207,7 @@ struct Heat64Args {            // FP64 reference-order step (heat64.hip)
     double* omega; double* thres;
     uint8_t* tmask;
     double arr_A, arr_dE, arr_R, arr_Tlo, arr_Thi, thr0, thr1, thr2;
-    double* energy;
+    double* eblk;              // per-block boundary outflow slots
     int* flags;
     const float* dyn_lon;      // graph replays, as in HeatArgs
     const double* dyn_tafter;
@@ -291,7 +290,7 @@ struct tam_ctx {
     uint8_t* tn_cls;
     double* box_psum;           // LDS tally box placement: per-plane sums (nz) and the chosen
     int* box_geom;              // geometry (o[3], n[3])
-    double* energy;             // [0] boundary outflow, [1..] reduction scratch
+    double* energy;             // heat content, summed on request
     int* flags;
     unsigned long long* counters;
     double time;                // heat time when no pulse state is passed
