@@ -261,6 +261,19 @@ RebuildArgs rebuild_args(tam_ctx* c)
     a.mask = c->mask; a.air_id = c->air_id;
     a.T64 = c->fp64 ? c->cur64 : nullptr;
     a.cls = c->lut ? c->cls : nullptr;
+    a.jmean = c->jmean;
+    a.src = c->fp64 ? nullptr : c->src;
+    return a;
+}
+
+ArrArgs arr_args(const tam_ctx* c, double delt, double time)
+{
+    ArrArgs a{};
+    a.omega = c->omega; a.thres = c->thres; a.tmask = c->tmask;
+    a.A = c->p.arr_A; a.dE = c->p.arr_dE; a.R = c->p.arr_R;
+    a.Tlo = c->p.arr_Tlo; a.Thi = c->p.arr_Thi;
+    a.thr0 = c->p.arr_thr[0]; a.thr1 = c->p.arr_thr[1]; a.thr2 = c->p.arr_thr[2];
+    a.delt = delt; a.time = time;
     return a;
 }
 
@@ -278,6 +291,21 @@ Heat64Args heat64_args(tam_ctx* c)
     a.arr_Tlo = c->p.arr_Tlo; a.arr_Thi = c->p.arr_Thi;
     a.thr0 = c->p.arr_thr[0]; a.thr1 = c->p.arr_thr[1]; a.thr2 = c->p.arr_thr[2];
     a.eblk = c->eblk; a.flags = c->flags;
+    return a;
+}
+
+Coeff64Args coeff64_args(tam_ctx* c)
+{
+    Coeff64Args a{};
+    a.nx = c->p.nx; a.ny = c->p.ny; a.nz = c->p.nz;
+    a.px = c->px; a.pxy = c->pxy;
+    a.dscale = c->p.dscale;
+    a.idx2 = 1.0 / (c->p.dx_m * c->p.dx_m);
+    a.idy2 = 1.0 / (c->p.dy_m * c->p.dy_m);
+    a.idz2 = 1.0 / (c->p.dz_m * c->p.dz_m);
+    a.kappa = c->kappa; a.density = c->density; a.heatcap = c->heatcap;
+    a.ax = c->ax; a.ay = c->ay; a.az = c->az;
+    a.rhokap = c->rhokap; a.removed_inert = c->p.removed_inert;
     return a;
 }
 
@@ -302,17 +330,7 @@ hipError_t build_coeffs(tam_ctx* c)
                                                               c->stream);
         return e;
     }
-    Coeff64Args a{};
-    a.nx = c->p.nx; a.ny = c->p.ny; a.nz = c->p.nz;
-    a.px = c->px; a.pxy = c->pxy;
-    a.dscale = c->p.dscale;
-    a.idx2 = 1.0 / (c->p.dx_m * c->p.dx_m);
-    a.idy2 = 1.0 / (c->p.dy_m * c->p.dy_m);
-    a.idz2 = 1.0 / (c->p.dz_m * c->p.dz_m);
-    a.kappa = c->kappa; a.density = c->density; a.heatcap = c->heatcap;
-    a.ax = c->ax; a.ay = c->ay; a.az = c->az;
-    a.rhokap = c->rhokap; a.removed_inert = c->p.removed_inert;
-    return launch_coeffs64(a, c->stream);
+    return launch_coeffs64(coeff64_args(c), c->stream);
 }
 
 float elapsed(tam_ctx* c)
@@ -356,6 +374,21 @@ int refresh_src(tam_ctx* c)
     return TAM_OK;
 }
 
+// setupThermalCoeff (3dFD.f90:312-361) on c->stream, with the cycle's damage
+// before it where arr is given
+int enqueue_rebuild(tam_ctx* c, const ArrArgs* arr)
+{
+    const RebuildArgs r = rebuild_args(c);
+    HIPCHK(c, launch_update(r, arr, c->stream));
+    if (c->fp64) {
+        HIPCHK(c, launch_rebuild64(r, coeff64_args(c), c->stream));
+    } else {
+        HIPCHK(c, launch_apply_props(r, c->stream));
+        HIPCHK(c, build_coeffs(c));
+    }
+    return TAM_OK;
+}
+
 // ---- captured coupling cycle -------------------------------------------
 
 // Drop the captured graphs (state or launch shape changed; the next
@@ -388,15 +421,14 @@ int enqueue_cycle(tam_ctx* c, int* swaps)
     const double* ta = (const double*)(c->cyc_dev + cycle_ta_off(c->cyc_loops));
     hipStream_t s = c->stream;
     // transport (mcpolar.f90:151-170) and normalisation (:173-174)
-    HIPCHK(c, launch_fill_u64(c->counters, TAM_CNT_SLOTS, s));
     McArgs m = mc_args(c, c->cyc_npk, c->cyc_seed, 0);
     m.clear_tally = 1;                     // after the LDS-box placement has read the last cycle's tally
     m.dyn_npk = &hdr->npk;
     m.dyn_stream = &hdr->stream;
     HIPCHK(c, launch_mc(m, s));
-    HIPCHK(c, launch_acc_u64(c->cnt_acc, c->counters, TAM_CNT_N, s));
     HIPCHK(c, launch_normalise(c->p.nx, c->p.ny, c->p.nz, c->px, c->pxy, c->tally, c->rhokap, c->mat,
-                               c->mua_frac, hdr, 0.0, c->coeff, c->jmean, c->src, s));
+                               c->mua_frac, hdr, 0.0, c->coeff, c->jmean, c->fp64 ? nullptr : c->src, c->cnt_acc,
+                               c->counters, s));
     // heat_sim_3D (3dFD.f90:21-230)
     const int boil = c->p.boil != 0, robin = c->p.robin_top != 0, dmg = c->p.damage_every_step != 0;
     HeatArgs a = heat_args(c);
@@ -424,19 +456,11 @@ int enqueue_cycle(tam_ctx* c, int* swaps)
             ++*swaps;
         }
     }
-    // Arrhenius at the reference cadence (mcpolar.f90:181)
-    if (c->cyc_arr) {
-        HeatArgs aa = heat_args(c);
-        aa.dyn_arr = hdr->arr;
-        HIPCHK(c, launch_arrhenius(aa, c->cur, c->fp64 ? c->cur64 : nullptr, 0.0, 0.0, s));
-    }
-    // setupThermalCoeff (mcpolar.f90:183, 3dFD.f90:312-361)
-    const RebuildArgs r = rebuild_args(c);
-    if (c->p.thermal_mode == TAM_THERMAL_WATER) HIPCHK(c, launch_water_update(r, s));
-    HIPCHK(c, launch_removal_mask(r, s));
-    HIPCHK(c, launch_apply_props(r, s));
-    HIPCHK(c, build_coeffs(c));
-    return refresh_src(c);
+    // Arrhenius at the reference cadence (mcpolar.f90:181) and setupThermalCoeff
+    // (:183, 3dFD.f90:312-361)
+    ArrArgs arr = arr_args(c, 0.0, 0.0);
+    arr.dyn = hdr->arr;
+    return enqueue_rebuild(c, c->cyc_arr ? &arr : nullptr);
 }
 
 // Capture enqueue_cycle from the current ping-pong parity into cyc_exec[par].
@@ -803,7 +827,6 @@ int tam_mc_run(tam_ctx* c, int64_t npackets, uint64_t seed, uint32_t stream, int
     if (npackets < 0) return fail(c, TAM_ERR_ARG, "negative packet count");
     if (!c->optics_set) return fail(c, TAM_ERR_STATE, "tam_set_optics must come first");
     Dev d(c->dev);
-    HIPCHK(c, launch_fill_u64(c->counters, TAM_CNT_SLOTS, c->stream));
     McArgs a = mc_args(c, npackets, seed, stream);
     a.clear_tally = accumulate ? 0 : 1;    // after the LDS-box placement has read the last run's tally
     HIPCHK(c, hipEventRecord(c->ev0, c->stream));
@@ -838,7 +861,8 @@ int tam_normalise(tam_ctx* c, double scale)
     Dev d(c->dev);
     HIPCHK(c, hipEventRecord(c->ev0, c->stream));
     HIPCHK(c, launch_normalise(c->p.nx, c->p.ny, c->p.nz, c->px, c->pxy, c->tally, c->rhokap, c->mat,
-                               c->mua_frac, nullptr, scale, c->coeff, c->jmean, c->src, c->stream));
+                               c->mua_frac, nullptr, scale, c->coeff, c->jmean, c->fp64 ? nullptr : c->src, nullptr,
+                               nullptr, c->stream));
     HIPCHK(c, hipEventRecord(c->ev1, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     c->timing.normalise_ms = elapsed(c);
@@ -897,7 +921,7 @@ int tam_arrhenius(tam_ctx* c, double delt, double time)
     if (!c->thermal_set) return fail(c, TAM_ERR_STATE, "tam_set_thermal must come first");
     Dev d(c->dev);
     HIPCHK(c, hipEventRecord(c->ev0, c->stream));
-    HIPCHK(c, launch_arrhenius(heat_args(c), c->cur, c->fp64 ? c->cur64 : nullptr, delt, time, c->stream));
+    HIPCHK(c, launch_arrhenius(rebuild_args(c), arr_args(c, delt, time), c->stream));
     HIPCHK(c, hipEventRecord(c->ev1, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     c->timing.arrhenius_ms = elapsed(c);
@@ -909,13 +933,8 @@ int tam_rebuild(tam_ctx* c)
     if (!c) return TAM_ERR_ARG;
     if (!c->thermal_set || !c->optics_set) return fail(c, TAM_ERR_STATE, "optics and thermal state must be set");
     Dev d(c->dev);
-    const RebuildArgs a = rebuild_args(c);
     HIPCHK(c, hipEventRecord(c->ev0, c->stream));
-    if (c->p.thermal_mode == TAM_THERMAL_WATER) HIPCHK(c, launch_water_update(a, c->stream));
-    HIPCHK(c, launch_removal_mask(a, c->stream));
-    HIPCHK(c, launch_apply_props(a, c->stream));
-    HIPCHK(c, build_coeffs(c));
-    if (refresh_src(c) != TAM_OK) return TAM_ERR_HIP;
+    if (enqueue_rebuild(c, nullptr) != TAM_OK) return TAM_ERR_HIP;
     HIPCHK(c, hipEventRecord(c->ev1, c->stream));
     HIPCHK(c, hipStreamSynchronize(c->stream));
     c->timing.rebuild_ms = elapsed(c);

@@ -915,33 +915,6 @@ __global__ __launch_bounds__(TX* TY) void stencil_t2_batch_kernel(const HeatBatc
     t2_body<TX, TY>(e.a, Tin, Tout, lon0, lon1, ta0, ta1, kz, flags, tl, gx, gy);
 }
 
-// Arrhenius at the reference cadence: every interior voxel, the full
-// threshold chain (3dFD.f90:447-464).
-__global__ __launch_bounds__(256) void arrhenius_kernel(HeatArgs a, const float* __restrict__ T,
-                                                        const double* __restrict__ T64, double delt,
-                                                        double time)
-{
-    if (a.dyn_arr) {              // graph replay: (delt, time) from device memory
-        delt = a.dyn_arr[0];
-        time = a.dyn_arr[1];
-    }
-    const long nv = (long)a.nx * a.ny * a.nz;
-    const long v = (long)blockIdx.x * 256 + threadIdx.x;
-    if (v >= nv) return;
-    const int i = (int)(v % a.nx) + 1;
-    const long r = v / a.nx;
-    const int j = (int)(r % a.ny) + 1;
-    const int k = (int)(r / a.ny) + 1;
-    const long c = i + a.px * j + a.pxy * k;
-    const double t = T64 ? T64[c] : a.t_ref + (double)T[c];
-    double om = a.omega[v];
-    if (t >= a.arr_Tlo && t < a.arr_Thi && a.rhokap[c] >= 0.0) {
-        om = om + delt * a.arr_A * exp(-a.arr_dE / (a.arr_R * t));
-        a.omega[v] = om;
-    }
-    thres_chain(a.thres, a.tmask, v, nv, om, a.thr0, a.thr1, a.thr2, time, a.tmask[v]);
-}
-
 template <int TX, int TY, bool LUT, bool DIRECT>
 hipError_t launch_t(const HeatArgs& a, const float* Tin, float* Tout, float lon, double t, int kz,
                     unsigned flags, hipStream_t s)
@@ -1092,11 +1065,3 @@ hipError_t launch_heat_step(const HeatArgs& a, const float* Tin, float* Tout, fl
     return hipErrorInvalidValue;
 }
 
-hipError_t launch_arrhenius(const HeatArgs& a, const float* T, const double* T64, double delt, double time,
-                            hipStream_t s)
-{
-    const long nv = (long)a.nx * a.ny * a.nz;
-    hipLaunchKernelGGL(arrhenius_kernel, dim3((unsigned)((nv + 255) / 256)), dim3(256), 0, s, a, T, T64, delt,
-                       time);
-    return hipGetLastError();
-}

@@ -112,37 +112,6 @@ __global__ __launch_bounds__(256) void heat64_kernel(Heat64Args a, const double*
     }
 }
 
-// a_f = dscale * kbar/(rhobar*cbar) / h^2 per face, in the reference's
-// operation order (3dFD.f90:119-129): one thread per halo cell, + faces.
-__global__ __launch_bounds__(256) void coeff64_kernel(Coeff64Args a)
-{
-    const long n = (long)(a.nx + 2) * (a.ny + 2) * (a.nz + 2);
-    const long c = (long)blockIdx.x * 256 + threadIdx.x;
-    if (c >= n) return;
-    const int i = (int)(c % a.px);
-    const long r = c / a.px;
-    const int j = (int)(r % (a.ny + 2));
-    const int k = (int)(r / (a.ny + 2));
-    const double* K = a.kappa;
-    const double* D = a.density;
-    const double* H = a.heatcap;
-    auto face = [&](long o, double ih2) {
-        const double kb = .5 * (K[c] + K[c + o]);
-        const double db = .5 * (D[c] + D[c + o]);
-        const double hb = .5 * (H[c] + H[c + o]);
-        return a.dscale * (kb / (db * hb)) * ih2;
-    };
-    const bool jin = j >= 1 && j <= a.ny, kin = k >= 1 && k <= a.nz, iin = i >= 1 && i <= a.nx;
-    auto removed = [&](long cc, bool interior) { return a.removed_inert && interior && a.rhokap[cc] == 0.0; };
-    const bool rc = removed(c, iin && jin && kin);
-    a.ax[c] = (i <= a.nx && jin && kin && !rc && !removed(c + 1, i + 1 <= a.nx && jin && kin))
-                  ? face(1, a.idx2) : 0.0;
-    a.ay[c] = (j <= a.ny && iin && kin && !rc && !removed(c + a.px, j + 1 <= a.ny && iin && kin))
-                  ? face(a.px, a.idy2) : 0.0;
-    a.az[c] = (k <= a.nz && iin && jin && !rc && !removed(c + a.pxy, k + 1 <= a.nz && iin && jin))
-                  ? face(a.pxy, a.idz2) : 0.0;
-}
-
 template <bool B, bool R, bool D, bool E>
 hipError_t launch_t(const Heat64Args& a, const double* Tin, double* Tout, double lon, double t, hipStream_t s)
 {
@@ -169,11 +138,4 @@ hipError_t launch_heat64_step(const Heat64Args& a, const double* Tin, double* To
 #undef TAM_CASE
     }
     return hipErrorInvalidValue;
-}
-
-hipError_t launch_coeffs64(const Coeff64Args& a, hipStream_t s)
-{
-    const long n = (long)(a.nx + 2) * (a.ny + 2) * (a.nz + 2);
-    hipLaunchKernelGGL(coeff64_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, s, a);
-    return hipGetLastError();
 }

@@ -835,7 +835,9 @@ hipError_t mc_prepare(int dev)
 hipError_t launch_mc(const McArgs& a, hipStream_t s)
 {
     const long nvox = (long)a.nx * a.ny * a.nz;
-    if (a.npk == 0) return a.clear_tally ? launch_fill_f64(a.tally, nvox, 0.0, s) : hipSuccess;
+    // the run's counters, and the tally unless the run adds to it
+    auto clear = [&] { return launch_clear(a.tally, a.clear_tally ? nvox : 0, a.counters, TAM_CNT_SLOTS, s); };
+    if (a.npk == 0) return clear();
     int dev = 0, ncu = 0, lds_cu = 0, lds_blk = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e == hipSuccess) e = hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
@@ -910,10 +912,8 @@ hipError_t launch_mc(const McArgs& a, hipStream_t s)
             hipLaunchKernelGGL(box_window_kernel, dim3(1), dim3(256), 0, s, a.box_psum, a.nz, bp, a.box_geom);
             b.box_geom = a.box_geom;
         }
-        if (a.clear_tally) {
-            const hipError_t ef = launch_fill_f64(a.tally, nvox, 0.0, s);
-            if (ef != hipSuccess) return ef;
-        }
+        const hipError_t ef = clear();
+        if (ef != hipSuccess) return ef;
         // the material table goes behind the box where that keeps the resident
         // blocks: LDS is given out in steps of lds_cu / 128
         const size_t tab_off = (lds + 15) & ~(size_t)15, tab_lds = tab_off + sizeof(MatEntry) * (size_t)a.nmat;
@@ -938,10 +938,8 @@ hipError_t launch_mc(const McArgs& a, hipStream_t s)
         }
 #undef TAM_BOX
     } else {
-        if (a.clear_tally) {
-            const hipError_t ef = launch_fill_f64(a.tally, nvox, 0.0, s);
-            if (ef != hipSuccess) return ef;
-        }
+        const hipError_t ef = clear();
+        if (ef != hipSuccess) return ef;
         // A short run takes as long as its longest packet's chain of events,
         // and a wave's pass costs the same for 4 lanes as for 64: up to 8
         // waves a CU (2 per SIMD) share fewer than 64 packets each, down to

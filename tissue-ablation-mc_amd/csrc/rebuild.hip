@@ -37,23 +37,50 @@ __device__ __forceinline__ double skin_cond(double W, double rho) { return rho *
 
 __device__ __forceinline__ void vox_ijk(long v, int nx, int ny, int& i, int& j, int& k)
 {
-    i = (int)(v % nx) + 1;
-    const long r = v / nx;
-    j = (int)(r % ny) + 1;
-    k = (int)(r / ny) + 1;
+    const unsigned u = (unsigned)v, r = u / (unsigned)nx;        // fewer than 2^32 voxels; 64-bit divides are slow
+    i = (int)(u - r * nx) + 1;
+    k = (int)(r / (unsigned)ny) + 1;
+    j = (int)(r - (unsigned)(k - 1) * ny) + 1;
 }
 
-__global__ __launch_bounds__(256) void water_kernel(RebuildArgs a)   // 3dFD.f90:328
+// cell c of a halo grid with px columns a row and n cells
+__device__ __forceinline__ void cell_ijk(long c, long n, int px, int py, int& i, int& j, int& k)
+{
+    if (n >> 32) {
+        i = (int)(c % px);
+        j = (int)(c / px % py);
+        k = (int)(c / px / py);
+    } else {
+        const unsigned u = (unsigned)c, r = u / (unsigned)px;
+        i = (int)(u - r * px);
+        k = (int)(r / (unsigned)py);
+        j = (int)(r - (unsigned)k * py);
+    }
+}
+
+__device__ __forceinline__ double cell_T(const RebuildArgs& a, long c)
+{
+    return a.T64 ? a.T64[c] : a.t_ref + (double)a.dT[c];
+}
+
+__global__ __launch_bounds__(256) void arrhenius_kernel(RebuildArgs a, ArrArgs arr)
 {
     const long nv = (long)a.nx * a.ny * a.nz;
     const long v = (long)blockIdx.x * 256 + threadIdx.x;
     if (v >= nv) return;
-    double w = kW0 - kW0 * (a.Q[v] / a.qvapor);
-    w = fmin(fmin(w, kW0), a.W[v]);
-    a.W[v] = fmax(w, 0.0);
+    int i, j, k;
+    vox_ijk(v, a.nx, a.ny, i, j, k);
+    const long c = i + a.px * j + a.pxy * k;
+    arrhenius_voxel(arr, v, nv, cell_T(a, c), a.rhokap[c]);
 }
 
-__global__ __launch_bounds__(256) void mask_kernel(RebuildArgs a)
+// What a coupling cycle does per voxel from the temperatures and the rhokap
+// before the removal: the cycle's damage (ARR), the water left (WATER,
+// 3dFD.f90:328) and the removal mask.  None of the three reads what another
+// writes, so they are one pass: at 80^3 each took 4 to 7 us alone, mostly its
+// launch and the same two fields.
+template <bool ARR, bool WATER>
+__global__ __launch_bounds__(256) void update_kernel(RebuildArgs a, ArrArgs arr)
 {
     const long nv = (long)a.nx * a.ny * a.nz;
     const long v = (long)blockIdx.x * 256 + threadIdx.x;
@@ -62,8 +89,15 @@ __global__ __launch_bounds__(256) void mask_kernel(RebuildArgs a)
     vox_ijk(v, a.nx, a.ny, i, j, k);
     const long c = i + a.px * j + a.pxy * k;
     const double* rk = a.rhokap;
-    auto hot = [&](long cc) { return (a.T64 ? a.T64[cc] : a.t_ref + (double)a.dT[cc]) >= a.ablate_K; };
-    const bool b = hot(c) || rk[c] == 0.0;
+    const double T = cell_T(a, c), rc = rk[c];
+    if (ARR) arrhenius_voxel(arr, v, nv, T, rc);
+    if (WATER) {
+        double w = kW0 - kW0 * (a.Q[v] / a.qvapor);
+        w = fmin(fmin(w, kW0), a.W[v]);
+        a.W[v] = fmax(w, 0.0);
+    }
+    auto hot = [&](long cc) { return cell_T(a, cc) >= a.ablate_K; };
+    const bool b = T >= a.ablate_K || rc == 0.0;
     const bool u = rk[c + 1] == 0.0 && rk[c + a.px] == 0.0 && rk[c + a.pxy] == 0.0;
     const bool bx = (i == 1) || hot(c - 1) || rk[c - 1] == 0.0;
     const bool by = (j == 1) || hot(c - a.px) || rk[c - a.px] == 0.0;
@@ -103,6 +137,71 @@ __global__ __launch_bounds__(256) void props_kernel(RebuildArgs a)   // 3dFD.f90
         a.coeff[c] = a.delt / (rho * hc);
         a.mut[v] = (float)rk;
     }
+    a.src[c] = (float)(a.coeff[c] * a.jmean[v]);       // the step's source, with the new delt / (rho c)
+}
+
+// a_f = dscale * kbar/(rhobar*cbar) / h^2 per face for the FP64 step, in the
+// reference's operation order (3dFD.f90:119-129): one thread per halo cell,
+// the face is between c and its + neighbour.
+//
+// PROPS: the rebuild after a cycle, properties and faces in one pass.  A thread
+// writes its own cell's properties and works out its three + neighbours' anew
+// from what they follow from (the mask, T, W), which nothing writes here; where
+// a neighbour keeps its properties, nothing writes those either.  At 80^3 the
+// two passes took 7.3 and 10.5 us, mostly launch and the fields passed between.
+struct CellProps {
+    double kappa, density, heatcap, rhokap;
+};
+template <bool PROPS>
+__global__ __launch_bounds__(256) void coeff64_kernel(Coeff64Args a, RebuildArgs r)
+{
+    const long n = (long)(a.nx + 2) * (a.ny + 2) * (a.nz + 2);
+    const long c = (long)blockIdx.x * 256 + threadIdx.x;
+    if (c >= n) return;
+    int i, j, k;
+    cell_ijk(c, n, a.nx + 2, a.ny + 2, i, j, k);
+    const bool jin = j >= 1 && j <= a.ny, kin = k >= 1 && k <= a.nz, iin = i >= 1 && i <= a.nx;
+    const long v = (i - 1) + (long)a.nx * ((j - 1) + (long)a.ny * (k - 1));    // interior cells
+    auto cell = [&](long cc, long vv, bool interior) {
+        if (PROPS && interior && r.mask[vv]) {
+            const double T = cell_T(r, cc);
+            return CellProps{air_thermal_cond(T), air_density(T), 1.006e3, 0.0};
+        }
+        if (PROPS && interior && r.mode == TAM_THERMAL_WATER) {
+            const double W = r.W[vv], rho = skin_density(W);
+            return CellProps{skin_cond(W, rho), rho, skin_heatcap(W), W * r.mu_water + r.mu_protein};
+        }
+        return CellProps{a.kappa[cc], a.density[cc], a.heatcap[cc], a.removed_inert ? a.rhokap[cc] : 0.0};
+    };
+    const bool in = iin && jin && kin;
+    const CellProps p = cell(c, v, in);
+    if (PROPS && in) {
+        const bool gone = r.mask[v];
+        if (gone || r.mode == TAM_THERMAL_WATER) {
+            r.kappa[c] = p.kappa;
+            r.density[c] = p.density;
+            r.heatcap[c] = p.heatcap;
+            r.rhokap[c] = p.rhokap;
+            r.coeff[c] = r.delt / (p.density * p.heatcap);
+            r.mut[v] = (float)p.rhokap;
+        }
+        if (gone) r.mat[v] = (uint8_t)r.air_id;
+    }
+    // a removed voxel is an interior cell whose rhokap is 0 (halo cells are
+    // empty too, but they carry the boundary condition)
+    const bool rc = a.removed_inert && in && p.rhokap == 0.0;
+    auto face = [&](long o, long ov, bool exists, bool interior, double ih2) {
+        if (!exists || rc) return 0.0;
+        const CellProps m = cell(c + o, v + ov, interior);
+        if (a.removed_inert && interior && m.rhokap == 0.0) return 0.0;
+        const double kb = .5 * (p.kappa + m.kappa);
+        const double db = .5 * (p.density + m.density);
+        const double hb = .5 * (p.heatcap + m.heatcap);
+        return a.dscale * (kb / (db * hb)) * ih2;
+    };
+    a.ax[c] = face(1, 1, i <= a.nx && jin && kin, i + 1 <= a.nx, a.idx2);
+    a.ay[c] = face(a.px, a.nx, j <= a.ny && iin && kin, j + 1 <= a.ny, a.idy2);
+    a.az[c] = face(a.pxy, (long)a.nx * a.ny, k <= a.nz && iin && jin, k + 1 <= a.nz, a.idz2);
 }
 
 // Face coefficients G = delt * s * kbar/(rhobar*cbar) / h^2 (3dFD.f90:119-166),
@@ -112,10 +211,8 @@ __global__ __launch_bounds__(256) void coeff_kernel(CoeffArgs a)
     const long n = (long)(a.nx + 2) * (a.ny + 2) * (a.nz + 2);
     const long c = (long)blockIdx.x * 256 + threadIdx.x;
     if (c >= n) return;
-    const int i = (int)(c % a.px);
-    const long r = c / a.px;
-    const int j = (int)(r % (a.ny + 2));
-    const int k = (int)(r / (a.ny + 2));
+    int i, j, k;
+    cell_ijk(c, n, a.nx + 2, a.ny + 2, i, j, k);
     const double* K = a.kappa;
     const double* D = a.density;
     const double* H = a.heatcap;
@@ -146,13 +243,16 @@ __global__ __launch_bounds__(256) void coeff_kernel(CoeffArgs a)
     }
 }
 
-// jmeanGLOBAL = scale * mu_a * L (mcpolar.f90:174); src = coeff * jmean.
+// jmeanGLOBAL = scale * mu_a * L (mcpolar.f90:174); src = coeff * jmean (FP32 step).
 __global__ __launch_bounds__(256) void normalise_kernel(int nx, int ny, int nz, long px, long pxy,
                                                         const double* tally, const double* rhokap,
                                                         const uint8_t* mat, const double* mua_frac,
                                                         const CycleHdr* dyn, double scale,
-                                                        const double* coeff, double* jmean, float* src)
+                                                        const double* coeff, double* jmean, float* src,
+                                                        unsigned long long* acc, const unsigned long long* counters)
 {
+    // the run's counters join the running sums
+    if (acc && blockIdx.x == 0 && threadIdx.x < TAM_CNT_N) acc[threadIdx.x] += counters[threadIdx.x];
     const long nv = (long)nx * ny * nz;
     const long v = (long)blockIdx.x * 256 + threadIdx.x;
     if (v >= nv) return;
@@ -166,7 +266,7 @@ __global__ __launch_bounds__(256) void normalise_kernel(int nx, int ny, int nz, 
     const double mua = rhokap[c] * mua_frac[mat[v]];
     const double jm = tally[v] * mua * scale;
     jmean[v] = jm;
-    src[c] = (float)(coeff[c] * jm);
+    if (src) src[c] = (float)(coeff[c] * jm);           // the FP64 step multiplies by itself
 }
 
 // A grid-stride sum: one add per block to the one result, at 12 ns each, so the
@@ -203,10 +303,12 @@ __global__ void fill_u64_kernel(unsigned long long* p, long n)
 {
     for (long i = (long)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (long)gridDim.x * blockDim.x) p[i] = 0ull;
 }
-// acc += src over n counters (one block; n is a handful)
-__global__ void acc_u64_kernel(unsigned long long* acc, const unsigned long long* src, long n)
+// f = 0 over n and the run's counters over m
+__global__ void clear_kernel(double* f, long n, unsigned long long* counters, long m)
 {
-    for (long i = threadIdx.x; i < n; i += blockDim.x) acc[i] += src[i];
+    const long q = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    for (long i = q; i < n; i += (long)gridDim.x * blockDim.x) f[i] = 0.0;
+    for (long i = q; i < m; i += (long)gridDim.x * blockDim.x) counters[i] = 0ull;
 }
 
 // Streaming copy (16-byte loads and stores): the measured-bandwidth
@@ -225,14 +327,33 @@ inline unsigned grid_fill(long n)
 
 }  // namespace
 
-hipError_t launch_water_update(const RebuildArgs& a, hipStream_t s)
+hipError_t launch_update(const RebuildArgs& a, const ArrArgs* arr, hipStream_t s)
 {
-    hipLaunchKernelGGL(water_kernel, dim3(grid_for((long)a.nx * a.ny * a.nz)), dim3(256), 0, s, a);
+    const dim3 grid(grid_for((long)a.nx * a.ny * a.nz));
+    const bool water = a.mode == TAM_THERMAL_WATER;
+    const ArrArgs none{};
+    if (arr && water) hipLaunchKernelGGL((update_kernel<true, true>), grid, dim3(256), 0, s, a, *arr);
+    else if (arr) hipLaunchKernelGGL((update_kernel<true, false>), grid, dim3(256), 0, s, a, *arr);
+    else if (water) hipLaunchKernelGGL((update_kernel<false, true>), grid, dim3(256), 0, s, a, none);
+    else hipLaunchKernelGGL((update_kernel<false, false>), grid, dim3(256), 0, s, a, none);
     return hipGetLastError();
 }
-hipError_t launch_removal_mask(const RebuildArgs& a, hipStream_t s)
+hipError_t launch_arrhenius(const RebuildArgs& a, const ArrArgs& arr, hipStream_t s)
 {
-    hipLaunchKernelGGL(mask_kernel, dim3(grid_for((long)a.nx * a.ny * a.nz)), dim3(256), 0, s, a);
+    hipLaunchKernelGGL(arrhenius_kernel, dim3(grid_for((long)a.nx * a.ny * a.nz)), dim3(256), 0, s, a, arr);
+    return hipGetLastError();
+}
+hipError_t launch_coeffs64(const Coeff64Args& a, hipStream_t s)
+{
+    const RebuildArgs none{};
+    hipLaunchKernelGGL((coeff64_kernel<false>), dim3(grid_for((long)(a.nx + 2) * (a.ny + 2) * (a.nz + 2))), dim3(256),
+                       0, s, a, none);
+    return hipGetLastError();
+}
+hipError_t launch_rebuild64(const RebuildArgs& r, const Coeff64Args& a, hipStream_t s)
+{
+    hipLaunchKernelGGL((coeff64_kernel<true>), dim3(grid_for((long)(a.nx + 2) * (a.ny + 2) * (a.nz + 2))), dim3(256),
+                       0, s, a, r);
     return hipGetLastError();
 }
 hipError_t launch_apply_props(const RebuildArgs& a, hipStream_t s)
@@ -248,10 +369,10 @@ hipError_t launch_coeffs(const CoeffArgs& a, hipStream_t s)
 hipError_t launch_normalise(int nx, int ny, int nz, long px, long pxy, const double* tally,
                             const double* rhokap, const uint8_t* mat, const double* mua_frac,
                             const CycleHdr* dyn, double scale, const double* coeff, double* jmean,
-                            float* src, hipStream_t s)
+                            float* src, unsigned long long* acc, const unsigned long long* counters, hipStream_t s)
 {
     hipLaunchKernelGGL(normalise_kernel, dim3(grid_for((long)nx * ny * nz)), dim3(256), 0, s, nx, ny, nz, px,
-                       pxy, tally, rhokap, mat, mua_frac, dyn, scale, coeff, jmean, src);
+                       pxy, tally, rhokap, mat, mua_frac, dyn, scale, coeff, jmean, src, acc, counters);
     return hipGetLastError();
 }
 // k^3 block sums of an interior FP64 field: one workgroup per block
@@ -386,9 +507,9 @@ hipError_t launch_copy(const void* in, void* out, long bytes, hipStream_t s)
     return hipGetLastError();
 }
 
-hipError_t launch_acc_u64(unsigned long long* acc, const unsigned long long* src, long n, hipStream_t s)
+hipError_t launch_clear(double* f, long n, unsigned long long* counters, long m, hipStream_t s)
 {
-    hipLaunchKernelGGL(acc_u64_kernel, dim3(1), dim3(64), 0, s, acc, src, n);
+    hipLaunchKernelGGL(clear_kernel, dim3(grid_fill(n > m ? n : m)), dim3(256), 0, s, f, n, counters, m);
     return hipGetLastError();
 }
 

@@ -79,6 +79,23 @@ __device__ __forceinline__ unsigned thres_chain(double* thres, uint8_t* tmask, l
     return m;
 }
 
+// Damage at the reference cadence (3dFD.f90:447-464): the whole interior over
+// a span `delt`, the full threshold chain at `time`.
+struct ArrArgs {
+    double* omega; double* thres; uint8_t* tmask;
+    double A, dE, R, Tlo, Thi, thr0, thr1, thr2, delt, time;
+    const double* dyn;         // graph replays: (delt, time) from device memory
+};
+__device__ __forceinline__ void arrhenius_voxel(const ArrArgs& a, long v, long nv, double t, double rhokap)
+{
+    const double delt = a.dyn ? a.dyn[0] : a.delt, time = a.dyn ? a.dyn[1] : a.time;
+    double om = a.omega[v];
+    if (t >= a.Tlo && t < a.Thi && rhokap >= 0.0) {
+        om = om + delt * a.A * exp(-a.dE / (a.R * t));
+        a.omega[v] = om;
+    }
+    thres_chain(a.thres, a.tmask, v, nv, om, a.thr0, a.thr1, a.thr2, time, a.tmask[v]);
+}
 
 struct MatEntry {          // per material, in device memory
     float albedo, g, n, mut;
@@ -165,11 +182,10 @@ struct HeatArgs {
     const float2* robin_lut;   // [16] convective ghost (beta, gamma') per top-cell class
     // FP32 pre-tests (conservative) before the exact FP64 tests
     float dT_neg, dT_boil_test, dT_lo_test, dT_hi_test;
-    // graph replays: this step's laser state and time after the step, and the
-    // Arrhenius (delt, time), read from device memory (nullptr: by value)
+    // graph replays: this step's laser state and time after the step, read from
+    // device memory (nullptr: by value)
     const float* dyn_lon;
     const double* dyn_tafter;
-    const double* dyn_arr;
 };
 
 // one instance of a batched heat step: its arguments and its ping-pong pair
@@ -237,6 +253,8 @@ struct RebuildArgs {
     uint8_t* mask;             // interior scratch
     int air_id;                // material id given to removed voxels
     uint8_t* cls;              // halo thermal classes (class mode), nullptr otherwise
+    const double* jmean;       // interior
+    float* src;                // halo: coeff * jmean (FP32 path), nullptr otherwise
 };
 
 struct CoeffArgs {
@@ -363,21 +381,20 @@ const char* heat_tile_name(int tile);
 hipError_t launch_heat64_step(const Heat64Args& a, const double* Tin, double* Tout, double lon,
                               double time_after, int boil, int robin, int damage, int energy, hipStream_t s);
 hipError_t launch_coeffs64(const Coeff64Args& a, hipStream_t s);
-hipError_t launch_acc_u64(unsigned long long* acc, const unsigned long long* src, long n, hipStream_t s);
-hipError_t launch_arrhenius(const HeatArgs& a, const float* T, const double* T64, double delt, double time,
-                            hipStream_t s);
-hipError_t launch_removal_mask(const RebuildArgs& a, hipStream_t s);
+hipError_t launch_clear(double* f, long n, unsigned long long* counters, long m, hipStream_t s);
+hipError_t launch_arrhenius(const RebuildArgs& a, const ArrArgs& arr, hipStream_t s);
+hipError_t launch_update(const RebuildArgs& a, const ArrArgs* arr, hipStream_t s);
 hipError_t launch_apply_props(const RebuildArgs& a, hipStream_t s);
-hipError_t launch_water_update(const RebuildArgs& a, hipStream_t s);
+hipError_t launch_rebuild64(const RebuildArgs& r, const Coeff64Args& a, hipStream_t s);
 hipError_t launch_coeffs(const CoeffArgs& a, hipStream_t s);
 // TAM_CLASS_HOM bits of the interior class bytes from the current classes
 hipError_t launch_class_flags(uint8_t* cls, int nx, int ny, int nz, long px, long pxy, hipStream_t s);
 // dyn (graph replays, else nullptr): scale from dyn->scale; nothing is
 // written when dyn->mc_on == 0 (laser off: jmean keeps its last value)
 hipError_t launch_normalise(int nx, int ny, int nz, long px, long pxy, const double* tally,
-                            const double* rhokap, const uint8_t* mat, const double* mua_tab,
+                            const double* rhokap, const uint8_t* mat, const double* mua_frac,
                             const CycleHdr* dyn, double scale, const double* coeff, double* jmean,
-                            float* src, hipStream_t s);
+                            float* src, unsigned long long* acc, const unsigned long long* counters, hipStream_t s);
 hipError_t launch_fill_f64(double* p, long n, double v, hipStream_t s);
 // error of a call that has no context (read back by tam_last_error(NULL))
 int tam_fail_noctx(int code, const std::string& msg);
