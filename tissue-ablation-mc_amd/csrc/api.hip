@@ -349,6 +349,46 @@ int check_flags(tam_ctx* c)
     return TAM_OK;
 }
 
+// A field to the caller's memory.  Pageable memory goes through the pinned
+// ring; what the device can write by itself is written directly, as is
+// everything where no ring can be had.
+int download(tam_ctx* c, const void* src, StageKind kind, long n, double offset, double* out)
+{
+    if (kind == STAGE_F64) {
+        hipPointerAttribute_t at{};
+        const hipError_t e = hipPointerGetAttributes(&at, out);
+        if (e != hipSuccess) (void)hipGetLastError();          // host memory that HIP does not know
+        if (e == hipSuccess && at.type != hipMemoryTypeUnregistered) {
+            HIPCHK(c, hipMemcpyAsync(out, src, sizeof(double) * (size_t)n, hipMemcpyDeviceToHost, c->stream));
+            HIPCHK(c, hipStreamSynchronize(c->stream));
+            return TAM_OK;
+        }
+    }
+    const hipError_t e = stage_download(c->dev, c->stream, src, kind, n, offset, out);
+    if (e != hipErrorOutOfMemory) {
+        HIPCHK(c, e);
+        return TAM_OK;
+    }
+    const size_t es = kind == STAGE_F64 ? 8 : kind == STAGE_F32 ? 4 : 1;
+    void* at = out;
+    std::vector<char> t;
+    if (kind != STAGE_F64) {
+        try {
+            t.resize(es * (size_t)n);
+        } catch (...) {
+            return fail(c, TAM_ERR_NOMEM, "no memory for the download");
+        }
+        at = t.data();
+    }
+    HIPCHK(c, hipMemcpyAsync(at, src, es * (size_t)n, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    if (kind == STAGE_F32)
+        for (long i = 0; i < n; ++i) out[i] = offset + (double)((const float*)at)[i];
+    else if (kind == STAGE_U8)
+        for (long i = 0; i < n; ++i) out[i] = ((const uint8_t*)at)[i];
+    return TAM_OK;
+}
+
 // src = coeff * jmean (after a property change the per-step source must use
 // the new delt/(rho c), as heat_sim_3D does with coeff(i,j,k)*jtmp)
 __global__ void src_kernel(int nx, int ny, int nz, long px, long pxy, const double* coeff,
@@ -550,6 +590,7 @@ int tam_create(const tam_params* p, tam_ctx** out)
     if (p->device < 0 || p->device >= ndev) return fail(nullptr, TAM_ERR_ARG, "device ordinal out of range");
     tam_ctx* c = new (std::nothrow) tam_ctx();
     if (!c) return fail(nullptr, TAM_ERR_NOMEM, "host allocation failed");
+    stage_user(1);
     c->p = *p;
     c->dev = p->device;
     Dev d(c->dev);
@@ -680,6 +721,7 @@ void tam_destroy(tam_ctx* c)
     if (c->ev0) hipEventDestroy(c->ev0);
     if (c->ev1) hipEventDestroy(c->ev1);
     if (c->stream) hipStreamDestroy(c->stream);
+    stage_user(-1);
     delete c;
 }
 
@@ -1084,25 +1126,12 @@ int tam_download(tam_ctx* c, int32_t field, double* out)
     const double* src64 = nullptr;
     long n = 0;
     switch (field) {
-    case TAM_FIELD_TEMP: {
-        if (c->fp64) {
-            HIPCHK(c, hipMemcpyAsync(out, c->cur64, sizeof(double) * (size_t)H, hipMemcpyDeviceToHost, c->stream));
-            HIPCHK(c, hipStreamSynchronize(c->stream));
-            return TAM_OK;
-        }
-        std::vector<float> t((size_t)H);
-        HIPCHK(c, hipMemcpyAsync(t.data(), c->cur, sizeof(float) * (size_t)H, hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(c, hipStreamSynchronize(c->stream));
-        for (long i = 0; i < H; ++i) out[i] = c->p.t_ref + (double)t[(size_t)i];
-        return TAM_OK;
-    }
-    case TAM_FIELD_MAT: {
-        std::vector<uint8_t> m((size_t)V);
-        HIPCHK(c, hipMemcpyAsync(m.data(), c->mat, (size_t)V, hipMemcpyDeviceToHost, c->stream));
-        HIPCHK(c, hipStreamSynchronize(c->stream));
-        for (long i = 0; i < V; ++i) out[i] = m[(size_t)i];
-        return TAM_OK;
-    }
+    case TAM_FIELD_TEMP:
+        if (!c->fp64) return download(c, c->cur, STAGE_F32, H, c->p.t_ref, out);
+        src64 = c->cur64;
+        n = H;
+        break;
+    case TAM_FIELD_MAT: return download(c, c->mat, STAGE_U8, V, 0.0, out);
     case TAM_FIELD_JMEAN: src64 = c->jmean; n = V; break;
     case TAM_FIELD_TALLY: src64 = c->tally; n = V; break;
     case TAM_FIELD_RHOKAP: src64 = c->rhokap; n = H; break;
@@ -1116,9 +1145,7 @@ int tam_download(tam_ctx* c, int32_t field, double* out)
     case TAM_FIELD_COEFF: src64 = c->coeff; n = H; break;
     default: return fail(c, TAM_ERR_ARG, "unknown field");
     }
-    HIPCHK(c, hipMemcpyAsync(out, src64, sizeof(double) * (size_t)n, hipMemcpyDeviceToHost, c->stream));
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    return TAM_OK;
+    return download(c, src64, STAGE_F64, n, 0.0, out);
 }
 
 int tam_upload(tam_ctx* c, int32_t field, const double* in)

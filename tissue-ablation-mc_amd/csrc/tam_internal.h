@@ -381,6 +381,10 @@ const char* heat_tile_name(int tile);
 hipError_t launch_heat64_step(const Heat64Args& a, const double* Tin, double* Tout, double lon,
                               double time_after, int boil, int robin, int damage, int energy, hipStream_t s);
 hipError_t launch_coeffs64(const Coeff64Args& a, hipStream_t s);
+// field downloads (stage.hip): out[i] = src[i], or offset + src[i] (FP32), or the byte
+enum StageKind { STAGE_F64, STAGE_F32, STAGE_U8 };
+void stage_user(int delta);    // +1 / -1 per context: idle rings go with the last
+hipError_t stage_download(int dev, hipStream_t s, const void* src, StageKind kind, long n, double offset, double* out);
 hipError_t launch_clear(double* f, long n, unsigned long long* counters, long m, hipStream_t s);
 hipError_t launch_arrhenius(const RebuildArgs& a, const ArrArgs& arr, hipStream_t s);
 hipError_t launch_update(const RebuildArgs& a, const ArrArgs* arr, hipStream_t s);
