@@ -77,6 +77,29 @@ __device__ __forceinline__ bf16x8 bload8(Rsrc r, unsigned voff, unsigned soff)
     return __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(r, (int)voff, (int)soff, 0));
 }
 
+// Four consecutive channels co .. co + 3 of voxel m, out of cout: bias, ReLU
+// and mask, one 8-byte store.  The convolutions give the weights to the MFMA
+// as its rows and the voxels as its columns, so a lane holds four channels of
+// one voxel and a wave's store covers whole 32-byte pieces of 16 voxels; with
+// the voxels as rows it held one channel of four voxels, in four 2-byte stores
+// (and loads of the mask).  The products and their order are the same.
+__device__ __forceinline__ void store4(const ConvArgs& a, const f32x4& acc, long m, int co, int cout)
+{
+    const float4 b = a.bias ? *(const float4*)(a.bias + co) : float4{0.f, 0.f, 0.f, 0.f};
+    float v[4] = {acc[0] + b.x, acc[1] + b.y, acc[2] + b.z, acc[3] + b.w};
+    uint2 mk = make_uint2(0u, 0u);
+    if (a.mask) mk = *(const uint2*)(a.mask + m * cout + co);
+    uint2 o;
+    uint16_t* h = (uint16_t*)&o;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        if (a.relu) v[j] = fmaxf(v[j], 0.f);
+        if (a.mask && !(bf2f(((const uint16_t*)&mk)[j]) > 0.f)) v[j] = 0.f;
+        h[j] = f2bf(v[j]);
+    }
+    *(uint2*)(a.y + m * cout + co) = o;
+}
+
 // Forward convolution (and, with flipped weights, the data gradient).
 // A wave computes MT x 16 consecutive voxels of the flattened grid (each
 // lane finds its voxel's x, y, z) for all NT x 16 output channels; CIN is
@@ -155,24 +178,12 @@ __global__ __launch_bounds__(256) void conv_kernel(ConvArgs a)
         for (int t = 0; t < MT; ++t)
 #pragma unroll
             for (int n = 0; n < NT; ++n)
-                acc[t][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[t], bfr[n], acc[t][n], 0, 0, 0);
+                acc[t][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bfr[n], af[t], acc[t][n], 0, 0, 0);
     }
-    // epilogue: lane holds voxels mbase + 16 t + 4 (lane/16) + j, channel 16 n + lane%16
 #pragma unroll
-    for (int n = 0; n < NT; ++n) {
-        const int co = n * 16 + (lane & 15);
-        const float b = a.bias ? a.bias[co] : 0.f;
+    for (int t = 0; t < MT; ++t)
 #pragma unroll
-        for (int t = 0; t < MT; ++t)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const long m = mbase + t * 16 + (lane >> 4) * 4 + j;
-                float v = acc[t][n][j] + b;
-                if (a.relu) v = fmaxf(v, 0.f);
-                if (a.mask && !(bf2f(a.mask[m * a.cout + co]) > 0.f)) v = 0.f;
-                a.y[m * a.cout + co] = f2bf(v);
-            }
-    }
+        for (int n = 0; n < NT; ++n) store4(a, acc[t][n], mbase + t * 16 + (lane & 15), n * 16 + g * 4, NT * 16);
 }
 
 // Convolutions with at most 32 output channels, their input staged in LDS.
@@ -188,17 +199,28 @@ __global__ __launch_bounds__(256) void conv_kernel(ConvArgs a)
 // weights at that (tap, channel)'s place in their tap-major order.
 // Grid edges must be multiples of 16 (x), 8 (y) and 4 (z); CIN a multiple of
 // 16; NT = output channels / 16.
+// 16 to 16 channels at 256^3: 459 us before the staging loads went out together
+// and the stores held four channels, 336 after (1.07 GB: 3.2 of 5.2 TB/s); 48 to
+// 16 1243, 977.  LDS reads take 110 us of the 336 and MFMAs 96; blocks that loop
+// over bricks with the next brick's loads in flight were slower (367).
 template <int CIN, int NT>
-__global__ __launch_bounds__(256) void conv_lds_kernel(ConvArgs a)
+__global__ __launch_bounds__(256, NT == 1 ? 4 : CIN == 16 ? 2 : 3) void conv_lds_kernel(ConvArgs a)
 {
     constexpr int BX = 18, BY = 10, BZ = 6, CG = CIN / 16;
     constexpr int KB = (27 * CIN + 31) / 32;                  // k-blocks of the packed weights
     __shared__ __attribute__((aligned(16))) uint16_t sx[BZ * BY * BX * 16];
     const int W = a.W, H = a.H, D = a.D;
     const int gx = W / 16, gy = H / 8;
-    const int bxi = blockIdx.x % gx, byi = (blockIdx.x / gx) % gy, bzi = blockIdx.x / (gx * gy);
+    // Workgroups go to the 8 XCDs in turn.  With several channel groups each XCD
+    // takes one contiguous eighth of the bricks, whose shared halos then meet in
+    // its L2 (48 channels at 256^3: 1040 us, 977; 96 at 128^3: 400, 382); one
+    // group's input is read fastest in order (338, 347 the other way).
+    const unsigned nb = gridDim.x;
+    const unsigned bid = CG > 1 && nb % 8 == 0 ? blockIdx.x % 8 * (nb / 8) + blockIdx.x / 8 : blockIdx.x;
+    const int bxi = bid % gx, byi = (bid / gx) % gy, bzi = bid / (gx * gy);
     const int x0 = bxi * 16, y0 = byi * 8, z0 = bzi * 4;
-    const int lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15, w = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15;
+    const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6);
     const Rsrc rw = rsrc_n(a.wp, (long)KB * NT * 512 * 2);
     f32x4 acc[8][NT];
 #pragma unroll
@@ -207,15 +229,45 @@ __global__ __launch_bounds__(256) void conv_lds_kernel(ConvArgs a)
         for (int n = 0; n < NT; ++n) acc[t][n] = f32x4{0.f, 0.f, 0.f, 0.f};
     for (int cg = 0; cg < CG; ++cg) {
         if (cg > 0) __syncthreads();                          // the previous group's reads are done
-        // stage channels 16 cg .. 16 cg + 15 of the input brick: 16-byte chunks, two per voxel
-        for (int q = threadIdx.x; q < BZ * BY * BX * 2; q += 256) {
-            const int vq = q >> 1, half = q & 1;
-            const int lx = vq % BX, ly = (vq / BX) % BY, lz = vq / (BX * BY);
-            const int xx = x0 - 1 + lx, yy = y0 - 1 + ly, zz = z0 - 1 + lz;
-            bf16x8 v = {};
-            if (xx >= 0 && xx < W && yy >= 0 && yy < H && zz >= 0 && zz < D)
-                v = *(const bf16x8*)cat_src(a.x, a.x2, a.c1, CIN, D, H, W, xx, yy, zz, 16 * cg + half * 8);
-            *(bf16x8*)(sx + vq * 16 + half * 8) = v;
+        // Stage channels 16 cg .. 16 cg + 15 of the input brick, 16-byte chunks,
+        // two per voxel: all of a thread's loads first, then its LDS writes.
+        // (One load at a time, each waiting for the last, was most of the
+        // kernel.)  A load of a wave takes the 16 inner voxels of two rows: its
+        // base is a scalar, its lane offsets are constants, and rows outside
+        // the grid read zeros past the descriptor's end.
+        {
+            const bool cat = a.x2 != nullptr, coarse = cat && 16 * cg < a.c1;
+            const uint16_t* src = cat && !coarse ? a.x2 : a.x;
+            const int sh = coarse ? 1 : 0, sc = !cat ? CIN : coarse ? a.c1 : CIN - a.c1;
+            const int c0 = cat && !coarse ? 16 * cg - a.c1 : 16 * cg;
+            const int Ws = W >> sh, Hs = H >> sh;
+            const int row = lane >> 5, lx = (lane & 31) >> 1, half = lane & 1;
+            const unsigned off = (unsigned)(((row * Ws + (lx >> sh)) * sc + half * 8) * 2);
+            constexpr unsigned OUT = 0x80000000u;                 // past every descriptor's end
+            constexpr int PAIRS = BZ * BY / 2;                    // row pairs; wave w takes w, w + 4, ..
+            bf16x8 v[(PAIRS + 3) / 4], vh = zero8();
+#pragma unroll
+            for (int i = 0; i < (PAIRS + 3) / 4; ++i) {
+                const int p = min(w + 4 * i, PAIRS - 1), lz = p / (BY / 2), ly = p % (BY / 2) * 2;
+                const int yy = y0 - 1 + ly, zz = z0 - 1 + lz;      // rows yy and yy + 1 of plane zz
+                const uint16_t* base =
+                    src + (((long)(zz >> sh) * Hs + (yy >> sh)) * Ws + (x0 >> sh)) * sc + c0;
+                const Rsrc rs = rsrc_n(base, zz >= 0 && zz < D ? 0x7fffffffL : 0L);
+                const bool outside = (yy < 0 && row == 0) || (yy + 1 >= H && row == 1);
+                v[i] = bload8(rs, outside ? OUT : off, 0);
+            }
+            // the columns beside them: a chunk a thread
+            const int hr = (int)threadIdx.x >> 2, side = ((int)threadIdx.x >> 1) & 1;
+            if (threadIdx.x < BZ * BY * 4) {
+                const int xx = side ? x0 + 16 : x0 - 1, yy = y0 - 1 + hr % BY, zz = z0 - 1 + hr / BY;
+                if (xx >= 0 && xx < W && yy >= 0 && yy < H && zz >= 0 && zz < D)
+                    vh = load8(src + (((long)(zz >> sh) * Hs + (yy >> sh)) * Ws + (xx >> sh)) * sc + c0 + half * 8);
+            }
+            uint16_t* dst = sx + ((w * 2 + row) * BX + 1 + lx) * 16 + half * 8;
+#pragma unroll
+            for (int i = 0; i < (PAIRS + 3) / 4; ++i)
+                if (w + 4 * i < PAIRS) *(bf16x8*)(dst + i * 8 * BX * 16) = v[i];
+            if (threadIdx.x < BZ * BY * 4) *(bf16x8*)(sx + (hr * BX + side * 17) * 16 + half * 8) = vh;
         }
         __syncthreads();
         // k-block kb: lane group g takes tap 2 kb + g / 2, channels 16 cg +
@@ -241,7 +293,7 @@ __global__ __launch_bounds__(256) void conv_lds_kernel(ConvArgs a)
             for (int t = 0; t < 8; ++t)
 #pragma unroll
                 for (int n = 0; n < NT; ++n)
-                    acc[t][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[t], bfr[n], acc[t][n], 0, 0, 0);
+                    acc[t][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bfr[n], af[t], acc[t][n], 0, 0, 0);
         };
         // two fragment sets in turn: the next k-block's reads are in flight
         // while the current one's MFMAs run
@@ -269,23 +321,11 @@ __global__ __launch_bounds__(256) void conv_lds_kernel(ConvArgs a)
             }
         }
     }
-    // lane holds voxels x0 + 4 (lane / 16) + j of row (y0 + t, z0 + w), channel 16 n + lane % 16
-    constexpr int COUT = NT * 16;
 #pragma unroll
-    for (int n = 0; n < NT; ++n) {
-        const int co = n * 16 + (lane & 15);
-        const float bb = a.bias ? a.bias[co] : 0.f;
+    for (int t = 0; t < 8; ++t)
 #pragma unroll
-        for (int t = 0; t < 8; ++t)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const long m = ((long)(z0 + w) * H + (y0 + t)) * W + x0 + (lane >> 4) * 4 + j;
-                float v = acc[t][n][j] + bb;
-                if (a.relu) v = fmaxf(v, 0.f);
-                if (a.mask && !(bf2f(a.mask[m * COUT + co]) > 0.f)) v = 0.f;
-                a.y[m * COUT + co] = f2bf(v);
-            }
-    }
+        for (int n = 0; n < NT; ++n)
+            store4(a, acc[t][n], ((long)(z0 + w) * H + (y0 + t)) * W + x0 + r, n * 16 + g * 4, NT * 16);
 }
 
 struct WgradArgs {
@@ -516,7 +556,9 @@ __global__ __launch_bounds__(256) void wgrad3_kernel(WgradArgs a)
 // one aligned 8-voxel x read plus two dwords give the dx = -1, 0, +1 fragments
 // (v_alignbyte), so one LDS read feeds 3 x COT MFMAs.  NDZ = 1: the block
 // covers all 27 taps; NDZ = 3: the 9 taps of one dz (blockIdx.y % 3).
-// blockIdx.y / NDZ is the input-channel tile.  Blocks loop over bricks and
+// blockIdx.y / NDZ is the input-channel tile.  At 128^3, 16 to 16 channels:
+// 121 us with the staging loads one after the other, 87 with all of them first;
+// 32 outputs 82, 62.  Blocks loop over bricks and
 // keep their sums in registers; at the end the four waves are summed in LDS
 // and each block writes its partial [taps][16][CO] to `part`, which
 // wgradb_reduce_kernel sums into gw.  The blocks of grid row 0 also sum dy
@@ -535,7 +577,7 @@ template <int COT, int NDZ>
 __global__ __launch_bounds__(256) void wgradb_kernel(WgradbArgs a)
 {
     constexpr int CO = COT * 16, NT = 27 / NDZ;
-    constexpr int XR = 24;                                  // x row: element 4 + v holds voxel x0 + v (v = -2 .. 17)
+    constexpr int XR = 24;                                  // x row: element 4 + v holds voxel x0 + v (v = -1 .. 16)
     constexpr int XC = 6 * 10 * XR + 4;                     // x channel stride (elements), padded against bank conflicts
     constexpr int DC = 4 * 8 * 16 + 8;                      // dy channel stride (elements), padded likewise
     constexpr int NW = NT * 16 * CO;                       // weights per partial
@@ -563,27 +605,57 @@ __global__ __launch_bounds__(256) void wgradb_kernel(WgradbArgs a)
     for (long b = blockIdx.x; b < a.bricks; b += gridDim.x) {
         const int x0 = (int)(b % bx) * 16, y0 = (int)((b / bx) % by) * 8, z0 = (int)(b / ((long)bx * by)) * 4;
         __syncthreads();                                    // the last brick's reads are done
-        // x: voxel pairs (x0 + 2p, x0 + 2p + 1), p = -1 .. 8, of 10 rows x 6
+        // x: voxel pairs (x0 + 2p, x0 + 2p + 1), p = 0 .. 7, of 10 rows x 6
         // planes, 16 channels as two 8-channel halves; each lane loads both
-        // voxels' half and writes one dword (the pair) per channel.  Voxels
-        // x0 - 2 and x0 + 17 come along; their halves are never used.
-        for (int q = threadIdx.x; q < 10 * 10 * 6 * 2; q += 256) {
-            const int vq = q >> 1, half = q & 1;
-            const int pp = vq % 10, ly = (vq / 10) % 10, lz = vq / 100;
-            const int xx = x0 + 2 * pp - 2, yy = y0 - 1 + ly, zz = z0 - 1 + lz;
-            uint4 v0 = make_uint4(0u, 0u, 0u, 0u), v1 = make_uint4(0u, 0u, 0u, 0u);
-            if (yy >= 0 && yy < H && zz >= 0 && zz < D) {
-                const int c0 = ct * 16 + half * 8;
-                if (xx >= 0 && xx < W)
-                    v0 = *(const uint4*)cat_src(a.x, a.x2, a.c1, a.cin, D, H, W, xx, yy, zz, c0);
-                if (xx + 1 >= 0 && xx + 1 < W)
-                    v1 = *(const uint4*)cat_src(a.x, a.x2, a.c1, a.cin, D, H, W, xx + 1, yy, zz, c0);
-            }
-            const uint16_t* e0 = (const uint16_t*)&v0;
-            const uint16_t* e1 = (const uint16_t*)&v1;
-            uint16_t* dst = sX + (half * 8) * XC + (lz * 10 + ly) * XR + 2 + 2 * pp;
+        // voxels' half and writes one dword (the pair) per channel.  All loads
+        // go out before the first write (an item at a time, five waits for
+        // memory came one after the other); outside the grid they read the
+        // tensor's first voxel and count as zeros.
+        {
+            const bool cat = a.x2 != nullptr, coarse = cat && ct * 16 < a.c1;
+            const uint16_t* src = cat && !coarse ? a.x2 : a.x;
+            const int sh = coarse ? 1 : 0, sc = !cat ? a.cin : coarse ? a.c1 : a.cin - a.c1;
+            const int c0 = cat && !coarse ? ct * 16 - a.c1 : ct * 16;
+            const int half = threadIdx.x & 1, pp = ((int)threadIdx.x >> 1) & 7;
+            uint4 v0[4], v1[4];
+            bool in[4];
 #pragma unroll
-            for (int j = 0; j < 8; ++j) *(uint32_t*)(dst + j * XC) = (uint32_t)e0[j] | ((uint32_t)e1[j] << 16);
+            for (int i = 0; i < 4; ++i) {
+                const int row = min(((int)threadIdx.x >> 4) + 16 * i, 59);     // the last rows twice, alike
+                const int yy = y0 - 1 + row % 10, zz = z0 - 1 + row / 10;
+                in[i] = yy >= 0 && yy < H && zz >= 0 && zz < D;
+                const long vr = ((long)(zz >> sh) * (H >> sh) + (yy >> sh)) * (W >> sh);
+                const long at = in[i] ? (vr + ((x0 + 2 * pp) >> sh)) * sc : 0;
+                const uint16_t* q = src + at + c0 + half * 8;
+                v0[i] = *(const uint4*)q;
+                v1[i] = *(const uint4*)(q + (coarse ? 0 : sc));
+            }
+            // the columns beside them: a voxel's half a thread
+            const int hr = (int)threadIdx.x >> 2, side = ((int)threadIdx.x >> 1) & 1;
+            uint4 vh = make_uint4(0u, 0u, 0u, 0u);
+            if (threadIdx.x < 240) {
+                const int xx = side ? x0 + 16 : x0 - 1, yy = y0 - 1 + hr % 10, zz = z0 - 1 + hr / 10;
+                if (xx >= 0 && xx < W && yy >= 0 && yy < H && zz >= 0 && zz < D)
+                    vh = *(const uint4*)(src +
+                                         (((long)(zz >> sh) * (H >> sh) + (yy >> sh)) * (W >> sh) + (xx >> sh)) * sc +
+                                         c0 + half * 8);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int row = min(((int)threadIdx.x >> 4) + 16 * i, 59);
+                if (!in[i]) v0[i] = v1[i] = make_uint4(0u, 0u, 0u, 0u);
+                const uint16_t* e0 = (const uint16_t*)&v0[i];
+                const uint16_t* e1 = (const uint16_t*)&v1[i];
+                uint16_t* dst = sX + (half * 8) * XC + row * XR + 4 + 2 * pp;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) *(uint32_t*)(dst + j * XC) = (uint32_t)e0[j] | ((uint32_t)e1[j] << 16);
+            }
+            if (threadIdx.x < 240) {
+                const uint16_t* e = (const uint16_t*)&vh;
+                uint16_t* dst = sX + (half * 8) * XC + hr * XR + (side ? 20 : 3);
+#pragma unroll
+                for (int j = 0; j < 8; ++j) dst[j * XC] = e[j];
+            }
         }
         // dy: voxel pairs of 16 x 8 x 4 voxels, CO channels in 8-channel groups
         for (int q = threadIdx.x; q < 256 * (CO / 8); q += 256) {
