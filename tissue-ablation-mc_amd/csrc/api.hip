@@ -466,9 +466,12 @@ int enqueue_cycle(tam_ctx* c, int* swaps)
     m.dyn_npk = &hdr->npk;
     m.dyn_stream = &hdr->stream;
     HIPCHK(c, launch_mc(m, s));
-    HIPCHK(c, launch_normalise(c->p.nx, c->p.ny, c->p.nz, c->px, c->pxy, c->tally, c->rhokap, c->mat,
-                               c->mua_frac, hdr, 0.0, c->coeff, c->jmean, c->fp64 ? nullptr : c->src, c->cnt_acc,
-                               c->counters, s));
+    // (the FP64 path's first step does it for itself)
+    const bool in_step = c->fp64 && c->cyc_loops > 0;
+    if (!in_step)
+        HIPCHK(c, launch_normalise(c->p.nx, c->p.ny, c->p.nz, c->px, c->pxy, c->tally, c->rhokap, c->mat,
+                                   c->mua_frac, hdr, 0.0, c->coeff, c->jmean, c->fp64 ? nullptr : c->src, c->cnt_acc,
+                                   c->counters, s));
     // heat_sim_3D (3dFD.f90:21-230)
     const int boil = c->p.boil != 0, robin = c->p.robin_top != 0, dmg = c->p.damage_every_step != 0;
     HeatArgs a = heat_args(c);
@@ -478,6 +481,9 @@ int enqueue_cycle(tam_ctx* c, int* swaps)
         if (c->fp64) {
             a64.dyn_lon = lon + k;
             a64.dyn_tafter = ta + k;
+            a64.tally = k == 0 ? c->tally : nullptr;
+            a64.rhokap = c->rhokap; a64.mua_frac = c->mua_frac; a64.mat = c->mat;
+            a64.acc = c->cnt_acc; a64.counters = c->counters; a64.dyn_hdr = hdr;
             HIPCHK(c, launch_heat64_step(a64, c->cur64, c->nxt64, 0.0, 0.0, boil, robin, dmg, 1, s));
             std::swap(c->cur64, c->nxt64);
             ++*swaps;
@@ -1451,7 +1457,9 @@ int tam_tune_heat(tam_ctx* c, int32_t reps, int32_t* tile, int32_t* kz, double* 
         a.eblk = eb;
         a.Q = qs;
         const int boil = c->p.boil != 0, robin = c->p.robin_top != 0, dmg = c->p.damage_every_step != 0;
-        const int kzs[] = {4, 8, 12, 16, 32, 64};
+        // the shallow ones give a grid of some 10^5 voxels enough blocks: 50^3 6.5
+        // us a step at 4, 4.4 at 2; 80^3 5.2 at 4, 4.7 at 3
+        const int kzs[] = {2, 3, 4, 6, 8, 12, 16, 32, 64};
         const bool two_ok = !boil && c->lut;
         const double ta = c->time + c->p.delt;
         for (int t = 0; t < heat_num_tiles() && e == hipSuccess; ++t) {
@@ -1461,7 +1469,7 @@ int tam_tune_heat(tam_ctx* c, int32_t reps, int32_t* tile, int32_t* kz, double* 
             // direct twins on every measured workload; they stay settable
             if (c->lut && t <= 2) continue;
             for (int kk : kzs) {
-                if (kk > c->p.nz && kk != 4) continue;
+                if (kk > c->p.nz && kk != 2) continue;
                 // a two-step candidate launches two steps, timed per step
                 auto run = [&]() {
                     return two ? launch_heat_step2(a, c->cur, c->nxt, 1.f, 1.f, ta, ta + c->p.delt, robin, dmg, 1, t,

@@ -38,6 +38,8 @@ __global__ __launch_bounds__(256) void heat64_kernel(Heat64Args a, const double*
         lon = (double)*a.dyn_lon;
         time_after = *a.dyn_tafter;
     }
+    // the run's counters join the running sums
+    if (a.tally && blockIdx.x == 0 && threadIdx.x < TAM_CNT_N) a.acc[threadIdx.x] += a.counters[threadIdx.x];
     const unsigned nv = (unsigned)a.nx * a.ny * a.nz;          // fewer than 2^32 voxels
     const unsigned v = blockIdx.x * 256 + threadIdx.x;
     double e_out = 0.0;
@@ -63,7 +65,13 @@ __global__ __launch_bounds__(256) void heat64_kernel(Heat64Args a, const double*
         ad = a.ax[c - 1]; dd = a.ax[c]; b = 0.5 * (ad + dd);
         const double u_xx = ad * Tin[c - 1] - 2.0 * b * Tc + dd * Tin[c + 1];
         const double tempIncrease = a.delt * (u_xx + u_yy + u_zz);
-        const double jt = a.jmean[v];
+        double jt;
+        if (a.tally && a.dyn_hdr->mc_on) {               // the first step after a run normalises its tally
+            jt = a.tally[v] * (a.rhokap[c] * a.mua_frac[a.mat[v]]) * a.dyn_hdr->scale;
+            a.jmean[v] = jt;
+        } else {
+            jt = a.jmean[v];
+        }
         double tn = Tc;
         if (Tc < 0.0) a.flags[0] = 1;                    // 3dFD.f90:179-182
         if (BOIL && tn >= 100. + 273. && a.Q[v] < a.qvapor) {

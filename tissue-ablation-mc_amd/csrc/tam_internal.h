@@ -207,6 +207,7 @@ struct HeatBatchEntry {
 // threshold time due outside the Arrhenius window costs the others nothing
 #define TAM_CLASS_DUE 0x40u
 
+struct CycleHdr;
 struct Heat64Args {            // FP64 reference-order step (heat64.hip)
     int nx, ny, nz;
     long px, pxy;
@@ -216,7 +217,7 @@ struct Heat64Args {            // FP64 reference-order step (heat64.hip)
     const double* kappa;       // halo (Robin ghost)
     const double* heatcap;     // halo
     const double* coeff;       // halo, delt/(rho c)
-    const double* jmean;       // interior, W/m^3
+    double* jmean;             // interior, W/m^3
     double* Q;
     double delt, volume_voxel, mass_voxel, qvapor;
     double h_top, t_amb, dz;
@@ -227,6 +228,11 @@ struct Heat64Args {            // FP64 reference-order step (heat64.hip)
     int* flags;
     const float* dyn_lon;      // graph replays, as in HeatArgs
     const double* dyn_tafter;
+    // first step of a captured cycle: the run's tally, normalised here
+    // (mcpolar.f90:174), and its counters; nullptr otherwise
+    const double* tally; const double* rhokap; const double* mua_frac; const uint8_t* mat;
+    unsigned long long* acc; const unsigned long long* counters;
+    const CycleHdr* dyn_hdr;
 };
 
 struct Coeff64Args {
