@@ -52,6 +52,37 @@ struct ConvArgs {
     int c1;
 };
 
+// What the last convolution does with its result when nothing needs its
+// activations afterwards: the head, and where `tally` is given the denoised
+// tally from it.
+struct HeadArgs {
+    const uint16_t* x0;     // network input [nvox][4]
+    const float* hw;        // 16 weights and the bias
+    float* out;
+    const float* mut;
+    double nv;
+    double* tally;
+};
+
+// head: x0[m][0] + hb + sum_c hw[c] a[m][c], a's 16 channels in u0 and u1
+__device__ __forceinline__ float head_value(float first, const float* hw, const uint4& u0, const uint4& u1)
+{
+    float v = first + hw[16];
+    const uint16_t* e0 = (const uint16_t*)&u0;
+    const uint16_t* e1 = (const uint16_t*)&u1;
+#pragma unroll
+    for (int c = 0; c < 8; ++c) v += hw[c] * bf2f(e0[c]);
+#pragma unroll
+    for (int c = 0; c < 8; ++c) v += hw[8 + c] * bf2f(e1[c]);
+    return v;
+}
+
+// the path length that the head's log1p(fluence) stands for; 0 in removed voxels
+__device__ __forceinline__ double tally_value(float v, float mut, double nv)
+{
+    return mut > 0.f ? fmax(expm1((double)v), 0.0) * nv : 0.0;
+}
+
 // 8 channels (c0 .. c0 + 7, c0 a multiple of 8) of fine voxel (xx, yy, zz):
 // from x, or with x2 from cat(upsample2(x), x2)
 __device__ __forceinline__ const uint16_t* cat_src(const uint16_t* x, const uint16_t* x2, int c1, int cin, int D,
@@ -83,7 +114,7 @@ __device__ __forceinline__ bf16x8 bload8(Rsrc r, unsigned voff, unsigned soff)
 // one voxel and a wave's store covers whole 32-byte pieces of 16 voxels; with
 // the voxels as rows it held one channel of four voxels, in four 2-byte stores
 // (and loads of the mask).  The products and their order are the same.
-__device__ __forceinline__ void store4(const ConvArgs& a, const f32x4& acc, long m, int co, int cout)
+__device__ __forceinline__ uint2 out4(const ConvArgs& a, const f32x4& acc, long m, int co, int cout)
 {
     const float4 b = a.bias ? *(const float4*)(a.bias + co) : float4{0.f, 0.f, 0.f, 0.f};
     float v[4] = {acc[0] + b.x, acc[1] + b.y, acc[2] + b.z, acc[3] + b.w};
@@ -97,7 +128,11 @@ __device__ __forceinline__ void store4(const ConvArgs& a, const f32x4& acc, long
         if (a.mask && !(bf2f(((const uint16_t*)&mk)[j]) > 0.f)) v[j] = 0.f;
         h[j] = f2bf(v[j]);
     }
-    *(uint2*)(a.y + m * cout + co) = o;
+    return o;
+}
+__device__ __forceinline__ void store4(const ConvArgs& a, const f32x4& acc, long m, int co, int cout)
+{
+    *(uint2*)(a.y + m * cout + co) = out4(a, acc, m, co, cout);
 }
 
 // Forward convolution (and, with flipped weights, the data gradient).
@@ -203,9 +238,16 @@ __global__ __launch_bounds__(256) void conv_kernel(ConvArgs a)
 // and the stores held four channels, 336 after (1.07 GB: 3.2 of 5.2 TB/s); 48 to
 // 16 1243, 977.  LDS reads take 110 us of the 336 and MFMAs 96; blocks that loop
 // over bricks with the next brick's loads in flight were slower (367).
-template <int CIN, int NT>
-__global__ __launch_bounds__(256, NT == 1 ? 4 : CIN == 16 ? 2 : 3) void conv_lds_kernel(ConvArgs a)
+// FIRST: the first layer, whose input holds 4 of the 16 channels per voxel (8
+// bytes to write and read instead of 32; the others are zero in LDS).
+// HEAD: the last layer without a later backward pass; the output goes through
+// LDS to the head instead of to memory and back (at 256^3 0.54 GB each way:
+// 337 us, the head 228 and the tally 61 apart, 424 together).
+enum { CONV_PLAIN, CONV_FIRST, CONV_HEAD };
+template <int CIN, int NT, int KIND>
+__global__ __launch_bounds__(256, NT == 1 ? 4 : CIN == 16 ? 2 : 3) void conv_lds_kernel(ConvArgs a, HeadArgs hd)
 {
+    constexpr bool FIRST = KIND == CONV_FIRST, HEAD = KIND == CONV_HEAD;
     constexpr int BX = 18, BY = 10, BZ = 6, CG = CIN / 16;
     constexpr int KB = (27 * CIN + 31) / 32;                  // k-blocks of the packed weights
     __shared__ __attribute__((aligned(16))) uint16_t sx[BZ * BY * BX * 16];
@@ -238,7 +280,7 @@ __global__ __launch_bounds__(256, NT == 1 ? 4 : CIN == 16 ? 2 : 3) void conv_lds
         {
             const bool cat = a.x2 != nullptr, coarse = cat && 16 * cg < a.c1;
             const uint16_t* src = cat && !coarse ? a.x2 : a.x;
-            const int sh = coarse ? 1 : 0, sc = !cat ? CIN : coarse ? a.c1 : CIN - a.c1;
+            const int sh = coarse ? 1 : 0, sc = !cat ? (FIRST ? 4 : CIN) : coarse ? a.c1 : CIN - a.c1;
             const int c0 = cat && !coarse ? 16 * cg - a.c1 : 16 * cg;
             const int Ws = W >> sh, Hs = H >> sh;
             const int row = lane >> 5, lx = (lane & 31) >> 1, half = lane & 1;
@@ -254,14 +296,27 @@ __global__ __launch_bounds__(256, NT == 1 ? 4 : CIN == 16 ? 2 : 3) void conv_lds
                     src + (((long)(zz >> sh) * Hs + (yy >> sh)) * Ws + (x0 >> sh)) * sc + c0;
                 const Rsrc rs = rsrc_n(base, zz >= 0 && zz < D ? 0x7fffffffL : 0L);
                 const bool outside = (yy < 0 && row == 0) || (yy + 1 >= H && row == 1);
-                v[i] = bload8(rs, outside ? OUT : off, 0);
+                if constexpr (FIRST) {
+                    typedef unsigned v2u __attribute__((ext_vector_type(2)));
+                    const v2u q = __builtin_amdgcn_raw_buffer_load_b64(rs, outside || half ? (int)OUT : (int)off, 0, 0);
+                    v[i] = __builtin_bit_cast(bf16x8, make_uint4(q.x, q.y, 0u, 0u));
+                } else {
+                    v[i] = bload8(rs, outside ? OUT : off, 0);
+                }
             }
             // the columns beside them: a chunk a thread
             const int hr = (int)threadIdx.x >> 2, side = ((int)threadIdx.x >> 1) & 1;
             if (threadIdx.x < BZ * BY * 4) {
                 const int xx = side ? x0 + 16 : x0 - 1, yy = y0 - 1 + hr % BY, zz = z0 - 1 + hr / BY;
-                if (xx >= 0 && xx < W && yy >= 0 && yy < H && zz >= 0 && zz < D)
-                    vh = load8(src + (((long)(zz >> sh) * Hs + (yy >> sh)) * Ws + (xx >> sh)) * sc + c0 + half * 8);
+                if (xx >= 0 && xx < W && yy >= 0 && yy < H && zz >= 0 && zz < D) {
+                    const long at = (((long)(zz >> sh) * Hs + (yy >> sh)) * Ws + (xx >> sh)) * sc + c0;
+                    if constexpr (FIRST) {
+                        const uint2 u = half ? make_uint2(0u, 0u) : *(const uint2*)(src + at);
+                        vh = __builtin_bit_cast(bf16x8, make_uint4(u.x, u.y, 0u, 0u));
+                    } else {
+                        vh = load8(src + at + half * 8);
+                    }
+                }
             }
             uint16_t* dst = sx + ((w * 2 + row) * BX + 1 + lx) * 16 + half * 8;
 #pragma unroll
@@ -321,11 +376,26 @@ __global__ __launch_bounds__(256, NT == 1 ? 4 : CIN == 16 ? 2 : 3) void conv_lds
             }
         }
     }
+    if constexpr (HEAD) {
+        __syncthreads();                                      // the input's reads are done
 #pragma unroll
-    for (int t = 0; t < 8; ++t)
+        for (int t = 0; t < 8; ++t)
+            *(uint2*)(sx + ((w * 8 + t) * 16 + r) * 16 + g * 4) = out4(a, acc[t][0], 0, g * 4, 16);
+        __syncthreads();
+        for (int q = threadIdx.x; q < 512; q += 256) {
+            const long m = ((long)(z0 + (q >> 7)) * H + (y0 + ((q >> 4) & 7))) * W + x0 + (q & 15);
+            const float v = head_value(bf2f(hd.x0[m * 4]), hd.hw, *(const uint4*)(sx + q * 16),
+                                       *(const uint4*)(sx + q * 16 + 8));
+            if (hd.tally) hd.tally[m] = tally_value(v, hd.mut[m], hd.nv);
+            else hd.out[m] = v;
+        }
+    } else {
 #pragma unroll
-        for (int n = 0; n < NT; ++n)
-            store4(a, acc[t][n], ((long)(z0 + w) * H + (y0 + t)) * W + x0 + r, n * 16 + g * 4, NT * 16);
+        for (int t = 0; t < 8; ++t)
+#pragma unroll
+            for (int n = 0; n < NT; ++n)
+                store4(a, acc[t][n], ((long)(z0 + w) * H + (y0 + t)) * W + x0 + r, n * 16 + g * 4, NT * 16);
+    }
 }
 
 struct WgradArgs {
@@ -573,7 +643,8 @@ struct WgradbArgs {
     int c1;
 };
 
-template <int COT, int NDZ>
+// FIRST: the first layer's input, 4 of the 16 channels per voxel.
+template <int COT, int NDZ, bool FIRST>
 __global__ __launch_bounds__(256) void wgradb_kernel(WgradbArgs a)
 {
     constexpr int CO = COT * 16, NT = 27 / NDZ;
@@ -614,7 +685,7 @@ __global__ __launch_bounds__(256) void wgradb_kernel(WgradbArgs a)
         {
             const bool cat = a.x2 != nullptr, coarse = cat && ct * 16 < a.c1;
             const uint16_t* src = cat && !coarse ? a.x2 : a.x;
-            const int sh = coarse ? 1 : 0, sc = !cat ? a.cin : coarse ? a.c1 : a.cin - a.c1;
+            const int sh = coarse ? 1 : 0, sc = !cat ? (FIRST ? 4 : a.cin) : coarse ? a.c1 : a.cin - a.c1;
             const int c0 = cat && !coarse ? ct * 16 - a.c1 : ct * 16;
             const int half = threadIdx.x & 1, pp = ((int)threadIdx.x >> 1) & 7;
             uint4 v0[4], v1[4];
@@ -626,23 +697,38 @@ __global__ __launch_bounds__(256) void wgradb_kernel(WgradbArgs a)
                 in[i] = yy >= 0 && yy < H && zz >= 0 && zz < D;
                 const long vr = ((long)(zz >> sh) * (H >> sh) + (yy >> sh)) * (W >> sh);
                 const long at = in[i] ? (vr + ((x0 + 2 * pp) >> sh)) * sc : 0;
-                const uint16_t* q = src + at + c0 + half * 8;
-                v0[i] = *(const uint4*)q;
-                v1[i] = *(const uint4*)(q + (coarse ? 0 : sc));
+                if constexpr (FIRST) {                       // 4 channels a voxel, the pair in 16 bytes
+                    v0[i] = *(const uint4*)(src + at);
+                } else {
+                    const uint16_t* q = src + at + c0 + half * 8;
+                    v0[i] = *(const uint4*)q;
+                    v1[i] = *(const uint4*)(q + (coarse ? 0 : sc));
+                }
             }
             // the columns beside them: a voxel's half a thread
             const int hr = (int)threadIdx.x >> 2, side = ((int)threadIdx.x >> 1) & 1;
             uint4 vh = make_uint4(0u, 0u, 0u, 0u);
             if (threadIdx.x < 240) {
                 const int xx = side ? x0 + 16 : x0 - 1, yy = y0 - 1 + hr % 10, zz = z0 - 1 + hr / 10;
-                if (xx >= 0 && xx < W && yy >= 0 && yy < H && zz >= 0 && zz < D)
-                    vh = *(const uint4*)(src +
-                                         (((long)(zz >> sh) * (H >> sh) + (yy >> sh)) * (W >> sh) + (xx >> sh)) * sc +
-                                         c0 + half * 8);
+                if (xx >= 0 && xx < W && yy >= 0 && yy < H && zz >= 0 && zz < D) {
+                    const uint16_t* q =
+                        src + (((long)(zz >> sh) * (H >> sh) + (yy >> sh)) * (W >> sh) + (xx >> sh)) * sc + c0;
+                    if constexpr (FIRST) {
+                        const uint2 u = half ? make_uint2(0u, 0u) : *(const uint2*)q;
+                        vh = make_uint4(u.x, u.y, 0u, 0u);
+                    } else {
+                        vh = *(const uint4*)(q + half * 8);
+                    }
+                }
             }
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int row = min(((int)threadIdx.x >> 4) + 16 * i, 59);
+                if constexpr (FIRST) {
+                    v1[i] = make_uint4(v0[i].z, v0[i].w, 0u, 0u);
+                    v0[i] = make_uint4(v0[i].x, v0[i].y, 0u, 0u);
+                    in[i] = in[i] && half == 0;
+                }
                 if (!in[i]) v0[i] = v1[i] = make_uint4(0u, 0u, 0u, 0u);
                 const uint16_t* e0 = (const uint16_t*)&v0[i];
                 const uint16_t* e1 = (const uint16_t*)&v1[i];
@@ -903,27 +989,14 @@ __global__ void skip_pool_bwd_kernel(const uint16_t* gcat, int Ccat, int C1, con
     }
 }
 
-// features (4 x nvox FP32, or built from a context) -> 16-channel input
+// features (4 x nvox FP32) -> the network's input, 4 BF16 channels a voxel
 __global__ void pack_input_kernel(const float* f, long nvox, uint16_t* x0)
 {
     for (long m = (long)blockIdx.x * blockDim.x + threadIdx.x; m < nvox; m += (long)gridDim.x * blockDim.x) {
-        uint16_t v[16];
-        for (int c = 0; c < 16; ++c) v[c] = c < 4 ? f2bf(f[(long)c * nvox + m]) : (uint16_t)0;
-        uint4* o = (uint4*)(x0 + m * 16);
-        o[0] = *(uint4*)&v[0];
-        o[1] = *(uint4*)&v[8];
-    }
-}
-
-// dataset slot (4 BF16 features + BF16 target per voxel) -> 16-channel input
-__global__ void pack_slot_kernel(const uint16_t* feat, long nvox, uint16_t* x0)
-{
-    for (long m = (long)blockIdx.x * blockDim.x + threadIdx.x; m < nvox; m += (long)gridDim.x * blockDim.x) {
-        uint16_t v[16];
-        for (int c = 0; c < 16; ++c) v[c] = c < 4 ? feat[m * 4 + c] : (uint16_t)0;
-        uint4* o = (uint4*)(x0 + m * 16);
-        o[0] = *(uint4*)&v[0];
-        o[1] = *(uint4*)&v[8];
+        uint2 o;
+        uint16_t* v = (uint16_t*)&o;
+        for (int c = 0; c < 4; ++c) v[c] = f2bf(f[(long)c * nvox + m]);
+        *(uint2*)(x0 + m * 4) = o;
     }
 }
 
@@ -942,7 +1015,7 @@ __global__ void ctx_features_kernel(const double* tally, const float* mut, const
     }
 }
 
-// the same features written straight into the 16-channel BF16 input (the
+// the same features written straight into the BF16 input (the
 // forward-only path: no FP32 staging)
 __global__ void ctx_input_kernel(const double* tally, const float* mut, const uint8_t* mat, const MatEntry* mtab,
                                  long nvox, double inv_nv, uint16_t* x0)
@@ -950,7 +1023,8 @@ __global__ void ctx_input_kernel(const double* tally, const float* mut, const ui
     for (long m = (long)blockIdx.x * blockDim.x + threadIdx.x; m < nvox; m += (long)gridDim.x * blockDim.x) {
         const float mu = mut[m], alb = mtab[mat[m]].albedo;
         const float mua = mu * (1.f - alb), mus = mu * alb;
-        uint16_t v[16];
+        uint2 o;
+        uint16_t* v = (uint16_t*)&o;
         // round to FP32 first, as the staged path stores it: the empty asm keeps
         // the compiler from folding double -> float -> BF16 into one rounding
         float l = (float)log1p(tally[m] * inv_nv);
@@ -959,11 +1033,7 @@ __global__ void ctx_input_kernel(const double* tally, const float* mut, const ui
         v[1] = f2bf(log10f(fmaxf(mua, 1e-3f)));
         v[2] = f2bf(log10f(fmaxf(mus, 1e-2f)) - 2.f);
         v[3] = f2bf(5.f * (mtab[mat[m]].g - 0.8f));
-#pragma unroll
-        for (int c = 4; c < 16; ++c) v[c] = 0;
-        uint4* o = (uint4*)(x0 + m * 16);
-        o[0] = *(uint4*)&v[0];
-        o[1] = *(uint4*)&v[8];
+        *(uint2*)(x0 + m * 4) = o;
     }
 }
 
@@ -977,8 +1047,8 @@ __global__ void store_slot_kernel(const float* f, const double* tally_hi, double
     }
 }
 
-// head: out[m] = x0[m][0] + hb + sum_c hw[c] a[m][c]; optional L1 against
-// an FP32 target with the loss summed into *loss
+// head of a training step: out[m], and its L1 against an FP32 target with the
+// loss summed into *loss (the input's into *base)
 __global__ __launch_bounds__(256) void head_kernel(const uint16_t* x0, const uint16_t* a, const float* hw,
                                                    long nvox, float* out, const float* tgt, double* loss,
                                                    double* base)
@@ -986,22 +1056,13 @@ __global__ __launch_bounds__(256) void head_kernel(const uint16_t* x0, const uin
     __shared__ double s[2][256];
     double l = 0.0, lb = 0.0;
     for (long m = (long)blockIdx.x * 256 + threadIdx.x; m < nvox; m += (long)gridDim.x * 256) {
-        float v = bf2f(x0[m * 16]) + hw[16];
-        const uint4 u0 = *(const uint4*)(a + m * 16), u1 = *(const uint4*)(a + m * 16 + 8);
-        const uint16_t* e0 = (const uint16_t*)&u0;
-        const uint16_t* e1 = (const uint16_t*)&u1;
-#pragma unroll
-        for (int c = 0; c < 8; ++c) v += hw[c] * bf2f(e0[c]);
-#pragma unroll
-        for (int c = 0; c < 8; ++c) v += hw[8 + c] * bf2f(e1[c]);
+        const float first = bf2f(x0[m * 4]);
+        const float v = head_value(first, hw, *(const uint4*)(a + m * 16), *(const uint4*)(a + m * 16 + 8));
         out[m] = v;
-        if (tgt) {
-            const float t = tgt[m];
-            l += fabsf(v - t);
-            lb += fabsf(bf2f(x0[m * 16]) - t);
-        }
+        const float t = tgt[m];
+        l += fabsf(v - t);
+        lb += fabsf(first - t);
     }
-    if (!tgt) return;
     s[0][threadIdx.x] = l;
     s[1][threadIdx.x] = lb;
     __syncthreads();
@@ -1118,13 +1179,6 @@ __global__ void fill_f64k(double* p, long n, double v)
     for (long q = (long)blockIdx.x * blockDim.x + threadIdx.x; q < n; q += (long)gridDim.x * blockDim.x) p[q] = v;
 }
 
-// prediction log(1 + phi) -> path length per voxel (zero where mu_t = 0)
-__global__ void write_tally_kernel(const float* out, const float* mut, long nvox, double nv, double* tally)
-{
-    for (long m = (long)blockIdx.x * blockDim.x + threadIdx.x; m < nvox; m += (long)gridDim.x * blockDim.x)
-        tally[m] = mut[m] > 0.f ? fmax(expm1((double)out[m]), 0.0) * nv : 0.0;
-}
-
 unsigned grid_of(long n, int per = 256)
 {
     long b = (n + per - 1) / per;
@@ -1191,7 +1245,7 @@ thread_local std::string g_dn_err;
 
 hipError_t conv_launch(tam_dn* n, const uint16_t* x, int lvl, int cin, const uint16_t* wp, int kb, const float* bias,
                        int cout, int relu, const uint16_t* mask, uint16_t* y, const uint16_t* x2 = nullptr,
-                       int c1 = 0)
+                       int c1 = 0, int c4 = 0, const HeadArgs* head = nullptr)
 {
     ConvArgs a{x, wp, bias, mask, y, n->D[lvl], n->H[lvl], n->W[lvl], cin, cout, kb, relu, x2, c1};
     const long nv = n->nv[lvl];
@@ -1207,7 +1261,15 @@ hipError_t conv_launch(tam_dn* n, const uint16_t* x, int lvl, int cin, const uin
         // LDS-staged input for the layers with 16 or 32 output channels (48
         // outputs as NT = 3 needs ~260 VGPRs there: the global form is faster)
         const dim3 grid((unsigned)((W / 16) * (H / 8) * (D / 4)));
-#define CL(CI, NT_) hipLaunchKernelGGL((conv_lds_kernel<CI, NT_>), grid, dim3(256), 0, n->stream, a)
+#define CL(CI, NT_) hipLaunchKernelGGL((conv_lds_kernel<CI, NT_, CONV_PLAIN>), grid, dim3(256), 0, n->stream, a, HeadArgs{})
+        if (head || c4) {
+            if (cin != 16 || cout != 16 || (head && c4)) return hipErrorInvalidValue;
+            if (head)
+                hipLaunchKernelGGL((conv_lds_kernel<16, 1, CONV_HEAD>), grid, dim3(256), 0, n->stream, a, *head);
+            else
+                hipLaunchKernelGGL((conv_lds_kernel<16, 1, CONV_FIRST>), grid, dim3(256), 0, n->stream, a, HeadArgs{});
+            return hipGetLastError();
+        }
         switch (cin * 1000 + cout) {
         case 16016: CL(16, 1); return hipGetLastError();
         case 16032: CL(16, 2); return hipGetLastError();
@@ -1218,7 +1280,8 @@ hipError_t conv_launch(tam_dn* n, const uint16_t* x, int lvl, int cin, const uin
         }
 #undef CL
     }
-    if (x2) return hipErrorInvalidValue;  // a concatenated input is read by the LDS form only
+    // read or done by the LDS form only; the full grid's edges are multiples of 32
+    if (x2 || c4 || head) return hipErrorInvalidValue;
     switch (cin * 1000 + cout) {
     case 16016: CV(16, 1, 4); break;      // layers 0, 1, 9 and the data gradients of 0, 1, 9
     case 16032: CV(16, 2, 4); break;      // layer 2
@@ -1267,7 +1330,7 @@ bool brick_plan(int D, int H, int W, int cin, int cout, BrickPlan* bp)
 // weight gradient of one layer into gw; the brick form also sums the bias
 // gradient into gb and says so in *bias_done
 hipError_t wgrad_launch(tam_dn* n, const uint16_t* x, const uint16_t* dy, int lvl, int cin, int cout, float* gw,
-                        float* gb, bool* bias_done, const uint16_t* x2 = nullptr, int c1 = 0)
+                        float* gb, bool* bias_done, const uint16_t* x2 = nullptr, int c1 = 0, int c4 = 0)
 {
     *bias_done = false;
     BrickPlan bp;
@@ -1276,10 +1339,12 @@ hipError_t wgrad_launch(tam_dn* n, const uint16_t* x, const uint16_t* dy, int lv
         WgradbArgs b{x, dy, n->wpart, n->D[lvl], n->H[lvl], n->W[lvl], cin, cout,
                      (long)(n->W[lvl] / 16) * (n->H[lvl] / 8) * (n->D[lvl] / 4), x2, c1};
         const dim3 grid((unsigned)bp.nb, (unsigned)bp.ny);
-        if (cout == 16 && bp.ndz == 1) hipLaunchKernelGGL((wgradb_kernel<1, 1>), grid, dim3(256), 0, n->stream, b);
-        else if (cout == 16) hipLaunchKernelGGL((wgradb_kernel<1, 3>), grid, dim3(256), 0, n->stream, b);
-        else if (cout == 32) hipLaunchKernelGGL((wgradb_kernel<2, 3>), grid, dim3(256), 0, n->stream, b);
-        else hipLaunchKernelGGL((wgradb_kernel<4, 3>), grid, dim3(256), 0, n->stream, b);
+        if (c4 && (cout != 16 || bp.ndz != 1)) return hipErrorInvalidValue;
+        if (c4) hipLaunchKernelGGL((wgradb_kernel<1, 1, true>), grid, dim3(256), 0, n->stream, b);
+        else if (cout == 16 && bp.ndz == 1) hipLaunchKernelGGL((wgradb_kernel<1, 1, false>), grid, dim3(256), 0, n->stream, b);
+        else if (cout == 16) hipLaunchKernelGGL((wgradb_kernel<1, 3, false>), grid, dim3(256), 0, n->stream, b);
+        else if (cout == 32) hipLaunchKernelGGL((wgradb_kernel<2, 3, false>), grid, dim3(256), 0, n->stream, b);
+        else hipLaunchKernelGGL((wgradb_kernel<4, 3, false>), grid, dim3(256), 0, n->stream, b);
         // ~1024 reduction blocks: each weight's nb partials split over ksplit of them
         const unsigned qb = grid_of(bp.ny * bp.per);
         long ks = 1024 / (long)qb;
@@ -1290,7 +1355,7 @@ hipError_t wgrad_launch(tam_dn* n, const uint16_t* x, const uint16_t* dy, int lv
         *bias_done = true;
         return hipGetLastError();
     }
-    if (x2) return hipErrorInvalidValue;  // a concatenated input is read by the brick form only
+    if (x2 || c4) return hipErrorInvalidValue;  // read by the brick form only
     WgradArgs a{x, dy, gw, n->D[lvl], n->H[lvl], n->W[lvl], cin, cout, 0, 0};
     a.blocks = n->nv[lvl] / 32;
     // rows of whole 32-voxel segments: one workgroup per (dz, dy) covers the three dx taps, ~288 per (dz, dy);
@@ -1339,15 +1404,21 @@ hipError_t repack(tam_dn* n)
     return hipGetLastError();
 }
 
-// forward from n->x0; with tgt: the L1 loss summed into red[0] (input's in red[1])
-hipError_t forward(tam_dn* n, const float* tgt)
+// forward from the input x0 ([nvox][4]).  With tgt: activations kept for
+// backward(), the prediction in n->out and the L1 loss summed into red[0]
+// (input's in red[1]).  Without: the prediction in n->out, or with c the
+// denoised tally in c (nv: packets times the voxel volume).
+hipError_t forward(tam_dn* n, const uint16_t* x0, const float* tgt, tam_ctx* c = nullptr, double nv = 0.0)
 {
     hipError_t e;
     auto conv = [&](int l, const uint16_t* in, uint16_t* o) {
         const Layer& L = n->L[l];
         return conv_launch(n, in, L.level, L.cin, L.wf, L.kb_f, n->p + L.b_off, L.cout, 1, nullptr, o);
     };
-    if ((e = conv(0, n->x0, n->a[0])) != hipSuccess) return e;
+    const Layer& L0 = n->L[0];
+    if ((e = conv_launch(n, x0, L0.level, L0.cin, L0.wf, L0.kb_f, n->p + L0.b_off, L0.cout, 1, nullptr, n->a[0], nullptr,
+                         0, 1)) != hipSuccess)
+        return e;
     if ((e = conv(1, n->a[0], n->a[1])) != hipSuccess) return e;
     hipLaunchKernelGGL(pool_kernel, dim3(grid_of(n->nv[1] * 16 / 8)), dim3(256), 0, n->stream, n->a[1], n->D[0], n->H[0],
                        n->W[0], 16, n->p1);
@@ -1365,31 +1436,35 @@ hipError_t forward(tam_dn* n, const float* tgt)
     if ((e = conv_cat(6, n->a[5], 64, n->a[3], n->a[6])) != hipSuccess) return e;
     if ((e = conv(7, n->a[6], n->a[7])) != hipSuccess) return e;
     if ((e = conv_cat(8, n->a[7], 32, n->a[1], n->a[8])) != hipSuccess) return e;
+    if (!tgt) {
+        const HeadArgs h{x0, n->p + n->head_off, n->out, c ? c->mut : nullptr, nv, c ? c->tally : nullptr};
+        const Layer& L9 = n->L[9];
+        return conv_launch(n, n->a[8], L9.level, L9.cin, L9.wf, L9.kb_f, n->p + L9.b_off, L9.cout, 1, nullptr, nullptr,
+                           nullptr, 0, 0, &h);
+    }
     if ((e = conv(9, n->a[8], n->a[9])) != hipSuccess) return e;
-    if (tgt) hipLaunchKernelGGL(fill_f64k, dim3(1), dim3(64), 0, n->stream, n->red, 2L, 0.0);
-    // with a target every workgroup ends in atomics onto two addresses: at most
-    // 1024 workgroups then; without one, a workgroup per 256 voxels (up to
-    // grid_of's cap) so the loads of many voxels are in flight at once
+    hipLaunchKernelGGL(fill_f64k, dim3(1), dim3(64), 0, n->stream, n->red, 2L, 0.0);
+    // every workgroup ends in atomics onto two addresses: at most 1024 workgroups
     const unsigned hg = grid_of(n->nv[0]);
-    const unsigned hb = tgt && hg > 1024u ? 1024u : hg;
-    hipLaunchKernelGGL(head_kernel, dim3(hb), dim3(256), 0, n->stream, n->x0, n->a[9],
+    hipLaunchKernelGGL(head_kernel, dim3(hg > 1024u ? 1024u : hg), dim3(256), 0, n->stream, x0, n->a[9],
                        n->p + n->head_off, n->nv[0], n->out, tgt, n->red, n->red + 1);
     return hipGetLastError();
 }
 
-// backward after forward(tgt): gradients of the mean L1 into n->g
-hipError_t backward(tam_dn* n, const float* tgt)
+// backward after forward(x0, tgt): gradients of the mean L1 into n->g
+hipError_t backward(tam_dn* n, const uint16_t* x0, const float* tgt)
 {
     hipError_t e;
     hipLaunchKernelGGL(fill_f32k, dim3(grid_of(n->nparam)), dim3(256), 0, n->stream, n->g, n->nparam, 0.f);
     const unsigned hb = grid_of(n->nv[0]) < 1024u ? grid_of(n->nv[0]) : 1024u;
     hipLaunchKernelGGL(head_bwd_kernel, dim3(hb), dim3(256), 0, n->stream, n->out, tgt, n->a[9],
                        n->p + n->head_off, n->nv[0], n->d[9], n->g + n->head_off);
-    auto grads = [&](int l, const uint16_t* in, const uint16_t* dl, const uint16_t* x2 = nullptr, int c1 = 0) {
+    auto grads = [&](int l, const uint16_t* in, const uint16_t* dl, const uint16_t* x2 = nullptr, int c1 = 0,
+                     int c4 = 0) {
         const Layer& L = n->L[l];
         bool bias_done = false;
         hipError_t r = wgrad_launch(n, in, dl, L.level, L.cin, L.cout, n->g + L.w_off, n->g + L.b_off, &bias_done,
-                                    x2, c1);
+                                    x2, c1, c4);
         if (r != hipSuccess || bias_done) return r;
         // at most 1024 blocks: every block ends in `cout` atomics onto the same few addresses, which serialise
         if (L.cout % 8 != 0 || L.cout > 2048) return hipErrorInvalidValue;
@@ -1429,7 +1504,7 @@ hipError_t backward(tam_dn* n, const float* tgt)
                        n->gp1, n->a[1], n->D[0], n->H[0], n->W[0], 16, n->d[1]);
     if ((e = grads(1, n->a[0], n->d[1])) != hipSuccess) return e;
     if ((e = dgrad(1, n->d[1], n->a[0], n->d[0])) != hipSuccess) return e;
-    if ((e = grads(0, n->x0, n->d[0])) != hipSuccess) return e;
+    if ((e = grads(0, x0, n->d[0], nullptr, 0, 1)) != hipSuccess) return e;
     return hipGetLastError();
 }
 
@@ -1533,7 +1608,7 @@ int tam_dn_create(int32_t device, int32_t nx, int32_t ny, int32_t nz, int32_t ca
         al((void**)&n->a[l], 2ull * n->nv[L.level] * L.cout);
         al((void**)&n->d[l], 2ull * n->nv[L.level] * L.cout);
     }
-    al((void**)&n->x0, 2ull * n->nv[0] * 16);
+    al((void**)&n->x0, 2ull * n->nv[0] * 4);
     al((void**)&n->p1, 2ull * n->nv[1] * 16);
     al((void**)&n->p3, 2ull * n->nv[2] * 32);
     al((void**)&n->gc6, 2ull * n->nv[1] * 96);
@@ -1574,7 +1649,6 @@ int tam_dn_create(int32_t device, int32_t nx, int32_t ny, int32_t nz, int32_t ca
     e = hipMemcpy(n->p, h.data(), sizeof(float) * h.size(), hipMemcpyHostToDevice);
     if (e == hipSuccess) e = hipMemset(n->m1, 0, sizeof(float) * n->nparam);
     if (e == hipSuccess) e = hipMemset(n->m2, 0, sizeof(float) * n->nparam);
-    if (e == hipSuccess) e = hipMemset(n->x0, 0, 2ull * n->nv[0] * 16);
     if (e == hipSuccess) e = repack(n);
     if (e == hipSuccess) e = hipStreamSynchronize(n->stream);
     if (e != hipSuccess) {
@@ -1687,11 +1761,10 @@ int tam_dn_train(tam_dn* n, int32_t nslots, int32_t steps, double lr, uint64_t s
     for (int s = 0; s < steps && e == hipSuccess; ++s) {
         const int slot = (int)(rng() % (uint64_t)nslots);
         const float* tgt = n->ds_tgt + (long)slot * nv;
-        hipLaunchKernelGGL(pack_slot_kernel, dim3(grid_of(nv)), dim3(256), 0, n->stream,
-                           n->ds_feat + (long)slot * nv * 4, nv, n->x0);
-        e = forward(n, tgt);
+        const uint16_t* x0 = n->ds_feat + (long)slot * nv * 4;    // a slot holds the input's layout
+        e = forward(n, x0, tgt);
         if (e == hipSuccess) e = hipMemcpyAsync(dred + 2 * s, n->red, 16, hipMemcpyDeviceToDevice, n->stream);
-        if (e == hipSuccess) e = backward(n, tgt);
+        if (e == hipSuccess) e = backward(n, x0, tgt);
         if (e == hipSuccess) e = adam(n, (float)lr);
     }
     if (e == hipSuccess) e = hipEventRecord(n->ev1, n->stream);
@@ -1713,10 +1786,8 @@ int tam_dn_eval(tam_dn* n, int32_t slot, double* l1_pred, double* l1_input)
     DevScope ds(n->dev);
     const long nv = n->nv[0];
     const float* tgt = n->ds_tgt + (long)slot * nv;
-    hipLaunchKernelGGL(pack_slot_kernel, dim3(grid_of(nv)), dim3(256), 0, n->stream, n->ds_feat + (long)slot * nv * 4,
-                       nv, n->x0);
     DNCHK(n, hipEventRecord(n->ev0, n->stream));
-    DNCHK(n, forward(n, tgt));
+    DNCHK(n, forward(n, n->ds_feat + (long)slot * nv * 4, tgt));
     DNCHK(n, hipEventRecord(n->ev1, n->stream));
     double r[2];
     DNCHK(n, hipMemcpyAsync(r, n->red, 16, hipMemcpyDeviceToHost, n->stream));
@@ -1733,9 +1804,7 @@ int tam_dn_predict_slot(tam_dn* n, int32_t slot, float* pred, float* target, flo
     if (slot < 0 || slot >= n->capacity) return dfail(n, TAM_ERR_ARG, "slot out of range");
     DevScope ds(n->dev);
     const long nv = n->nv[0];
-    hipLaunchKernelGGL(pack_slot_kernel, dim3(grid_of(nv)), dim3(256), 0, n->stream, n->ds_feat + (long)slot * nv * 4,
-                       nv, n->x0);
-    DNCHK(n, forward(n, nullptr));
+    DNCHK(n, forward(n, n->ds_feat + (long)slot * nv * 4, nullptr));
     if (pred) DNCHK(n, hipMemcpyAsync(pred, n->out, sizeof(float) * nv, hipMemcpyDeviceToHost, n->stream));
     if (target)
         DNCHK(n, hipMemcpyAsync(target, n->ds_tgt + (long)slot * nv, sizeof(float) * nv, hipMemcpyDeviceToHost,
@@ -1764,7 +1833,7 @@ int tam_dn_forward_host(tam_dn* n, const float* features, float* out)
     DNCHK(n, hipMemcpyAsync(n->feat, features, sizeof(float) * 4 * nv, hipMemcpyHostToDevice, n->stream));
     hipLaunchKernelGGL(pack_input_kernel, dim3(grid_of(nv)), dim3(256), 0, n->stream, n->feat, nv, n->x0);
     DNCHK(n, hipEventRecord(n->ev0, n->stream));
-    DNCHK(n, forward(n, nullptr));
+    DNCHK(n, forward(n, n->x0, nullptr));
     DNCHK(n, hipEventRecord(n->ev1, n->stream));
     DNCHK(n, hipMemcpyAsync(out, n->out, sizeof(float) * nv, hipMemcpyDeviceToHost, n->stream));
     DNCHK(n, hipStreamSynchronize(n->stream));
@@ -1781,9 +1850,8 @@ int tam_dn_gradients_host(tam_dn* n, const float* features, const float* target,
     const int rc = tam_dn_store_host(n, 0, features, target);
     if (rc != TAM_OK) return rc;
     const float* tgt = n->ds_tgt;
-    hipLaunchKernelGGL(pack_slot_kernel, dim3(grid_of(nv)), dim3(256), 0, n->stream, n->ds_feat, nv, n->x0);
-    DNCHK(n, forward(n, tgt));
-    DNCHK(n, backward(n, tgt));
+    DNCHK(n, forward(n, n->ds_feat, tgt));
+    DNCHK(n, backward(n, n->ds_feat, tgt));
     double r[2];
     DNCHK(n, hipMemcpyAsync(r, n->red, 16, hipMemcpyDeviceToHost, n->stream));
     DNCHK(n, hipMemcpyAsync(grads, n->g, sizeof(float) * n->nparam, hipMemcpyDeviceToHost, n->stream));
@@ -1805,10 +1873,7 @@ int tam_dn_apply(tam_dn* n, tam_ctx* c, double npk)
     DNCHK(n, hipEventRecord(n->ev0, n->stream));
     hipLaunchKernelGGL(ctx_input_kernel, dim3(grid_of(nv)), dim3(256), 0, n->stream, c->tally, c->mut, c->mat,
                        c->mtab, nv, 1.0 / (npk * vcm), n->x0);
-    DNCHK(n, forward(n, nullptr));
-    hipLaunchKernelGGL(write_tally_kernel, dim3(grid_of(nv)), dim3(256), 0, n->stream, n->out, c->mut, nv, npk * vcm,
-                       c->tally);
-    DNCHK(n, hipGetLastError());
+    DNCHK(n, forward(n, n->x0, nullptr, c, npk * vcm));
     DNCHK(n, hipEventRecord(n->ev1, n->stream));
     DNCHK(n, hipStreamSynchronize(n->stream));
     n->last_ms = ms_between(n);
