@@ -221,7 +221,7 @@ __global__ __launch_bounds__(256) void conv_kernel(ConvArgs a)
         for (int n = 0; n < NT; ++n) store4(a, acc[t][n], mbase + t * 16 + (lane & 15), n * 16 + g * 4, NT * 16);
 }
 
-// Convolutions with at most 32 output channels, their input staged in LDS.
+// Convolutions with at most 48 output channels, their input staged in LDS.
 // In conv_kernel each A fragment of these layers feeds one or two MFMAs, so
 // the vector-memory path, not the matrix cores, sets the rate.  Here a block
 // computes an output brick of 16 (x) x 8 (y) x 4 (z) voxels.  For each group
@@ -1258,8 +1258,9 @@ hipError_t conv_launch(tam_dn* n, const uint16_t* x, int lvl, int cin, const uin
     hipLaunchKernelGGL((conv_kernel<CI, NT_, MT_>), dim3(MT_ == 8 ? b8 : b4), dim3(256), 0, n->stream, a)
     const int D = n->D[lvl], H = n->H[lvl], W = n->W[lvl];
     if (W % 16 == 0 && H % 8 == 0 && D % 4 == 0) {
-        // LDS-staged input for the layers with 16 or 32 output channels (48
-        // outputs as NT = 3 needs ~260 VGPRs there: the global form is faster)
+        // LDS-staged input for up to 48 output channels from 16 (at 128^3 107 us
+        // against 157 with the input read by each fragment); 64 outputs of the
+        // coarse levels are faster without (32^3: 49 us against 65)
         const dim3 grid((unsigned)((W / 16) * (H / 8) * (D / 4)));
 #define CL(CI, NT_) hipLaunchKernelGGL((conv_lds_kernel<CI, NT_, CONV_PLAIN>), grid, dim3(256), 0, n->stream, a, HeadArgs{})
         if (head || c4) {
@@ -1273,6 +1274,7 @@ hipError_t conv_launch(tam_dn* n, const uint16_t* x, int lvl, int cin, const uin
         switch (cin * 1000 + cout) {
         case 16016: CL(16, 1); return hipGetLastError();
         case 16032: CL(16, 2); return hipGetLastError();
+        case 16048: CL(16, 3); return hipGetLastError();
         case 32032: CL(32, 2); return hipGetLastError();
         case 96032: CL(96, 2); return hipGetLastError();
         case 48016: CL(48, 1); return hipGetLastError();
@@ -1293,7 +1295,6 @@ hipError_t conv_launch(tam_dn* n, const uint16_t* x, int lvl, int cin, const uin
     case 32016: CV(32, 1, 4); break;      // data gradient of layer 2
     case 64032: CV(64, 2, 4); break;      // data gradient of layer 4
     case 32096: CV(32, 6, 4); break;      // data gradient of layer 6
-    case 16048: CV(16, 3, 4); break;      // data gradient of layer 8
     default: return hipErrorInvalidValue;
     }
 #undef CV
