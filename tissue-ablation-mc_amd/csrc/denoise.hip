@@ -627,8 +627,9 @@ __global__ __launch_bounds__(256) void wgrad3_kernel(WgradArgs a)
 // (v_alignbyte), so one LDS read feeds 3 x COT MFMAs.  NDZ = 1: the block
 // covers all 27 taps; NDZ = 3: the 9 taps of one dz (blockIdx.y % 3).
 // blockIdx.y / NDZ is the input-channel tile.  At 128^3, 16 to 16 channels:
-// 121 us with the staging loads one after the other, 87 with all of them first;
-// 32 outputs 82, 62.  Blocks loop over bricks and
+// 121 us with the staging loads one after the other, 81 with all of them first
+// and one round of blocks; 32 outputs 82, 47.  The products alone take 53 and 27.
+// Blocks loop over bricks and
 // keep their sums in registers; at the end the four waves are summed in LDS
 // and each block writes its partial [taps][16][CO] to `part`, which
 // wgradb_reduce_kernel sums into gw.  The blocks of grid row 0 also sum dy
@@ -673,90 +674,102 @@ __global__ __launch_bounds__(256) void wgradb_kernel(WgradbArgs a)
 #pragma unroll
     for (int i = 0; i < COT; ++i) bsum[i] = 0.f;
 
-    for (long b = blockIdx.x; b < a.bricks; b += gridDim.x) {
+    // Staging.  x: voxel pairs (x0 + 2p, x0 + 2p + 1), p = 0 .. 7, of 10 rows x 6
+    // planes (4 where the block does one dz), 16 channels as two 8-channel
+    // halves; each lane loads both voxels' half and writes one dword (the pair)
+    // per channel; then the columns beside them, a voxel's half a thread.  dy:
+    // voxel pairs of 16 x 8 x 4 voxels, CO channels in 8-channel groups.  All
+    // loads of a brick go out before its first write (an item at a time, seven
+    // waits for memory came one after the other); outside the grid x reads the
+    // tensor's first voxel and counts as zeros.
+    constexpr int ROWS = NDZ == 1 ? 60 : 40, NI = (ROWS * 16 + 255) / 256, ND = CO / 8;
+    const int lz0 = NDZ == 1 ? 0 : dz0 + 1;                 // first plane of the x brick that is needed
+    const bool cat = a.x2 != nullptr, coarse = cat && ct * 16 < a.c1;
+    const uint16_t* xs = cat && !coarse ? a.x2 : a.x;
+    const int sh = coarse ? 1 : 0, sc = !cat ? (FIRST ? 4 : a.cin) : coarse ? a.c1 : a.cin - a.c1;
+    const int c0 = cat && !coarse ? ct * 16 - a.c1 : ct * 16;
+    const int half = threadIdx.x & 1, pp = ((int)threadIdx.x >> 1) & 7;
+    const int hr = (int)threadIdx.x >> 2, side = ((int)threadIdx.x >> 1) & 1;
+    const bool halo = threadIdx.x < ROWS * 4;
+    uint4 v0[NI], v1[NI], vh, d0[ND], d1[ND];
+    bool in[NI];
+    auto fetch = [&](long b) {
         const int x0 = (int)(b % bx) * 16, y0 = (int)((b / bx) % by) * 8, z0 = (int)(b / ((long)bx * by)) * 4;
-        __syncthreads();                                    // the last brick's reads are done
-        // x: voxel pairs (x0 + 2p, x0 + 2p + 1), p = 0 .. 7, of 10 rows x 6
-        // planes, 16 channels as two 8-channel halves; each lane loads both
-        // voxels' half and writes one dword (the pair) per channel.  All loads
-        // go out before the first write (an item at a time, five waits for
-        // memory came one after the other); outside the grid they read the
-        // tensor's first voxel and count as zeros.
-        {
-            const bool cat = a.x2 != nullptr, coarse = cat && ct * 16 < a.c1;
-            const uint16_t* src = cat && !coarse ? a.x2 : a.x;
-            const int sh = coarse ? 1 : 0, sc = !cat ? (FIRST ? 4 : a.cin) : coarse ? a.c1 : a.cin - a.c1;
-            const int c0 = cat && !coarse ? ct * 16 - a.c1 : ct * 16;
-            const int half = threadIdx.x & 1, pp = ((int)threadIdx.x >> 1) & 7;
-            uint4 v0[4], v1[4];
-            bool in[4];
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int row = min(((int)threadIdx.x >> 4) + 16 * i, 59);     // the last rows twice, alike
-                const int yy = y0 - 1 + row % 10, zz = z0 - 1 + row / 10;
-                in[i] = yy >= 0 && yy < H && zz >= 0 && zz < D;
-                const long vr = ((long)(zz >> sh) * (H >> sh) + (yy >> sh)) * (W >> sh);
-                const long at = in[i] ? (vr + ((x0 + 2 * pp) >> sh)) * sc : 0;
-                if constexpr (FIRST) {                       // 4 channels a voxel, the pair in 16 bytes
-                    v0[i] = *(const uint4*)(src + at);
-                } else {
-                    const uint16_t* q = src + at + c0 + half * 8;
-                    v0[i] = *(const uint4*)q;
-                    v1[i] = *(const uint4*)(q + (coarse ? 0 : sc));
-                }
-            }
-            // the columns beside them: a voxel's half a thread
-            const int hr = (int)threadIdx.x >> 2, side = ((int)threadIdx.x >> 1) & 1;
-            uint4 vh = make_uint4(0u, 0u, 0u, 0u);
-            if (threadIdx.x < 240) {
-                const int xx = side ? x0 + 16 : x0 - 1, yy = y0 - 1 + hr % 10, zz = z0 - 1 + hr / 10;
-                if (xx >= 0 && xx < W && yy >= 0 && yy < H && zz >= 0 && zz < D) {
-                    const uint16_t* q =
-                        src + (((long)(zz >> sh) * (H >> sh) + (yy >> sh)) * (W >> sh) + (xx >> sh)) * sc + c0;
-                    if constexpr (FIRST) {
-                        const uint2 u = half ? make_uint2(0u, 0u) : *(const uint2*)q;
-                        vh = make_uint4(u.x, u.y, 0u, 0u);
-                    } else {
-                        vh = *(const uint4*)(q + half * 8);
-                    }
-                }
-            }
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int row = min(((int)threadIdx.x >> 4) + 16 * i, 59);
-                if constexpr (FIRST) {
-                    v1[i] = make_uint4(v0[i].z, v0[i].w, 0u, 0u);
-                    v0[i] = make_uint4(v0[i].x, v0[i].y, 0u, 0u);
-                    in[i] = in[i] && half == 0;
-                }
-                if (!in[i]) v0[i] = v1[i] = make_uint4(0u, 0u, 0u, 0u);
-                const uint16_t* e0 = (const uint16_t*)&v0[i];
-                const uint16_t* e1 = (const uint16_t*)&v1[i];
-                uint16_t* dst = sX + (half * 8) * XC + row * XR + 4 + 2 * pp;
-#pragma unroll
-                for (int j = 0; j < 8; ++j) *(uint32_t*)(dst + j * XC) = (uint32_t)e0[j] | ((uint32_t)e1[j] << 16);
-            }
-            if (threadIdx.x < 240) {
-                const uint16_t* e = (const uint16_t*)&vh;
-                uint16_t* dst = sX + (half * 8) * XC + hr * XR + (side ? 20 : 3);
-#pragma unroll
-                for (int j = 0; j < 8; ++j) dst[j * XC] = e[j];
+        for (int i = 0; i < NI; ++i) {
+            const int row = min(((int)threadIdx.x >> 4) + 16 * i, ROWS - 1);   // the last rows twice, alike
+            const int yy = y0 - 1 + row % 10, zz = z0 - 1 + lz0 + row / 10;
+            in[i] = yy >= 0 && yy < H && zz >= 0 && zz < D;
+            const long vr = ((long)(zz >> sh) * (H >> sh) + (yy >> sh)) * (W >> sh);
+            const long at = in[i] ? (vr + ((x0 + 2 * pp) >> sh)) * sc : 0;
+            if constexpr (FIRST) {                           // 4 channels a voxel, the pair in 16 bytes
+                v0[i] = *(const uint4*)(xs + at);
+            } else {
+                const uint16_t* q = xs + at + c0 + half * 8;
+                v0[i] = *(const uint4*)q;
+                v1[i] = *(const uint4*)(q + (coarse ? 0 : sc));
             }
         }
-        // dy: voxel pairs of 16 x 8 x 4 voxels, CO channels in 8-channel groups
-        for (int q = threadIdx.x; q < 256 * (CO / 8); q += 256) {
-            const int vp = q / (CO / 8), c8 = (q % (CO / 8)) * 8;
-            const int vq = 2 * vp;
+#pragma unroll
+        for (int i = 0; i < ND; ++i) {
+            const int q = (int)threadIdx.x + 256 * i, vq = 2 * (q / ND), c8 = (q % ND) * 8;
             const int lx = vq & 15, ly = (vq >> 4) & 7, lz = vq >> 7;
             const uint16_t* src = a.dy + (((long)(z0 + lz) * H + (y0 + ly)) * W + (x0 + lx)) * a.cout + c8;
-            const uint4 v0 = *(const uint4*)src;
-            const uint4 v1 = *(const uint4*)(src + a.cout);
-            const uint16_t* e0 = (const uint16_t*)&v0;
-            const uint16_t* e1 = (const uint16_t*)&v1;
+            d0[i] = *(const uint4*)src;
+            d1[i] = *(const uint4*)(src + a.cout);
+        }
+        vh = make_uint4(0u, 0u, 0u, 0u);
+        if (halo) {
+            const int xx = side ? x0 + 16 : x0 - 1, yy = y0 - 1 + hr % 10, zz = z0 - 1 + lz0 + hr / 10;
+            if (xx >= 0 && xx < W && yy >= 0 && yy < H && zz >= 0 && zz < D) {
+                const uint16_t* q = xs + (((long)(zz >> sh) * (H >> sh) + (yy >> sh)) * (W >> sh) + (xx >> sh)) * sc + c0;
+                if constexpr (FIRST) {
+                    const uint2 u = half ? make_uint2(0u, 0u) : *(const uint2*)q;
+                    vh = make_uint4(u.x, u.y, 0u, 0u);
+                } else {
+                    vh = *(const uint4*)(q + half * 8);
+                }
+            }
+        }
+    };
+    auto commit = [&] {
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            const int row = min(((int)threadIdx.x >> 4) + 16 * i, ROWS - 1);
+            if constexpr (FIRST) {
+                v1[i] = make_uint4(v0[i].z, v0[i].w, 0u, 0u);
+                v0[i] = make_uint4(v0[i].x, v0[i].y, 0u, 0u);
+                in[i] = in[i] && half == 0;
+            }
+            if (!in[i]) v0[i] = v1[i] = make_uint4(0u, 0u, 0u, 0u);
+            const uint16_t* e0 = (const uint16_t*)&v0[i];
+            const uint16_t* e1 = (const uint16_t*)&v1[i];
+            uint16_t* dst = sX + (half * 8) * XC + (lz0 * 10 + row) * XR + 4 + 2 * pp;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) *(uint32_t*)(dst + j * XC) = (uint32_t)e0[j] | ((uint32_t)e1[j] << 16);
+        }
+#pragma unroll
+        for (int i = 0; i < ND; ++i) {
+            const int q = (int)threadIdx.x + 256 * i, vq = 2 * (q / ND), c8 = (q % ND) * 8;
+            const uint16_t* e0 = (const uint16_t*)&d0[i];
+            const uint16_t* e1 = (const uint16_t*)&d1[i];
             uint16_t* dst = sD + c8 * DC + vq;
 #pragma unroll
             for (int j = 0; j < 8; ++j) *(uint32_t*)(dst + j * DC) = (uint32_t)e0[j] | ((uint32_t)e1[j] << 16);
         }
+        if (halo) {
+            const uint16_t* e = (const uint16_t*)&vh;
+            uint16_t* dst = sX + (half * 8) * XC + (lz0 * 10 + hr) * XR + (side ? 20 : 3);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) dst[j * XC] = e[j];
+        }
+    };
+    // (The next brick's loads in flight during a brick's products gave nothing,
+    // 48 us against 47 for 32 outputs: two blocks a CU already overlap.)
+    for (long b = blockIdx.x; b < a.bricks; b += gridDim.x) {
+        fetch(b);
+        __syncthreads();                                    // the last brick's reads are done
+        commit();
         __syncthreads();
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
