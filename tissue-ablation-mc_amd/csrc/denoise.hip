@@ -83,16 +83,6 @@ __device__ __forceinline__ double tally_value(float v, float mut, double nv)
     return mut > 0.f ? fmax(expm1((double)v), 0.0) * nv : 0.0;
 }
 
-// 8 channels (c0 .. c0 + 7, c0 a multiple of 8) of fine voxel (xx, yy, zz):
-// from x, or with x2 from cat(upsample2(x), x2)
-__device__ __forceinline__ const uint16_t* cat_src(const uint16_t* x, const uint16_t* x2, int c1, int cin, int D,
-                                                   int H, int W, int xx, int yy, int zz, int c0)
-{
-    if (!x2) return x + (((long)zz * H + yy) * W + xx) * cin + c0;
-    if (c0 < c1) return x + (((long)(zz >> 1) * (H >> 1) + (yy >> 1)) * (W >> 1) + (xx >> 1)) * c1 + c0;
-    return x2 + (((long)zz * H + yy) * W + xx) * (cin - c1) + (c0 - c1);
-}
-
 // Raw buffer descriptor over `bytes` bytes from p (at most 2^31 - 1): loads
 // at offsets past it return zero.  0x00020000: gfx9 buffer word 3 (32-bit
 // data format, untyped access).
@@ -135,8 +125,9 @@ __device__ __forceinline__ void store4(const ConvArgs& a, const f32x4& acc, long
     *(uint2*)(a.y + m * cout + co) = out4(a, acc, m, co, cout);
 }
 
-// Forward convolution (and, with flipped weights, the data gradient).
-// A wave computes MT x 16 consecutive voxels of the flattened grid (each
+// Convolutions of the quarter grid, whose x edge need not be a multiple of 16,
+// and of 96 output channels: forward and, with flipped weights, data gradients.
+// A wave computes 16 MT consecutive voxels of the flattened grid (each
 // lane finds its voxel's x, y, z) for all NT x 16 output channels; CIN is
 // the input channel count.
 // Addressing: the input descriptor starts HW + W + 1 voxels before the
@@ -146,9 +137,10 @@ __device__ __forceinline__ void store4(const ConvArgs& a, const f32x4& acc, long
 // 27-bit mask of its voxel's valid taps.  With the k loop unrolled, a
 // k-block's tap and channel for each of the four lane groups are constants,
 // and their offsets scalar values.
-template <int CIN, int NT, int MT>
+template <int CIN, int NT>
 __global__ __launch_bounds__(256) void conv_kernel(ConvArgs a)
 {
+    constexpr int MT = 4;
     constexpr int KB = (27 * CIN + 31) / 32;
     constexpr unsigned OUT = 0x80000000u;          // past every descriptor's end
     const int lane = threadIdx.x & 63, g = lane >> 4;
@@ -1262,13 +1254,11 @@ hipError_t conv_launch(tam_dn* n, const uint16_t* x, int lvl, int cin, const uin
 {
     ConvArgs a{x, wp, bias, mask, y, n->D[lvl], n->H[lvl], n->W[lvl], cin, cout, kb, relu, x2, c1};
     const long nv = n->nv[lvl];
-    // 16 x MT-voxel wave tiles: 64 voxels, or 128 for the 48-channel input
-    // layer (its long k loop amortises the extra registers); every level's
-    // voxel count is a multiple of 512
+    // conv_kernel's blocks are 4 waves of 64 voxels; every level's voxel count is
+    // a multiple of 512
     if (nv % 512 != 0 || kb != (27 * cin + 31) / 32) return hipErrorInvalidValue;
-    const unsigned b8 = (unsigned)(nv / (4 * 16 * 8)), b4 = (unsigned)(nv / (4 * 16 * 4));
-#define CV(CI, NT_, MT_) \
-    hipLaunchKernelGGL((conv_kernel<CI, NT_, MT_>), dim3(MT_ == 8 ? b8 : b4), dim3(256), 0, n->stream, a)
+    const unsigned nb = (unsigned)(nv / (4 * 64));
+#define CV(CI, NT_) hipLaunchKernelGGL((conv_kernel<CI, NT_>), dim3(nb), dim3(256), 0, n->stream, a)
     const int D = n->D[lvl], H = n->H[lvl], W = n->W[lvl];
     if (W % 16 == 0 && H % 8 == 0 && D % 4 == 0) {
         // LDS-staged input for up to 48 output channels from 16 (at 128^3 107 us
@@ -1295,19 +1285,14 @@ hipError_t conv_launch(tam_dn* n, const uint16_t* x, int lvl, int cin, const uin
         }
 #undef CL
     }
-    // read or done by the LDS form only; the full grid's edges are multiples of 32
+    // read or done by the LDS form only, which every other layer takes: the full
+    // and the half grid's edges are multiples of 32 and 16
     if (x2 || c4 || head) return hipErrorInvalidValue;
     switch (cin * 1000 + cout) {
-    case 16016: CV(16, 1, 4); break;      // layers 0, 1, 9 and the data gradients of 0, 1, 9
-    case 16032: CV(16, 2, 4); break;      // layer 2
-    case 32032: CV(32, 2, 4); break;      // layers 3, 7 and their data gradients
-    case 32064: CV(32, 4, 4); break;      // layer 4
-    case 64064: CV(64, 4, 4); break;      // layer 5 and its data gradient
-    case 96032: CV(96, 2, 4); break;      // layer 6
-    case 48016: CV(48, 1, 8); break;      // layer 8
-    case 32016: CV(32, 1, 4); break;      // data gradient of layer 2
-    case 64032: CV(64, 2, 4); break;      // data gradient of layer 4
-    case 32096: CV(32, 6, 4); break;      // data gradient of layer 6
+    case 32064: CV(32, 4); break; // layer 4
+    case 64064: CV(64, 4); break; // layer 5 and its data gradient
+    case 64032: CV(64, 2); break; // data gradient of layer 4
+    case 32096: CV(32, 6); break; // data gradient of layer 6
     default: return hipErrorInvalidValue;
     }
 #undef CV
