@@ -1,0 +1,47 @@
+"""The LDS box of a transport run on the device: a run whose packets justify
+fewer blocks a CU than its launch shape names gets the larger box that those
+leave room for, and the tuner launches a shape's own blocks on its samples."""
+import numpy as np
+import pytest
+
+from tam_amd import configs, lib
+
+pytestmark = pytest.mark.gpu
+
+ONE, TWO, THREE = (42, 42, 46), (34, 34, 34), (28, 28, 34)          # boxes of one, two, three blocks a CU
+
+
+def _grid():
+    return configs.three_layer_skin(n=(64, 64, 64), ext=(0.5, 0.5, 0.25), packets=1, steps=1).grid()
+
+
+@pytest.mark.parametrize("shape,packets,box", [(8, 1_000_000, ONE), (6, 1_000_000, ONE), (4, 1_000_000, ONE),
+                                               (3, 1_000_000, THREE), (2, 1_000_000, TWO), (8, 8_388_608, TWO)])
+def test_box_of_the_blocks_that_run(shape, packets, box):
+    print("case", shape, packets, box, flush=True)
+    g = _grid()
+    g.set_mc_box(False)
+    g.set_mc_launch(shape, 32)
+    a = g.mc_run(packets, seed=11)
+    ta = g.download(lib.FIELD_TALLY)
+    g.set_mc_box(True, fp64=False)
+    b = g.mc_run(packets, seed=11)
+    tb = g.download(lib.FIELD_TALLY)
+    assert g.mc_box()[1] == box
+    assert b.box_adds > 0
+    for k in ("absorbed", "specular", "missed", "killed", "crossings", "interactions", "tally_adds"):
+        assert getattr(a, k) == getattr(b, k), k
+    assert list(a.escaped) == list(b.escaped)
+    # each deposit rounded to 2^-13 of dx + dy + dz, half a unit at most: relative to a voxel's deposits,
+    # of a few hundredths of that length on average, below 1e-3, and single ones by a few units
+    unit = (0.5 / 64 + 0.5 / 64 + 0.25 / 64) / 2 ** 13
+    np.testing.assert_allclose(tb, ta, rtol=1e-3, atol=16 * unit)
+    g.close()
+
+
+def test_the_tuner_launches_all_blocks_of_a_shape():
+    print("case: tuning on 1e6 packets; its last launch is 8 blocks a CU with the box", flush=True)
+    g = _grid()
+    g.tune_mc(1_000_000)
+    assert g.mc_box()[1] == TWO
+    g.close()

@@ -1,0 +1,71 @@
+"""The transport's launch plan (host arithmetic, CPU only): a run's blocks are
+chosen in waves per CU whatever the block size, and the LDS box is sized for
+the blocks that are launched."""
+import ctypes as C
+import random
+
+import pytest
+
+from tam_amd import lib
+
+NCU, LDS = 256, 160 * 1024
+FIELDS = ("box", "lanes", "per_cu", "blocks", "sd", "d", "ntab", "tab_off", "lds")
+
+
+def plan(npk, n=(200, 200, 200), shape=8, box=1, nmat=4, by_mat=1, full=0, ncu=NCU, lds_cu=LDS, lds_blk=LDS):
+    i64 = C.c_int64
+    out = (i64 * len(FIELDS))()
+    lib.load().tam_internal_mc_plan((i64 * 12)(npk, *n, shape, box, nmat, by_mat, full, ncu, lds_cu, lds_blk), out)
+    return dict(zip(FIELDS, out))
+
+
+def waves(p):
+    """Waves a CU, over the whole device."""
+    return p["blocks"] * (p["lanes"] // 64) / NCU
+
+
+@pytest.mark.parametrize("shape", [1, 2, 3, 4, 5, 6, 7, 8, 12, 16, 64])
+@pytest.mark.parametrize("packets", [130_000, 300_000, 1_000_000, 3_000_000, 6_300_000, 8_400_000, 20_000_000, 10 ** 8])
+def test_short_box_runs_keep_sixteen_waves_a_cu(shape, packets):
+    p = plan(packets, shape=shape)
+    few = packets < 64 * NCU * shape
+    assert p["box"] == (0 if few else 1)
+    if few:
+        return
+    assert waves(p) >= min(16, 4 * shape)                       # the shape's own where it is smaller
+    assert waves(p) <= 4 * shape
+    if packets >= 4096 * NCU * shape:                           # 1024 packets for each wave of the shape
+        assert waves(p) == 4 * shape
+    assert waves(p) <= max(16, packets / (1024 * NCU))
+    # the box is sized for the blocks that run
+    assert p["blocks"] == NCU * p["per_cu"]
+    share = LDS // p["per_cu"] - 1024
+    assert p["sd"] == int((share // 2) ** (1 / 3)) & ~1
+    assert 2 * p["sd"] ** 2 * (p["d"] + 1) > share >= 2 * p["sd"] ** 2 * p["d"]
+
+
+@pytest.mark.parametrize("shape", [1, 2, 3, 4, 6, 8])
+def test_tuner_samples_run_the_whole_shape(shape):
+    long_run = plan(10 ** 8, shape=shape)
+    for packets in (2_000_000, 5_000_000):
+        assert plan(packets, shape=shape, full=1) == long_run
+
+
+def test_box_leaves_the_lds_that_its_blocks_need():
+    rng = random.Random(5)
+    for _ in range(4000):
+        q = dict(npk=int(10 ** rng.uniform(0, 9)), n=tuple(rng.randint(1, 300) for _ in range(3)),
+                 shape=rng.randint(1, 64), box=rng.randint(0, 2), nmat=rng.randint(2, 256), by_mat=rng.randint(0, 1),
+                 full=rng.randint(0, 1))
+        p = plan(**q)
+        assert p["blocks"] >= 1 and p["lanes"] in (256, 1024), q
+        if not p["box"]:
+            assert p["lds"] == 32 * p["ntab"] <= 32 * 64 and waves(p) <= 4 * q["shape"], q
+            continue
+        esz = 2 if q["box"] == 1 else 8
+        bytes_ = esz * p["sd"] ** 2 * p["d"]
+        assert p["sd"] <= min(q["n"][:2]) and p["d"] <= q["n"][2], q
+        assert bytes_ <= LDS // p["per_cu"] - 1024, q
+        assert p["ntab"] in (0, q["nmat"]) and (q["by_mat"] or not p["ntab"]), q
+        if p["ntab"]:
+            assert p["tab_off"] % 16 == 0 and p["tab_off"] >= bytes_ and p["lds"] == p["tab_off"] + 32 * p["ntab"], q

@@ -123,6 +123,7 @@ McArgs mc_args(tam_ctx* c, int64_t npackets, uint64_t seed, uint32_t stream)
     a.p0 = 0; a.npk = (uint64_t)npackets;
     a.key0 = (uint32_t)seed; a.key1 = (uint32_t)(seed >> 32); a.stream = stream;
     a.blocks_per_cu = c->mc_bpc;
+    a.full_grid = c->mc_full ? 1 : 0;
     a.rng_batch = c->mc_batch;
     a.box_enable = c->mc_box;
     a.box_psum = c->box_psum;              // the box follows the last run's path
@@ -1346,6 +1347,12 @@ int tam_tune_mc(tam_ctx* c, int64_t sample, int32_t* blocks_per_cu, int32_t* rng
         double rate;
     };
     std::vector<Cand> rates;
+    // a sample stands for a longer run: candidates launch all of their blocks
+    struct FullGrid {
+        tam_ctx* c;
+        explicit FullGrid(tam_ctx* q) : c(q) { c->mc_full = true; }
+        ~FullGrid() { c->mc_full = false; }
+    } full(c);
     for (int x = 0; x < 2; ++x)
         for (int b : bpcs) {
             for (int t : batches) {

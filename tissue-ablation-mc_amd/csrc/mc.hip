@@ -778,27 +778,34 @@ hipError_t launch_atomic_rate(double* t, long slots, long count, hipStream_t s)
     return hipGetLastError();
 }
 
+// The current device's CUs, and LDS per CU and per block (160 KiB each on MI355X)
+McDevice mc_device()
+{
+    int dev = 0;
+    McDevice d{0, 0, 0};
+    hipError_t e = hipGetDevice(&dev);
+    if (e == hipSuccess) e = hipDeviceGetAttribute(&d.ncu, hipDeviceAttributeMultiprocessorCount, dev);
+    if (e != hipSuccess || d.ncu <= 0) d.ncu = 256;
+    if (hipDeviceGetAttribute(&d.lds_cu, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, dev) != hipSuccess ||
+        d.lds_cu <= 0)
+        d.lds_cu = 64 * 1024;
+    if (hipDeviceGetAttribute(&d.lds_blk, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess ||
+        d.lds_blk <= 0)
+        d.lds_blk = 64 * 1024;
+    return d;
+}
+
 hipError_t launch_mc_batch(const McArgs* dtab, int n, long total_npk, int blocks_per_cu, hipStream_t s)
 {
     if (n <= 0 || total_npk <= 0) return hipSuccess;
-    int dev = 0, ncu = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e == hipSuccess) e = hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
-    if (e != hipSuccess || ncu <= 0) ncu = 256;
+    const McDevice dev = mc_device();
     const int bpc = blocks_per_cu > 0 ? blocks_per_cu : 8;
-    long blocks = (long)ncu * bpc;
+    long blocks = (long)dev.ncu * bpc;
     const long need = (total_npk + 255) / 256;
     if (need < blocks) blocks = need;
     // per-wave LDS tally boxes: the block's share of the CU's LDS (1 KiB kept
     // for the kernel's own use), split over its 4 waves
-    int lds_cu = 0, lds_blk = 0;
-    if (hipDeviceGetAttribute(&lds_cu, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, dev) != hipSuccess ||
-        lds_cu <= 0)
-        lds_cu = 64 * 1024;
-    if (hipDeviceGetAttribute(&lds_blk, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess ||
-        lds_blk <= 0)
-        lds_blk = 64 * 1024;
-    const long per_block = std::min((long)lds_blk - kLdsOwn, (long)lds_cu / bpc - kLdsOwn);
+    const long per_block = std::min((long)dev.lds_blk - kLdsOwn, (long)dev.lds_cu / bpc - kLdsOwn);
     // 16-bit slots, a multiple of 8 per wave
     const int wbox = per_block > 0 ? (int)(per_block / 4 / 2) & ~7 : 0;
     const size_t lds = sizeof(uint16_t) * 4 * (size_t)wbox;
@@ -832,61 +839,120 @@ hipError_t mc_prepare(int dev)
     return hipFuncSetAttribute((const void*)mc_batch_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds_blk);
 }
 
+// The launch of a transport run: its blocks first, then the LDS box and table
+// that so many blocks a CU leave room for.
+McPlan mc_plan(const McArgs& a, const McDevice& dev)
+{
+    McPlan p{};
+    // blocks_per_cu 256-lane blocks per CU (autotuned): the most waves of a run
+    const int shape = a.blocks_per_cu > 0 ? a.blocks_per_cu : 8;
+    // A launch with fewer packets than a quarter of the shape's lanes (the reference's
+    // own run: 125 000 packets per cycle of a few deposits each) goes without
+    // the box: clearing and flushing the box would cost more than it saves.
+    const bool few = (double)a.npk < 64.0 * (double)dev.ncu * shape;
+    if (a.box_enable && !few) {
+        // A block's box costs a clearing and a device add per touched voxel,
+        // and waves that share a SIMD slow each other's longest packets: 16
+        // waves a CU (all of a smaller shape's), further ones where each has
+        // 1024 packets (8 blocks of 256 lanes a CU at 100^3: 3e6 packets 12.7
+        // ms on 256 blocks of 1024 lanes, 13.9 on 512; 1e7 39.3 on both).  In
+        // waves, so that 256-lane blocks fill a CU too: 1e6 packets at 100^3,
+        // shapes 2, 3, 6, 8: 5.0, 5.7, 4.6, 4.6 ms; with one block a CU of
+        // whatever size, its box that of the shape, 6.7, 6.8, 6.7, 5.3.
+        int bpc = shape;
+        const int64_t justified = (int64_t)(a.npk / ((uint64_t)dev.ncu * 4096u));
+        if (!a.full_grid && justified < shape) bpc = std::min(shape, std::max(4, (int)justified & ~3));
+        // a multiple of 4 runs as bpc / 4 blocks of 1024 lanes: the same waves
+        // per CU, one box per 16 waves
+        const bool wide = bpc % 4 == 0;
+        p.lanes = wide ? 1024 : 256;
+        p.per_cu = wide ? bpc / 4 : bpc;
+        p.blocks = (int64_t)dev.ncu * p.per_cu;
+        // LDS tally box: the blocks of a CU share its LDS (160 KiB on
+        // MI355X, also the most one block may take), 1 KiB per block kept for
+        // the kernel's own use: with 16-bit sums 42^2 x 46 voxels at 1 block per CU
+        // (1 or 4 blocks_per_cu), 34^2 x 34 at 2 (2 or 8), 28^2 x 34 at 3; with
+        // FP64 27^3, 21^3, 18^2 x 20.  The cube sits on the beam axis (its x edge
+        // even with 16-bit sums, so the two voxels of a word share a row).  Its z range is where
+        // the last run's path was largest, or the top face (where most of the
+        // path of a surface beam lies) before any run.  On the c1 skin cycles a
+        // cube caught more deposits past the first cycle than flatter (d ~ s/2,
+        // s/8) or taller (d ~ 2s) boxes of the same volume, and than a per-launch
+        // choice among depths of 2-32 planes made from the last run's path.
+        // The box holds 16-bit fixed-point sums (box_enable 1: four times the
+        // voxels of FP64) or FP64 ones (box_enable 2).  Fixed-point unit: 2^-13 of
+        // dx + dy + dz, so a deposit is rounded by at most ~1e-4 of a voxel-sized
+        // path, and a slot wraps (one carry) every ~40 typical deposits.
+        const bool fx = a.box_enable == 1;
+        const long esz = fx ? 2 : 8;
+        const long vox = std::min((long)dev.lds_blk - kLdsOwn, (long)dev.lds_cu / p.per_cu - kLdsOwn) / esz;
+        p.sd = std::min((int)std::cbrt((double)vox), std::min(a.nx, a.ny));
+        if (fx && p.sd > 1) p.sd &= ~1;
+        p.d = p.sd > 0 ? (int)std::min<long>(a.nz, vox / ((long)p.sd * p.sd)) : 0;
+        p.box = p.sd >= 4 && p.d >= 1;
+        if (p.box) {
+            const int64_t lds = (int64_t)esz * p.sd * p.sd * p.d;
+            // the material table goes behind the box where that keeps the resident
+            // blocks: LDS is given out in steps of lds_cu / 128
+            p.tab_off = (int)((lds + 15) & ~(int64_t)15);
+            const int64_t tab_lds = p.tab_off + (int64_t)sizeof(MatEntry) * a.nmat;
+            const int64_t own = sizeof(unsigned long long) * TAM_CNT_N, step = dev.lds_cu / 128;
+            const bool tab = a.mut_by_mat && tab_lds + own <= lds + kLdsOwn &&
+                             (tab_lds + own + step - 1) / step * step * p.per_cu <= dev.lds_cu;
+            p.ntab = tab ? a.nmat : 0;
+            p.lds = tab ? tab_lds : lds;
+            return p;
+        }
+    }
+    // A short run takes as long as its longest packet's chain of events,
+    // and a wave's pass costs the same for 4 lanes as for 64: up to 8
+    // waves a CU (2 per SIMD) share fewer than 64 packets each, down to
+    // 4; past that every wave starts with a full set of lanes.  20 000
+    // packets at 64^3: 1.35 ms, against 2.7 ms on full waves alone
+    // (1.6 at 4 waves a CU, 1.35 at 16); 125 000 packets of a pure
+    // absorber: 40 us, against 68 (44 at 16 waves a CU).
+    p = McPlan{};
+    p.lanes = 256;
+    p.per_cu = shape;
+    const int64_t waves = std::max((int64_t)((a.npk + 63) / 64),
+                                   std::min((int64_t)8 * dev.ncu, (int64_t)((a.npk + 3) / 4)));
+    p.blocks = std::min((int64_t)dev.ncu * shape, (waves + 3) / 4);
+    p.ntab = a.mut_by_mat && a.nmat <= kTabMax ? a.nmat : 0;
+    p.lds = (int64_t)sizeof(MatEntry) * p.ntab;
+    return p;
+}
+
+extern "C" void tam_internal_mc_plan(const int64_t* in, int64_t* out)
+{
+    McArgs a{};
+    a.npk = (uint64_t)in[0];
+    a.nx = (int)in[1]; a.ny = (int)in[2]; a.nz = (int)in[3];
+    a.blocks_per_cu = (int)in[4]; a.box_enable = (int)in[5];
+    a.nmat = (int)in[6]; a.mut_by_mat = (int)in[7]; a.full_grid = (int)in[8];
+    const McPlan p = mc_plan(a, McDevice{(int)in[9], (int)in[10], (int)in[11]});
+    const int64_t r[] = {p.box, p.lanes, p.per_cu, p.blocks, p.sd, p.d, p.ntab, p.tab_off, p.lds};
+    std::copy(std::begin(r), std::end(r), out);
+}
+
 hipError_t launch_mc(const McArgs& a, hipStream_t s)
 {
     const long nvox = (long)a.nx * a.ny * a.nz;
     // the run's counters, and the tally unless the run adds to it
     auto clear = [&] { return launch_clear(a.tally, a.clear_tally ? nvox : 0, a.counters, TAM_CNT_SLOTS, s); };
     if (a.npk == 0) return clear();
-    int dev = 0, ncu = 0, lds_cu = 0, lds_blk = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e == hipSuccess) e = hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev);
-    if (e != hipSuccess || ncu <= 0) ncu = 256;
-    // LDS per CU and per block (160 KiB each on MI355X)
-    if (hipDeviceGetAttribute(&lds_cu, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, dev) != hipSuccess ||
-        lds_cu <= 0)
-        lds_cu = 64 * 1024;
-    if (hipDeviceGetAttribute(&lds_blk, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) != hipSuccess ||
-        lds_blk <= 0)
-        lds_blk = 64 * 1024;
-    // blocks_per_cu 256-lane blocks per CU (autotuned) set the LDS box and the
-    // most blocks; runs of fewer packets launch fewer (below)
-    const int bpc = a.blocks_per_cu > 0 ? a.blocks_per_cu : 8;
-    // with the box on, a multiple of 4 runs as bpc / 4 blocks of 1024 lanes:
-    // the same waves per CU, one box per 16 waves
-    const bool wide = a.box_enable && bpc % 4 == 0;
-    const int lanes = wide ? 1024 : 256, bpc_l = wide ? bpc / 4 : bpc;
-    // LDS tally box: the resident blocks of a CU share its LDS (160 KiB on
-    // MI355X, also the most one block may take), 1 KiB per block kept for
-    // the kernel's own use: with 16-bit sums 42^2 x 46 voxels at 1 block per CU
-    // (1 or 4 blocks_per_cu), 34^2 x 34 at 2 (2 or 8), 28^2 x 34 at 3; with
-    // FP64 27^3, 21^3, 18^2 x 20.  The cube sits on the beam axis (its x edge
-    // even with 16-bit sums, so the two voxels of a word share a row).  Its z range is where
-    // the last run's path was largest, or the top face (where most of the
-    // path of a surface beam lies) before any run.  On the c1 skin cycles a
-    // cube caught more deposits past the first cycle than flatter (d ~ s/2,
-    // s/8) or taller (d ~ 2s) boxes of the same volume, and than a per-launch
-    // choice among depths of 2-32 planes made from the last run's path.
-    // The box holds 16-bit fixed-point sums (box_enable 1: four times the
-    // voxels of FP64) or FP64 ones (box_enable 2).  Fixed-point unit: 2^-13 of
-    // dx + dy + dz, so a deposit is rounded by at most ~1e-4 of a voxel-sized
-    // path, and a slot wraps (one carry) every ~40 typical deposits.
-    const bool fx = a.box_enable == 1;
-    const long esz = fx ? 2 : 8;
+    const McPlan p = mc_plan(a, mc_device());
     McArgs b = a;
     mc_box_units(b);
     b.box_n[0] = b.box_n[1] = b.box_n[2] = 0;
     b.box_geom = nullptr;
-    const long vox = std::min((long)lds_blk - kLdsOwn, (long)lds_cu / bpc_l - kLdsOwn) / esz;
-    BoxPlace bp{};
-    bp.sd = std::min((int)std::cbrt((double)vox), std::min(a.nx, a.ny));
-    if (fx && bp.sd > 1) bp.sd &= ~1;
-    bp.d = bp.sd > 0 ? (int)std::min<long>(a.nz, vox / ((long)bp.sd * bp.sd)) : 0;
-    // A launch with fewer packets than a quarter of the lanes (the reference's
-    // own run: 125 000 packets per cycle of a few deposits each) goes without
-    // the box: clearing and flushing the box would cost more than it saves.
-    const bool few = (double)a.npk < 0.25 * (double)ncu * bpc_l * lanes;
-    if (a.box_enable && !few && bp.sd >= 4 && bp.d >= 1) {
+    b.ntab = p.ntab;
+    b.tab_off = p.tab_off;
+    const dim3 grid((unsigned)p.blocks), block((unsigned)p.lanes);
+    const size_t lds = (size_t)p.lds;
+    if (p.box) {
+        BoxPlace bp{};
+        bp.sd = p.sd;
+        bp.d = p.d;
         bp.ox = std::max(0, std::min((int)std::lround(a.cx / a.dx) - bp.sd / 2, a.nx - bp.sd));
         bp.oy = std::max(0, std::min((int)std::lround(a.cy / a.dy) - bp.sd / 2, a.ny - bp.sd));
         b.box_o[0] = bp.ox;
@@ -894,18 +960,6 @@ hipError_t launch_mc(const McArgs& a, hipStream_t s)
         b.box_o[2] = a.nz - bp.d;
         b.box_n[0] = b.box_n[1] = bp.sd;
         b.box_n[2] = bp.d;
-        // A block's box costs a clearing and a device add per touched voxel,
-        // and waves that share a SIMD slow each other's longest packets: a
-        // block per CU from 16 packets a wave on, the further blocks of the
-        // launch shape from 1024 a wave on (100^3 cube, 8 blocks of 256 lanes a
-        // CU: 3e6 packets 12.7 ms on 256 blocks of 1024 lanes, 13.9 on 512;
-        // 1e7 39.3 on both.  Down to 16 a wave instead of 256: 140 000 packets
-        // 2.4 against 3.9 ms, 400 000 3.3 against 3.9, 1e6 5.4 on both).
-        const long wpb = lanes / 64;
-        long blocks = std::max((long)(a.npk / (uint64_t)(wpb * 1024)),
-                               std::min((long)ncu, (long)(a.npk / (uint64_t)(wpb * 16))));
-        blocks = std::max(1L, std::min(blocks, (long)ncu * bpc_l));
-        const size_t lds = (size_t)esz * (size_t)bp.sd * (size_t)bp.sd * (size_t)bp.d;
         if (a.box_psum && a.box_geom) {
             hipLaunchKernelGGL(box_plane_kernel, dim3((unsigned)a.nz), dim3(256), 0, s, a.tally, a.mut, a.nx, a.ny,
                                bp, a.box_psum);
@@ -914,22 +968,13 @@ hipError_t launch_mc(const McArgs& a, hipStream_t s)
         }
         const hipError_t ef = clear();
         if (ef != hipSuccess) return ef;
-        // the material table goes behind the box where that keeps the resident
-        // blocks: LDS is given out in steps of lds_cu / 128
-        const size_t tab_off = (lds + 15) & ~(size_t)15, tab_lds = tab_off + sizeof(MatEntry) * (size_t)a.nmat;
-        const size_t step = (size_t)lds_cu / 128;
-        const bool tab = a.mut_by_mat && tab_lds + sizeof(unsigned long long) * TAM_CNT_N <= lds + (size_t)kLdsOwn &&
-                         (tab_lds + sizeof(unsigned long long) * TAM_CNT_N + step - 1) / step * step * (size_t)bpc_l <=
-                             (size_t)lds_cu;
-        b.ntab = tab ? a.nmat : 0;
-        b.tab_off = (int)tab_off;
-#define TAM_BOX(NT_, BT_)                                                                                          \
-    do {                                                                                                           \
-        if (tab)                                                                                                   \
-            hipLaunchKernelGGL((mc_box_kernel<NT_, BT_, true>), dim3((unsigned)blocks), dim3(NT_), tab_lds, s, b); \
-        else hipLaunchKernelGGL((mc_box_kernel<NT_, BT_, false>), dim3((unsigned)blocks), dim3(NT_), lds, s, b);   \
+#define TAM_BOX(NT_, BT_)                                                                       \
+    do {                                                                                        \
+        if (p.ntab) hipLaunchKernelGGL((mc_box_kernel<NT_, BT_, true>), grid, block, lds, s, b); \
+        else hipLaunchKernelGGL((mc_box_kernel<NT_, BT_, false>), grid, block, lds, s, b);       \
     } while (0)
-        if (fx) {
+        const bool wide = p.lanes == 1024;
+        if (a.box_enable == 1) {
             if (wide) TAM_BOX(1024, uint16_t);
             else TAM_BOX(256, uint16_t);
         } else {
@@ -940,21 +985,8 @@ hipError_t launch_mc(const McArgs& a, hipStream_t s)
     } else {
         const hipError_t ef = clear();
         if (ef != hipSuccess) return ef;
-        // A short run takes as long as its longest packet's chain of events,
-        // and a wave's pass costs the same for 4 lanes as for 64: up to 8
-        // waves a CU (2 per SIMD) share fewer than 64 packets each, down to
-        // 4; past that every wave starts with a full set of lanes.  20 000
-        // packets at 64^3: 1.35 ms, against 2.7 ms on full waves alone
-        // (1.6 at 4 waves a CU, 1.35 at 16); 125 000 packets of a pure
-        // absorber: 40 us, against 68 (44 at 16 waves a CU).
-        const long waves = std::max((long)((a.npk + 63) / 64), std::min(8L * ncu, (long)((a.npk + 3) / 4)));
-        const long blocks = std::min((long)ncu * bpc, (waves + 3) / 4);
-        const bool tab = a.mut_by_mat && a.nmat <= kTabMax;
-        b.ntab = tab ? a.nmat : 0;
-        if (tab)
-            hipLaunchKernelGGL((mc_kernel<true>), dim3((unsigned)blocks), dim3(256), sizeof(MatEntry) * (size_t)a.nmat,
-                               s, b);
-        else hipLaunchKernelGGL((mc_kernel<false>), dim3((unsigned)blocks), dim3(256), 0, s, b);
+        if (p.ntab) hipLaunchKernelGGL((mc_kernel<true>), grid, block, lds, s, b);
+        else hipLaunchKernelGGL((mc_kernel<false>), grid, block, lds, s, b);
     }
     return hipGetLastError();
 }

@@ -124,6 +124,7 @@ struct McArgs {
     uint64_t p0, npk;
     uint32_t key0, key1, stream;
     int blocks_per_cu;         // 256-lane blocks per CU (lanes = packets in flight)
+    int full_grid;             // all of them whatever npk (the tuner, whose samples stand for longer runs)
     int rng_batch;             // pending lanes of a wave that start its random phase
     // graph replays: packet count and Philox stream read from device memory
     // at launch (nullptr: npk and stream above)
@@ -299,6 +300,7 @@ struct tam_ctx {
     long neblk;                 // slots: enough for the largest launch grid
     int mc_bpc;                 // transport launch: blocks per CU (autotuned)
     int mc_batch;               // transport launch: random-phase batch (autotuned)
+    bool mc_full;               // transport launch: all blocks of the shape whatever the packets (while tuning)
     int mc_box;                 // transport launch: LDS tally box off / 16-bit fixed point / FP64 (0 / 1 / 2; on-off autotuned)
     float2* robin;
     double *kappa, *density, *heatcap, *coeff, *rhokap;
@@ -349,6 +351,20 @@ struct CycleHdr {
 static_assert(sizeof(CycleHdr) == 64, "cycle header layout");
 
 // ---- launchers (each enqueues on `s`, returns hipError_t) --------------
+struct McDevice { int ncu, lds_cu, lds_blk; };
+McDevice mc_device();
+struct McPlan {
+    int box;                   // with the LDS tally box (sd x sd x d voxels)
+    int lanes, per_cu;         // of a block; blocks per CU
+    int64_t blocks;
+    int sd, d;
+    int ntab, tab_off;         // material table in LDS
+    int64_t lds;               // dynamic LDS of a block, bytes
+};
+McPlan mc_plan(const McArgs& a, const McDevice& dev);
+// the plan of (npk, nx, ny, nz, blocks_per_cu, box_enable, nmat, mut_by_mat, full_grid, ncu, lds_cu, lds_blk)
+// as (box, lanes, per_cu, blocks, sd, d, ntab, tab_off, lds); host only
+extern "C" void tam_internal_mc_plan(const int64_t* in, int64_t* out);
 hipError_t launch_mc(const McArgs& a, hipStream_t s);
 // once per context, before any capture: lets the LDS-box kernel take the
 // device's whole per-block LDS
