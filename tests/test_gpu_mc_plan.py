@@ -45,3 +45,28 @@ def test_the_tuner_launches_all_blocks_of_a_shape():
     g.tune_mc(1_000_000)
     assert g.mc_box()[1] == TWO
     g.close()
+
+
+# the table behind the largest box: 15 materials and air are 16 entries, the
+# most that fit below the box's own 1 KiB; 28 entries the most that fit at all
+@pytest.mark.parametrize("materials", [15, 16, 27, 28, 63, 64])
+def test_material_tables_at_the_lds_limit(materials):
+    print("case: materials", materials, flush=True)
+    prob = configs.three_layer_skin(n=(64, 64, 64), ext=(0.5, 0.5, 0.25), packets=1, steps=1)
+    prob.table = [(2.0 + 0.1 * m, 150.0 + m, 0.8, 1.4) for m in range(materials)]
+    prob.mat = (np.arange(prob.mat.size) % materials).astype(np.uint8).reshape(prob.mat.shape)
+    a, b = prob.grid(), prob.grid()
+    b.upload(lib.FIELD_RHOKAP, b.download(lib.FIELD_RHOKAP))          # mu_t from the array
+    for shape, box in ((4, True), (1, True), (4, False)):
+        for g in (a, b):
+            g.set_mc_launch(shape, 32)
+            g.set_mc_box(box)
+        sa, sb = (g.mc_run(300_000, seed=4) for g in (a, b))
+        assert not box or a.mc_box()[1] == ONE
+        for k in ("absorbed", "specular", "missed", "killed", "crossings", "interactions", "tally_adds", "box_adds"):
+            assert getattr(sa, k) == getattr(sb, k), k
+        assert list(sa.escaped) == list(sb.escaped)
+        ta, tb = (g.download(lib.FIELD_TALLY) for g in (a, b))
+        np.testing.assert_allclose(ta, tb, rtol=1e-9, atol=1e-9 * tb.max())
+    a.close()
+    b.close()

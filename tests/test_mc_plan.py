@@ -9,7 +9,7 @@ import pytest
 from tam_amd import lib
 
 NCU, LDS = 256, 160 * 1024
-FIELDS = ("box", "lanes", "per_cu", "blocks", "sd", "d", "ntab", "tab_off", "lds")
+FIELDS = ("box", "lanes", "per_cu", "blocks", "sd", "d", "ntab", "tab_off", "lds", "limit")
 
 
 def plan(npk, n=(200, 200, 200), shape=8, box=1, nmat=4, by_mat=1, full=0, ncu=NCU, lds_cu=LDS, lds_blk=LDS):
@@ -69,3 +69,25 @@ def test_box_leaves_the_lds_that_its_blocks_need():
         assert p["ntab"] in (0, q["nmat"]) and (q["by_mat"] or not p["ntab"]), q
         if p["ntab"]:
             assert p["tab_off"] % 16 == 0 and p["tab_off"] >= bytes_ and p["lds"] == p["tab_off"] + 32 * p["ntab"], q
+
+
+COUNTS = 14 * 8                                                 # a block's static LDS: its counts
+
+
+@pytest.mark.parametrize("entries", [2, 16, 17, 28, 29, 64, 256])
+def test_box_and_table_fit_what_the_kernel_is_allowed(entries):
+    p = plan(10 ** 7, n=(64, 64, 64), shape=4, nmat=entries)
+    assert (p["sd"], p["sd"], p["d"]) == (42, 42, 46) and p["ntab"] == (entries if entries <= 28 else 0)
+    assert p["lds"] <= p["limit"] == LDS - COUNTS
+
+
+def test_no_plan_asks_for_more_lds_than_is_allowed():
+    rng = random.Random(9)
+    for _ in range(4000):
+        q = dict(npk=10 ** 9, n=tuple(rng.randint(4, 300) for _ in range(3)), shape=rng.choice([1, 2, 3, 4, 5, 8, 12]),
+                 box=rng.randint(1, 2), nmat=rng.randint(2, 64))
+        p = plan(**q)
+        assert p["lds"] <= p["limit"], q
+        if p["ntab"]:                                           # and every block a CU finds its place
+            step = LDS // 128
+            assert -(-(p["lds"] + COUNTS) // step) * step * p["per_cu"] <= LDS, q

@@ -115,8 +115,11 @@ constexpr uint32_t kMaxEvents = 1u << 24;   // walk steps + random events of one
 constexpr int kBoxUnitBits = 13;            // fixed-point box unit: 2^-13 of dx + dy + dz
 
 constexpr long kLdsOwn = 1024;              // LDS per block kept for the kernel's own use (counts, material table)
+constexpr long kCountLds = sizeof(unsigned long long) * TAM_CNT_N;     // a block's counts, static
 constexpr int kTabMax = 64;                 // materials in the LDS of a kernel without the box
 constexpr int kBatchTab = 4;                // materials per wave in a batched block's own LDS
+constexpr long kBatchLds = 4 * (kCountLds + kBatchTab * (long)sizeof(MatEntry));   // a batched block's static LDS
+static_assert(kCountLds <= kLdsOwn && kBatchLds <= kLdsOwn, "the boxes leave kLdsOwn bytes of a block's LDS");
 
 // The LDS tally box of a launch: voxels [o, o + n).
 struct BoxGeom {
@@ -696,6 +699,7 @@ __global__ __launch_bounds__(256) void mc_batch_kernel(const McArgs* __restrict_
     // per wave: counts of the current instance and its material table
     __shared__ unsigned long long wsums[4][TAM_CNT_N];
     __shared__ __attribute__((aligned(16))) MatEntry wtab[4][kBatchTab];
+    static_assert(sizeof(wsums) + sizeof(wtab) == kBatchLds, "static LDS of a batched block");
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
     unsigned long long* sums = wsums[threadIdx.x >> 6];
@@ -819,24 +823,28 @@ void mc_box_units(McArgs& a)
     a.box_quantum = 1.0 / (double)a.box_scale;
 }
 
+// the most dynamic LDS that a box launch may ask for
+long mc_lds_limit(long lds_blk) { return lds_blk - kCountLds; }
+
 hipError_t mc_prepare(int dev)
 {
     int lds_blk = 0;
     hipError_t e = hipDeviceGetAttribute(&lds_blk, hipDeviceAttributeMaxSharedMemoryPerBlock, dev);
     if (e != hipSuccess || lds_blk <= 64 * 1024) return e;
-    // allow the box kernels the device's whole per-block LDS, less 1 KiB for
-    // their own use (outside any graph capture)
-    lds_blk -= kLdsOwn;
+    // allow the kernels all of a block's LDS but their static part (outside any
+    // graph capture): a material table may take what the box leaves of it
+    const int box_lds = (int)mc_lds_limit(lds_blk);
     const void* box_kernels[] = {
         (const void*)mc_box_kernel<256, uint16_t, false>, (const void*)mc_box_kernel<1024, uint16_t, false>,
         (const void*)mc_box_kernel<256, double, false>,   (const void*)mc_box_kernel<1024, double, false>,
         (const void*)mc_box_kernel<256, uint16_t, true>,  (const void*)mc_box_kernel<1024, uint16_t, true>,
         (const void*)mc_box_kernel<256, double, true>,    (const void*)mc_box_kernel<1024, double, true>};
     for (const void* k : box_kernels) {
-        e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, lds_blk);
+        e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, box_lds);
         if (e != hipSuccess) return e;
     }
-    return hipFuncSetAttribute((const void*)mc_batch_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds_blk);
+    return hipFuncSetAttribute((const void*)mc_batch_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               lds_blk - (int)kBatchLds);
 }
 
 // The launch of a transport run: its blocks first, then the LDS box and table
@@ -896,9 +904,9 @@ McPlan mc_plan(const McArgs& a, const McDevice& dev)
             // blocks: LDS is given out in steps of lds_cu / 128
             p.tab_off = (int)((lds + 15) & ~(int64_t)15);
             const int64_t tab_lds = p.tab_off + (int64_t)sizeof(MatEntry) * a.nmat;
-            const int64_t own = sizeof(unsigned long long) * TAM_CNT_N, step = dev.lds_cu / 128;
-            const bool tab = a.mut_by_mat && tab_lds + own <= lds + kLdsOwn &&
-                             (tab_lds + own + step - 1) / step * step * p.per_cu <= dev.lds_cu;
+            const int64_t step = dev.lds_cu / 128;
+            const bool tab = a.mut_by_mat && tab_lds + kCountLds <= lds + kLdsOwn &&
+                             (tab_lds + kCountLds + step - 1) / step * step * p.per_cu <= dev.lds_cu;
             p.ntab = tab ? a.nmat : 0;
             p.lds = tab ? tab_lds : lds;
             return p;
@@ -930,7 +938,7 @@ extern "C" void tam_internal_mc_plan(const int64_t* in, int64_t* out)
     a.blocks_per_cu = (int)in[4]; a.box_enable = (int)in[5];
     a.nmat = (int)in[6]; a.mut_by_mat = (int)in[7]; a.full_grid = (int)in[8];
     const McPlan p = mc_plan(a, McDevice{(int)in[9], (int)in[10], (int)in[11]});
-    const int64_t r[] = {p.box, p.lanes, p.per_cu, p.blocks, p.sd, p.d, p.ntab, p.tab_off, p.lds};
+    const int64_t r[] = {p.box, p.lanes, p.per_cu, p.blocks, p.sd, p.d, p.ntab, p.tab_off, p.lds, mc_lds_limit(in[11])};
     std::copy(std::begin(r), std::end(r), out);
 }
 

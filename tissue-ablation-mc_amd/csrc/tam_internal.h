@@ -362,8 +362,9 @@ struct McPlan {
     int64_t lds;               // dynamic LDS of a block, bytes
 };
 McPlan mc_plan(const McArgs& a, const McDevice& dev);
+long mc_lds_limit(long lds_blk);      // dynamic LDS that mc_prepare allows the box kernels
 // the plan of (npk, nx, ny, nz, blocks_per_cu, box_enable, nmat, mut_by_mat, full_grid, ncu, lds_cu, lds_blk)
-// as (box, lanes, per_cu, blocks, sd, d, ntab, tab_off, lds); host only
+// as (box, lanes, per_cu, blocks, sd, d, ntab, tab_off, lds) and mc_lds_limit; host only
 extern "C" void tam_internal_mc_plan(const int64_t* in, int64_t* out);
 hipError_t launch_mc(const McArgs& a, hipStream_t s);
 // once per context, before any capture: lets the LDS-box kernel take the
