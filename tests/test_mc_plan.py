@@ -91,3 +91,14 @@ def test_no_plan_asks_for_more_lds_than_is_allowed():
         if p["ntab"]:                                           # and every block a CU finds its place
             step = LDS // 128
             assert -(-(p["lds"] + COUNTS) // step) * step * p["per_cu"] <= LDS, q
+
+
+@pytest.mark.parametrize("shape", range(1, 65))
+def test_batched_blocks_of_a_cu_find_their_lds(shape):
+    slots = lib.load().tam_internal_batch_slots(NCU, LDS, LDS, shape)
+    assert slots % 8 == 0 and slots >= 0
+    static, step = 4 * (COUNTS + 4 * 32), LDS // 128            # a wave's counts and four materials, four times
+    block = static + 4 * 2 * slots
+    assert block <= LDS and -(-block // step) * step * shape <= LDS
+    # and little of it stays idle: a step, the 1 KiB left beside the box, the rounding to 8 slots a wave
+    assert block > LDS // shape - step - 1024 - 64

@@ -799,6 +799,23 @@ McDevice mc_device()
     return d;
 }
 
+// 16-bit slots of a batched wave's LDS tally box: a quarter of its block's share
+// of the CU's LDS, less 1 KiB for the kernel's own use, in whole steps in which
+// LDS is given out (a share of lds_cu / 3 or / 5 is not: with the counts and
+// tables in it 2 blocks a CU were resident instead of 3, 4 instead of 5: eight
+// tissues of four materials 46.3 ms at 3 a CU, 42.2 now; of one 41.5, 40.9)
+int mc_batch_slots(const McDevice& dev, int bpc)
+{
+    const long step = dev.lds_cu / 128, whole = 128 / bpc * step;
+    const long box = std::min({(long)dev.lds_blk - kLdsOwn, (long)dev.lds_cu / bpc - kLdsOwn, whole - kBatchLds});
+    return box > 0 ? (int)(box / 4 / 2) & ~7 : 0;              // a multiple of 8 per wave
+}
+
+extern "C" int tam_internal_batch_slots(int ncu, int lds_cu, int lds_blk, int bpc)
+{
+    return mc_batch_slots(McDevice{ncu, lds_cu, lds_blk}, bpc);
+}
+
 hipError_t launch_mc_batch(const McArgs* dtab, int n, long total_npk, int blocks_per_cu, hipStream_t s)
 {
     if (n <= 0 || total_npk <= 0) return hipSuccess;
@@ -807,11 +824,7 @@ hipError_t launch_mc_batch(const McArgs* dtab, int n, long total_npk, int blocks
     long blocks = (long)dev.ncu * bpc;
     const long need = (total_npk + 255) / 256;
     if (need < blocks) blocks = need;
-    // per-wave LDS tally boxes: the block's share of the CU's LDS (1 KiB kept
-    // for the kernel's own use), split over its 4 waves
-    const long per_block = std::min((long)dev.lds_blk - kLdsOwn, (long)dev.lds_cu / bpc - kLdsOwn);
-    // 16-bit slots, a multiple of 8 per wave
-    const int wbox = per_block > 0 ? (int)(per_block / 4 / 2) & ~7 : 0;
+    const int wbox = mc_batch_slots(dev, bpc);
     const size_t lds = sizeof(uint16_t) * 4 * (size_t)wbox;
     hipLaunchKernelGGL(mc_batch_kernel, dim3((unsigned)blocks), dim3(256), lds, s, dtab, n, wbox);
     return hipGetLastError();
