@@ -102,3 +102,21 @@ def test_batched_blocks_of_a_cu_find_their_lds(shape):
     assert block <= LDS and -(-block // step) * step * shape <= LDS
     # and little of it stays idle: a step, the 1 KiB left beside the box, the rounding to 8 slots a wave
     assert block > LDS // shape - step - 1024 - 64
+
+
+@pytest.mark.parametrize("w", [4, 1024, 4096, 8192])
+@pytest.mark.parametrize("packets", [1, 70_000, 300_000, 1_000_000, 3_000_000, 10 ** 7, 3 * 10 ** 7, 10 ** 8, 10 ** 9])
+def test_queue_draws_stay_few_and_end_small(w, packets):
+    """The draws of all waves are one chain on one address.  A draw of 64 k
+    packets is made while 128 w k to 128 w (k + 1) are left (to 0 for k = 1):
+    4 w draws of 64 and 2 w / k of each further size up to 256, which is
+    never 3.7 w more than draws of 256 would be."""
+    last = C.c_int64()
+    f = lib.load().tam_internal_mc_draws
+    f.restype = C.c_int64
+    n = f(C.c_int64(packets), C.c_int64(w), C.byref(last))
+    left = max(0, packets - w * min(64, -(-packets // w)))
+    assert (n == 0) == (left == 0) and n <= -(-left // 64)
+    if left:
+        assert last.value == 64
+        assert n <= -(-left // 256) + 3.7 * w + 1

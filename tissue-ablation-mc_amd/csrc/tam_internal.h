@@ -366,6 +366,8 @@ long mc_lds_limit(long lds_blk);      // dynamic LDS that mc_prepare allows the 
 // the plan of (npk, nx, ny, nz, blocks_per_cu, box_enable, nmat, mut_by_mat, full_grid, ncu, lds_cu, lds_blk)
 // as (box, lanes, per_cu, blocks, sd, d, ntab, tab_off, lds) and mc_lds_limit; host only
 extern "C" void tam_internal_mc_plan(const int64_t* in, int64_t* out);
+// draws of a run from its packet queue, and the size of the last; host only
+extern "C" int64_t tam_internal_mc_draws(int64_t npk, int64_t waves, int64_t* last);
 hipError_t launch_mc(const McArgs& a, hipStream_t s);
 // once per context, before any capture: lets the LDS-box kernel take the
 // device's whole per-block LDS
