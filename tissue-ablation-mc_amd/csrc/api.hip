@@ -350,9 +350,9 @@ int check_flags(tam_ctx* c)
     return TAM_OK;
 }
 
-// A field to the caller's memory.  Pageable memory goes through the pinned
-// ring; what the device can write by itself is written directly, as is
-// everything where no ring can be had.
+// A field to the caller's memory.  Large ones to pageable memory go through the
+// pinned ring; what the device can write by itself is written directly, as is
+// everything that is small or has no ring.
 int download(tam_ctx* c, const void* src, StageKind kind, long n, double offset, double* out)
 {
     if (kind == STAGE_F64) {

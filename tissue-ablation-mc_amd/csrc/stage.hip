@@ -6,6 +6,7 @@
 // (56 GB/s) while a few threads move them on, converting on the way where the
 // device keeps a narrower type.  To a new array, before and after:
 // 64 MB 6.1 ms, 1.8; 134 MB 12.8, 3.5 (2.5 at the link's rate); 4 MB 0.7, 0.35.
+// Fields that are too small for it are copied plainly (stage_route).
 //
 // Rings outlive a context: pinning 16 MiB takes 0.7 ms.  Idle rings are kept
 // for any context (at most kIdleRings of them) and freed with the last context.
@@ -55,8 +56,9 @@ void ring_free(Ring* r)
     delete r;
 }
 
-// dev is the current device.  nullptr: no memory; the caller copies plainly.
-Ring* ring_take(int dev)
+// dev is the current device.  nullptr: none idle and none to be made, or no
+// memory; the caller copies plainly.
+Ring* ring_take(int dev, bool make)
 {
     {
         std::lock_guard<std::mutex> l(pool().mu);
@@ -67,7 +69,7 @@ Ring* ring_take(int dev)
                 return r;
             }
     }
-    Ring* r = new (std::nothrow) Ring;
+    Ring* r = make ? new (std::nothrow) Ring : nullptr;
     if (!r) return nullptr;
     r->dev = dev;
     // an allocation must not break a capture that another thread has under way
@@ -185,10 +187,26 @@ void stage_user(int delta)
     for (Ring* r : drop) ring_free(r);
 }
 
+// A field by the size of its result, in us plain and through a ring (FP64; FP32 or
+// bytes): 4 KiB 24, 14; 22-24, 14, so small ones take a ring that is idle, and
+// make none.  32 KiB 12, 20; 256 KiB 22, 30-40; 22, 28; 500 KiB 32, 40-48; 31, 35-44;
+// 1.4 MiB 87, 93-103; 70, 72.  2 MiB 122, 116; 130, 78, and all larger ones.
+// (A plain copy of less than 16 KiB costs more than one of 32, and so does a
+// narrower field's below 160 KiB of result: 24^3 41 us, 23.)
+StageRoute stage_route(StageKind kind, long n)
+{
+    const size_t bytes = sizeof(double) * (size_t)n;
+    if (bytes >= kSlotBytes) return STAGE_RING;
+    return bytes < (size_t)(kind == STAGE_F64 ? 16 : 160) << 10 ? STAGE_IDLE : STAGE_PLAIN;
+}
+
+extern "C" int tam_internal_stage_route(int kind, int64_t n) { return (int)stage_route((StageKind)kind, (long)n); }
+
 hipError_t stage_download(int dev, hipStream_t s, const void* src, StageKind kind, long n, double offset, double* out)
 {
     if (n <= 0) return hipSuccess;
-    Ring* r = ring_take(dev);
+    const StageRoute route = stage_route(kind, n);
+    Ring* r = route == STAGE_PLAIN ? nullptr : ring_take(dev, route == STAGE_RING);
     if (!r) return hipErrorOutOfMemory;
     Job j;
     j.ring = r;

@@ -410,7 +410,11 @@ hipError_t launch_heat64_step(const Heat64Args& a, const double* Tin, double* To
 hipError_t launch_coeffs64(const Coeff64Args& a, hipStream_t s);
 // field downloads (stage.hip): out[i] = src[i], or offset + src[i] (FP32), or the byte
 enum StageKind { STAGE_F64, STAGE_F32, STAGE_U8 };
+enum StageRoute { STAGE_PLAIN, STAGE_IDLE, STAGE_RING };     // a plain copy; an idle ring or a plain copy; a ring
+StageRoute stage_route(StageKind kind, long n);
+extern "C" int tam_internal_stage_route(int kind, int64_t n);     // host only
 void stage_user(int delta);    // +1 / -1 per context: idle rings go with the last
+// hipErrorOutOfMemory: no ring; the caller copies plainly
 hipError_t stage_download(int dev, hipStream_t s, const void* src, StageKind kind, long n, double offset, double* out);
 hipError_t launch_clear(double* f, long n, unsigned long long* counters, long m, hipStream_t s);
 hipError_t launch_arrhenius(const RebuildArgs& a, const ArrArgs& arr, hipStream_t s);
