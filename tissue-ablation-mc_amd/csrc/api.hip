@@ -1464,13 +1464,7 @@ int tam_tune_heat(tam_ctx* c, int32_t reps, int32_t* tile, int32_t* kz, double* 
         a.eblk = eb;
         a.Q = qs;
         const int boil = c->p.boil != 0, robin = c->p.robin_top != 0, dmg = c->p.damage_every_step != 0;
-        // Shallow marches give a grid of some 10^5 voxels enough blocks (50^3 6.5 us a
-        // step at 4, 4.4 at 2; 80^3 5.2 at 4, 4.7 at 3; 113x97x101 6.5 at 4, 6.3 at 6);
-        // deep ones leave it too few.  From 4 blocks a CU at depth 4 on (420 columns a
-        // block) the shallow ones lose (120^3 12.6 at 4, 14.5 at 2).
-        static const int small[] = {2, 3, 4, 6, 8, 12, 16}, large[] = {4, 8, 12, 16, 32, 64};
-        const bool few = c->nvox < 4L * 256 * 420 * 4;
-        const std::vector<int> kzs(few ? small : large, few ? small + 7 : large + 6);
+        const int ncu = mc_device().ncu;
         const bool two_ok = !boil && c->lut;
         const double ta = c->time + c->p.delt;
         for (int t = 0; t < heat_num_tiles() && e == hipSuccess; ++t) {
@@ -1479,8 +1473,7 @@ int tam_tune_heat(tam_ctx* c, int32_t reps, int32_t* tile, int32_t* kz, double* 
             // class mode: the LDS-plane shapes (0-2) are slower than their
             // direct twins on every measured workload; they stay settable
             if (c->lut && t <= 2) continue;
-            for (int kk : kzs) {
-                if (kk > c->p.nz && kk != kzs[0]) continue;
+            for (int kk : heat_depths(t, c->p.nx, c->p.ny, c->p.nz, ncu)) {
                 // a two-step candidate launches two steps, timed per step
                 auto run = [&]() {
                     return two ? launch_heat_step2(a, c->cur, c->nxt, 1.f, 1.f, ta, ta + c->p.delt, robin, dmg, 1, t,

@@ -26,6 +26,7 @@
 // the owned tile, handed to the second through LDS.
 #include "tam_internal.h"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace {
@@ -967,6 +968,33 @@ int heat_tile_dims(int tile, int* tx, int* ty)
     *tx = d[tile][0];
     *ty = d[tile][1];
     return 0;
+}
+
+// March depths worth timing for a shape on a grid, by the blocks they give it.
+// Fewer than half a block a CU: a shallower march ends sooner, its blocks still
+// on CUs of their own.  Fewer than 4 a CU at depth 4: shallow ones gain (32x16
+// two-step: 50^3 6.5 us a step at 4, 4.4 at 2; 80^3 5.2 at 4, 4.7 at 3); from
+// there on they lose (120^3 12.6 at 4, 14.5 at 2).  6 fills the CUs once where 4
+// needs another round (119^3 8.1, 8.8 at 4 and 8).
+std::vector<int> heat_depths(int tile, int nx, int ny, int nz, int ncu)
+{
+    int tx = 1, ty = 1;
+    heat_tile_dims(tile, &tx, &ty);
+    auto blocks = [&](int kz) { return (long)((nx + tx - 1) / tx) * ((ny + ty - 1) / ty) * ((nz + kz - 1) / kz); };
+    const bool few = blocks(4) < 4L * ncu;
+    std::vector<int> out;
+    for (int kz : {2, 3, 4, 6, 8, 12, 16, 32, 64}) {
+        if (kz < 4 ? !few : kz > 4 && 2 * blocks(kz) < ncu) continue;
+        if (kz <= nz || out.empty()) out.push_back(kz);
+    }
+    return out;
+}
+
+extern "C" int tam_internal_heat_depths(int tile, int nx, int ny, int nz, int ncu, int* out)
+{
+    const std::vector<int> d = heat_depths(tile, nx, ny, nz, ncu);
+    std::copy(d.begin(), d.end(), out);
+    return (int)d.size();
 }
 
 hipError_t launch_heat_batch(const HeatBatchEntry* tab, int n, const int* tile_start, int total_tiles, float lon,

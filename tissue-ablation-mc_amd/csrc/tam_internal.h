@@ -17,6 +17,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 #include <string>
+#include <vector>
 
 #include "../../include/tam.h"
 
@@ -394,6 +395,8 @@ hipError_t launch_heat_step2(const HeatArgs& a, const float* Tin, float* Tout, f
                              double time_after0, double time_after1, int robin, int damage, int energy, int tile,
                              int kz, hipStream_t s);
 // upper bound of the block count of any heat launch shape (energy slots)
+std::vector<int> heat_depths(int tile, int nx, int ny, int nz, int ncu);
+extern "C" int tam_internal_heat_depths(int tile, int nx, int ny, int nz, int ncu, int* out);     // host only
 long heat_max_blocks(int nx, int ny, int nz);
 // one step of every instance of a table (direct shapes 3-5 only); parity 0
 // reads cur and writes nxt, parity 1 the reverse
