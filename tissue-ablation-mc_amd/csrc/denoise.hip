@@ -1209,7 +1209,7 @@ constexpr int LEVEL[NL] = {0, 0, 1, 1, 2, 2, 1, 1, 0, 0};
 }  // namespace
 
 struct tam_dn {
-    int dev;
+    int dev, ncu;
     hipStream_t stream;
     hipEvent_t ev0, ev1;
     std::string err;
@@ -1307,7 +1307,7 @@ struct BrickPlan {
     int ny, ndz;
     long nb, per;
 };
-bool brick_plan(int D, int H, int W, int cin, int cout, BrickPlan* bp)
+bool brick_plan(int ncu, int D, int H, int W, int cin, int cout, BrickPlan* bp)
 {
     if (W % 16 != 0 || H % 8 != 0 || D % 4 != 0 || cin % 16 != 0) return false;
     if (cout != 16 && cout != 32 && cout != 64) return false;
@@ -1318,13 +1318,23 @@ bool brick_plan(int D, int H, int W, int cin, int cout, BrickPlan* bp)
     // channels one), with the same number of bricks each: at 128^3 16 to 16
     // channels 85 us with 1024 blocks, 78; 64 outputs 44, 36; the partials' sum
     // 9.4, 5.8
-    long nb = 256 * (cout == 64 ? 1 : 2) / bp->ny;
+    long nb = (long)ncu * (cout == 64 ? 1 : 2) / bp->ny;
     if (nb < 1) nb = 1;
     const long each = (bricks + nb - 1) / nb;
     bp->nb = (bricks + each - 1) / each;
     bp->per = (27 / bp->ndz) * 16L * cout + cout;
     return true;
 }
+
+}  // namespace
+
+extern "C" int64_t tam_internal_brick_blocks(int ncu, int D, int H, int W, int cin, int cout)
+{
+    BrickPlan bp;
+    return brick_plan(ncu, D, H, W, cin, cout, &bp) ? bp.nb * bp.ny : 0;
+}
+
+namespace {
 
 // weight gradient of one layer into gw; the brick form also sums the bias
 // gradient into gb and says so in *bias_done
@@ -1333,7 +1343,7 @@ hipError_t wgrad_launch(tam_dn* n, const uint16_t* x, const uint16_t* dy, int lv
 {
     *bias_done = false;
     BrickPlan bp;
-    if (brick_plan(n->D[lvl], n->H[lvl], n->W[lvl], cin, cout, &bp) && n->wpart &&
+    if (brick_plan(n->ncu, n->D[lvl], n->H[lvl], n->W[lvl], cin, cout, &bp) && n->wpart &&
         (long)bp.ny * bp.nb * bp.per <= n->wpart_n) {
         WgradbArgs b{x, dy, n->wpart, n->D[lvl], n->H[lvl], n->W[lvl], cin, cout,
                      (long)(n->W[lvl] / 16) * (n->H[lvl] / 8) * (n->D[lvl] / 4), x2, c1};
@@ -1567,6 +1577,7 @@ int tam_dn_create(int32_t device, int32_t nx, int32_t ny, int32_t nz, int32_t ca
     if (!n) return TAM_ERR_NOMEM;
     n->dev = device;
     DevScope ds(device);
+    n->ncu = mc_device().ncu;
     for (int l = 0; l < 3; ++l) {
         n->W[l] = nx >> l;
         n->H[l] = ny >> l;
@@ -1621,7 +1632,7 @@ int tam_dn_create(int32_t device, int32_t nx, int32_t ny, int32_t nz, int32_t ca
     for (int l = 0; l < NL; ++l) {
         const Layer& L = n->L[l];
         BrickPlan bp;
-        if (brick_plan(n->D[L.level], n->H[L.level], n->W[L.level], L.cin, L.cout, &bp))
+        if (brick_plan(n->ncu, n->D[L.level], n->H[L.level], n->W[L.level], L.cin, L.cout, &bp))
             n->wpart_n = std::max(n->wpart_n, (long)bp.ny * bp.nb * bp.per);
     }
     if (n->wpart_n > 0) al((void**)&n->wpart, sizeof(float) * n->wpart_n);

@@ -433,6 +433,8 @@ hipError_t launch_normalise(int nx, int ny, int nz, long px, long pxy, const dou
                             const double* rhokap, const uint8_t* mat, const double* mua_frac,
                             const CycleHdr* dyn, double scale, const double* coeff, double* jmean,
                             float* src, unsigned long long* acc, const unsigned long long* counters, hipStream_t s);
+// blocks of a denoiser layer's brick weight gradient (0: another form); host only
+extern "C" int64_t tam_internal_brick_blocks(int ncu, int D, int H, int W, int cin, int cout);
 hipError_t launch_fill_f64(double* p, long n, double v, hipStream_t s);
 // error of a call that has no context (read back by tam_last_error(NULL))
 int tam_fail_noctx(int code, const std::string& msg);
