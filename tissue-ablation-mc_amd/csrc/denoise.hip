@@ -487,126 +487,6 @@ __global__ __launch_bounds__(256) void wgrad_kernel(WgradArgs a)
         if (sR[q] != 0.f) atomicAdd(&a.gw[(long)tap * CI * CO + q], sR[q]);
 }
 
-// Weight gradient of the three taps dx = -1, 0, 1 that share (dz, dy) = blockIdx.y over a range of 32-voxel row
-// segments (rows of W % 32 == 0 voxels, so a segment never leaves its row).  Each wave stages its segment's dy and
-// the 34 x voxels x0-1 .. x0+32 of the source row (z+dz, y+dy) in its own LDS slice, channel-major; the operand
-// of tap dx is the aligned 8-voxel fragment shifted by one bf16 (v_alignbyte on dword pairs), so one staging
-// serves three taps.  Segments whose source row lies outside the grid contribute nothing and are skipped.
-template <int CIT, int COT>
-__global__ __launch_bounds__(256) void wgrad3_kernel(WgradArgs a)
-{
-    constexpr int CI = CIT * 16, CO = COT * 16;
-    constexpr int XR = 48;                                  // x row: element 8 + v holds voxel x0 + v (v = -1 .. 32)
-    constexpr int DR = 40;                                  // dy row: 32 voxels + pad against bank conflicts
-    __shared__ __attribute__((aligned(16))) uint16_t sX[4][CI][XR];
-    __shared__ __attribute__((aligned(16))) uint16_t sD[4][CO][DR];
-    __shared__ float sR[CI * CO];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    const int dz = (int)blockIdx.y / 3 - 1, dy = (int)blockIdx.y % 3 - 1;
-    f32x4 acc[3][COT][CIT];
-#pragma unroll
-    for (int s = 0; s < 3; ++s)
-#pragma unroll
-        for (int i = 0; i < COT; ++i)
-#pragma unroll
-            for (int c = 0; c < CIT; ++c) acc[s][i][c] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-    const long b0 = (long)blockIdx.x * a.per_wg;
-    const long b1 = b0 + a.per_wg < a.blocks ? b0 + a.per_wg : a.blocks;
-    const int k8 = (lane >> 4) * 8, r16 = lane & 15;
-    for (long blk = b0 + wv; blk < b1; blk += 4) {
-        const long m0 = blk * 32;
-        const int x0 = (int)(m0 % a.W);
-        const long r = m0 / a.W;
-        const int sy = (int)(r % a.H) + dy, sz = (int)(r / a.H) + dz;
-        if (sy < 0 || sy >= a.H || sz < 0 || sz >= a.D) continue;      // wave-uniform
-        // staging by voxel pairs: each lane loads 8 channels of two neighbouring voxels and writes one dword
-        // (both voxels) per channel
-        for (int q = lane; q < 16 * (CO / 8); q += 64) {
-            const int p = q / (CO / 8), c8 = (q % (CO / 8)) * 8;
-            const uint4 d0 = *(const uint4*)(a.dy + (m0 + 2 * p) * a.cout + c8);
-            const uint4 d1 = *(const uint4*)(a.dy + (m0 + 2 * p + 1) * a.cout + c8);
-            const uint16_t* e0 = (const uint16_t*)&d0;
-            const uint16_t* e1 = (const uint16_t*)&d1;
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-                *(uint32_t*)&sD[wv][c8 + j][2 * p] = (uint32_t)e0[j] | ((uint32_t)e1[j] << 16);
-        }
-        const long srow = ((long)sz * a.H + sy) * a.W;
-        // pairs p = 0 .. 17: voxels x0 + 2p - 2 and x0 + 2p - 1 at elements 2p + 6, 2p + 7 (elements 7 .. 40 are
-        // the ones read; 6 and 41 come along)
-        for (int q = lane; q < 18 * (CI / 8); q += 64) {
-            const int p = q / (CI / 8), c8 = (q % (CI / 8)) * 8;
-            const int sx = x0 + 2 * p - 2;
-            uint4 d0 = make_uint4(0u, 0u, 0u, 0u), d1 = make_uint4(0u, 0u, 0u, 0u);
-            if (sx >= 0 && sx < a.W) d0 = *(const uint4*)(a.x + (srow + sx) * a.cin + c8);
-            if (sx + 1 >= 0 && sx + 1 < a.W) d1 = *(const uint4*)(a.x + (srow + sx + 1) * a.cin + c8);
-            const uint16_t* e0 = (const uint16_t*)&d0;
-            const uint16_t* e1 = (const uint16_t*)&d1;
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-                *(uint32_t*)&sX[wv][c8 + j][2 * p + 6] = (uint32_t)e0[j] | ((uint32_t)e1[j] << 16);
-        }
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");         // the slice is written before it is read
-        __builtin_amdgcn_wave_barrier();
-        bf16x8 bx[3][CIT];
-#pragma unroll
-        for (int c = 0; c < CIT; ++c) {
-            const uint16_t* row = &sX[wv][c * 16 + r16][0];
-            const uint4 mid = *(const uint4*)(row + 8 + k8);                  // voxels k8 .. k8+7
-            const unsigned prev = *(const unsigned*)(row + 6 + k8);          // high half: voxel k8-1
-            const unsigned next = *(const unsigned*)(row + 16 + k8);         // low half: voxel k8+8
-            uint4 lo, hi;
-            lo.x = __builtin_amdgcn_alignbyte(mid.x, prev, 2);
-            lo.y = __builtin_amdgcn_alignbyte(mid.y, mid.x, 2);
-            lo.z = __builtin_amdgcn_alignbyte(mid.z, mid.y, 2);
-            lo.w = __builtin_amdgcn_alignbyte(mid.w, mid.z, 2);
-            hi.x = __builtin_amdgcn_alignbyte(mid.y, mid.x, 2);
-            hi.y = __builtin_amdgcn_alignbyte(mid.z, mid.y, 2);
-            hi.z = __builtin_amdgcn_alignbyte(mid.w, mid.z, 2);
-            hi.w = __builtin_amdgcn_alignbyte(next, mid.w, 2);
-            bx[0][c] = __builtin_bit_cast(bf16x8, lo);
-            bx[1][c] = __builtin_bit_cast(bf16x8, mid);
-            bx[2][c] = __builtin_bit_cast(bf16x8, hi);
-        }
-#pragma unroll
-        for (int i = 0; i < COT; ++i) {
-            const bf16x8 ad = load8(&sD[wv][i * 16 + r16][k8]);
-#pragma unroll
-            for (int s = 0; s < 3; ++s)
-#pragma unroll
-                for (int c = 0; c < CIT; ++c)
-                    acc[s][i][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ad, bx[s][c], acc[s][i][c], 0, 0, 0);
-        }
-        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");         // the reads finish before the next writes
-        __builtin_amdgcn_wave_barrier();
-    }
-    // per tap: reduce the four waves in LDS, then one atomic per weight
-#pragma unroll
-    for (int s = 0; s < 3; ++s) {
-        for (int q = threadIdx.x; q < CI * CO; q += 256) sR[q] = 0.f;
-        __syncthreads();
-        for (int w = 0; w < 4; ++w) {
-            if (wv == w) {
-#pragma unroll
-                for (int i = 0; i < COT; ++i)
-#pragma unroll
-                    for (int c = 0; c < CIT; ++c)
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) {
-                            const int co = i * 16 + (lane >> 4) * 4 + j, ci = c * 16 + (lane & 15);
-                            sR[ci * CO + co] += acc[s][i][c][j];
-                        }
-            }
-            __syncthreads();
-        }
-        const int tap = (int)blockIdx.y * 3 + s;
-        for (int q = threadIdx.x; q < CI * CO; q += 256)
-            if (sR[q] != 0.f) atomicAdd(&a.gw[(long)tap * CI * CO + q], sR[q]);
-        __syncthreads();
-    }
-}
-
 // Weight gradient by output bricks, all of a 16-channel input tile's taps at
 // once: dW^T[co][ci] += sum_m dy[m][co] x[m + tap][ci].
 //
@@ -1311,7 +1191,7 @@ bool brick_plan(int ncu, int D, int H, int W, int cin, int cout, BrickPlan* bp)
 {
     if (W % 16 != 0 || H % 8 != 0 || D % 4 != 0 || cin % 16 != 0) return false;
     if (cout != 16 && cout != 32 && cout != 64) return false;
-    bp->ndz = (cout == 16 && cin <= 48) ? 1 : 3;           // all 27 taps' sums in registers when they fit
+    bp->ndz = cout == 16 ? 1 : 3;                          // all 27 taps' sums in registers when they fit
     bp->ny = (cin / 16) * bp->ndz;
     const long bricks = (long)(W / 16) * (H / 8) * (D / 4);
     // one round of resident blocks (their LDS lets a CU hold two, of 64 output
@@ -1348,10 +1228,9 @@ hipError_t wgrad_launch(tam_dn* n, const uint16_t* x, const uint16_t* dy, int lv
         WgradbArgs b{x, dy, n->wpart, n->D[lvl], n->H[lvl], n->W[lvl], cin, cout,
                      (long)(n->W[lvl] / 16) * (n->H[lvl] / 8) * (n->D[lvl] / 4), x2, c1};
         const dim3 grid((unsigned)bp.nb, (unsigned)bp.ny);
-        if (c4 && (cout != 16 || bp.ndz != 1)) return hipErrorInvalidValue;
+        if (c4 && cout != 16) return hipErrorInvalidValue;
         if (c4) hipLaunchKernelGGL((wgradb_kernel<1, 1, true>), grid, dim3(256), 0, n->stream, b);
-        else if (cout == 16 && bp.ndz == 1) hipLaunchKernelGGL((wgradb_kernel<1, 1, false>), grid, dim3(256), 0, n->stream, b);
-        else if (cout == 16) hipLaunchKernelGGL((wgradb_kernel<1, 3, false>), grid, dim3(256), 0, n->stream, b);
+        else if (cout == 16) hipLaunchKernelGGL((wgradb_kernel<1, 1, false>), grid, dim3(256), 0, n->stream, b);
         else if (cout == 32) hipLaunchKernelGGL((wgradb_kernel<2, 3, false>), grid, dim3(256), 0, n->stream, b);
         else hipLaunchKernelGGL((wgradb_kernel<4, 3, false>), grid, dim3(256), 0, n->stream, b);
         // ~1024 reduction blocks: each weight's nb partials split over ksplit of them
@@ -1365,35 +1244,18 @@ hipError_t wgrad_launch(tam_dn* n, const uint16_t* x, const uint16_t* dy, int lv
         return hipGetLastError();
     }
     if (x2 || c4) return hipErrorInvalidValue;  // read by the brick form only
+    // one workgroup per tap and range of segments, ~96 per tap
     WgradArgs a{x, dy, gw, n->D[lvl], n->H[lvl], n->W[lvl], cin, cout, 0, 0};
     a.blocks = n->nv[lvl] / 32;
-    // rows of whole 32-voxel segments: one workgroup per (dz, dy) covers the three dx taps, ~288 per (dz, dy);
-    // otherwise one per tap, ~96 per tap (~2600 workgroups in all either way)
-    // (the 64 x 64 layer keeps one workgroup per tap: three taps' accumulators leave it one wave per SIMD)
-    const bool rows = n->W[lvl] % 32 == 0 && (cin / 16) * (cout / 16) <= 12;
-    const long wgs = rows ? 288 : 96;
-    long per = (a.blocks + wgs - 1) / wgs;
+    long per = (a.blocks + 95) / 96;
     per = (per + 3) / 4 * 4;
     if (per < 4) per = 4;
     a.per_wg = per;
-    const dim3 grid((unsigned)((a.blocks + per - 1) / per), rows ? 9 : 27);
-#define WG(CI, CO)                                                                                     \
-    do {                                                                                               \
-        if (rows) hipLaunchKernelGGL((wgrad3_kernel<CI, CO>), grid, dim3(256), 0, n->stream, a);       \
-        else hipLaunchKernelGGL((wgrad_kernel<CI, CO>), grid, dim3(256), 0, n->stream, a);             \
-    } while (0)
-    const int key = (cin / 16) * 16 + cout / 16;
-    switch (key) {
-    case 1 * 16 + 1: WG(1, 1); break;
-    case 1 * 16 + 2: WG(1, 2); break;
-    case 2 * 16 + 2: WG(2, 2); break;
-    case 2 * 16 + 4: WG(2, 4); break;
-    case 4 * 16 + 4: WG(4, 4); break;
-    case 6 * 16 + 2: WG(6, 2); break;
-    case 3 * 16 + 1: WG(3, 1); break;
-    default: return hipErrorInvalidValue;
-    }
-#undef WG
+    const dim3 grid((unsigned)((a.blocks + per - 1) / per), 27);
+    // the layers of the quarter grid, whose x edge may be an odd multiple of 8
+    if (cin == 32 && cout == 64) hipLaunchKernelGGL((wgrad_kernel<2, 4>), grid, dim3(256), 0, n->stream, a);
+    else if (cin == 64 && cout == 64) hipLaunchKernelGGL((wgrad_kernel<4, 4>), grid, dim3(256), 0, n->stream, a);
+    else return hipErrorInvalidValue;
     return hipGetLastError();
 }
 

@@ -105,6 +105,7 @@ __global__ __launch_bounds__(256) void update_kernel(RebuildArgs a, ArrArgs arr)
     a.mask[v] = (uint8_t)(b || (u && bx && by && bz));
 }
 
+// the FP32 step's properties (coeff64_kernel<true> does the FP64 step's)
 __global__ __launch_bounds__(256) void props_kernel(RebuildArgs a)   // 3dFD.f90:334-357
 {
     const long nv = (long)a.nx * a.ny * a.nz;
@@ -114,7 +115,7 @@ __global__ __launch_bounds__(256) void props_kernel(RebuildArgs a)   // 3dFD.f90
     vox_ijk(v, a.nx, a.ny, i, j, k);
     const long c = i + a.px * j + a.pxy * k;
     if (a.mask[v]) {
-        const double T = a.T64 ? a.T64[c] : a.t_ref + (double)a.dT[c];
+        const double T = a.t_ref + (double)a.dT[c];
         const double rho = air_density(T);
         const double hc = 1.006e3;
         a.density[c] = rho;
