@@ -70,3 +70,37 @@ def test_material_tables_at_the_lds_limit(materials):
         np.testing.assert_allclose(ta, tb, rtol=1e-9, atol=1e-9 * tb.max())
     a.close()
     b.close()
+
+
+# a batched wave's table holds 4 entries, air included; past that mu_t comes from the array
+@pytest.mark.parametrize("materials", [3, 4, 9])
+@pytest.mark.parametrize("shape", [3, 4])
+def test_batched_tissues_of_several_materials(materials, shape):
+    print("case: batch,", materials, "materials,", shape, "blocks a CU", flush=True)
+    probs = []
+    for q, n in enumerate(((33, 28, 40), (48, 48, 48), (20, 61, 17))):
+        prob = configs.three_layer_skin(n=n, ext=(0.5, 0.5, 0.25), packets=1, steps=1)
+        prob.table = [(2.0 + 0.3 * m, 90.0 + 5.0 * q + m, 0.8, 1.4) for m in range(materials)]
+        prob.mat = (np.arange(prob.mat.size) % materials).astype(np.uint8).reshape(prob.mat.shape)
+        prob.params.damage_every_step = 0
+        probs.append(prob)
+    gs = [p.grid() for p in probs]
+    b = lib.Batch(gs)
+    b.set_launch(4, 8, shape, 32)
+    npk = [60_000, 150_000, 40_000]
+    st = b.mc_run(npk, seed=6, stream0=2)
+    tb = [g.download(lib.FIELD_TALLY) for g in gs]
+    b.close()
+    for i, g in enumerate(gs):
+        g.set_mc_launch(8, 32)
+        g.set_mc_box(False)
+        s1 = g.mc_run(npk[i], seed=6, stream=2 + i)
+        t1 = g.download(lib.FIELD_TALLY)
+        for k in ("absorbed", "specular", "missed", "killed", "crossings", "interactions", "tally_adds"):
+            assert getattr(st[i], k) == getattr(s1, k), (i, k)
+        assert list(st[i].escaped) == list(s1.escaped)
+        p = probs[i].params
+        # deposits rounded to the box's unit, half a unit each: as for one material (test_gpu_batch)
+        unit = 2.0 * (p.xmax / p.nx + p.ymax / p.ny + p.zmax / p.nz) / 2 ** 13
+        np.testing.assert_allclose(tb[i], t1, rtol=1e-4, atol=16 * unit)
+        g.close()
