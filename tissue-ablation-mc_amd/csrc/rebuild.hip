@@ -71,7 +71,7 @@ __global__ __launch_bounds__(256) void arrhenius_kernel(RebuildArgs a, ArrArgs a
     int i, j, k;
     vox_ijk(v, a.nx, a.ny, i, j, k);
     const long c = i + a.px * j + a.pxy * k;
-    arrhenius_voxel(arr, v, nv, cell_T(a, c), a.rhokap[c]);
+    arrhenius_voxel(arr, v, nv, cell_T(a, c), [&] { return a.rhokap[c]; });
 }
 
 // What a coupling cycle does per voxel from the temperatures and the rhokap
@@ -90,7 +90,7 @@ __global__ __launch_bounds__(256) void update_kernel(RebuildArgs a, ArrArgs arr)
     const long c = i + a.px * j + a.pxy * k;
     const double* rk = a.rhokap;
     const double T = cell_T(a, c), rc = rk[c];
-    if (ARR) arrhenius_voxel(arr, v, nv, T, rc);
+    if (ARR) arrhenius_voxel(arr, v, nv, T, [&] { return rc; });
     if (WATER) {
         double w = kW0 - kW0 * (a.Q[v] / a.qvapor);
         w = fmin(fmin(w, kW0), a.W[v]);
