@@ -47,6 +47,22 @@ Pool& pool()
     return *p;
 }
 
+// The calling thread in another capture mode for a scope: what HIP refuses while
+// a stream is being captured goes by the mode of the thread that asks.
+struct CaptureMode {
+    hipStreamCaptureMode old;
+    bool swapped;
+    explicit CaptureMode(hipStreamCaptureMode mode)
+        : old(mode), swapped(hipThreadExchangeStreamCaptureMode(&old) == hipSuccess)
+    {
+    }
+    ~CaptureMode()
+    {
+        if (swapped) (void)hipThreadExchangeStreamCaptureMode(&old);
+    }
+    CaptureMode(const CaptureMode&) = delete;
+};
+
 void ring_free(Ring* r)
 {
     if (!r) return;
@@ -72,13 +88,14 @@ Ring* ring_take(int dev, bool make)
     Ring* r = make ? new (std::nothrow) Ring : nullptr;
     if (!r) return nullptr;
     r->dev = dev;
-    // an allocation must not break a capture that another thread has under way
-    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
-    const bool swapped = hipThreadExchangeStreamCaptureMode(&mode) == hipSuccess;
-    hipError_t e = hipHostMalloc((void**)&r->pin, kSlots * kSlotBytes, hipHostMallocDefault);
-    for (hipEvent_t& ev : r->ev)
-        if (e == hipSuccess) e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
-    if (swapped) (void)hipThreadExchangeStreamCaptureMode(&mode);
+    hipError_t e;
+    {
+        // an allocation must not break a capture that another thread has under way
+        const CaptureMode relaxed(hipStreamCaptureModeRelaxed);
+        e = hipHostMalloc((void**)&r->pin, kSlots * kSlotBytes, hipHostMallocDefault);
+        for (hipEvent_t& ev : r->ev)
+            if (e == hipSuccess) e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+    }
     if (e != hipSuccess) {
         (void)hipGetLastError();
         ring_free(r);
@@ -222,12 +239,15 @@ hipError_t stage_download(int dev, hipStream_t s, const void* src, StageKind kin
     j.chunks = 1 + (n - j.first + j.chunk - 1) / j.chunk;
     for (auto& q : j.issued) q = -1;
     for (long k = 0; k < std::min<long>(j.chunks, kSlots); ++k) issue(j, k);
+    // the threads wait as the caller may: in its capture mode, not a new thread's
+    const hipStreamCaptureMode mode = CaptureMode(hipStreamCaptureModeRelaxed).old;
     const long want = std::min<long>({(long)kThreads, j.chunks, (long)(n * sizeof(double) / kSlotBytes)});
     std::thread extra[kThreads];
     int started = 0;
     try {
         for (; started + 1 < want; ++started)
-            extra[started] = std::thread([&j, dev] {
+            extra[started] = std::thread([&j, dev, mode] {
+                const CaptureMode own(mode);
                 const hipError_t e = hipSetDevice(dev);
                 if (e != hipSuccess) j.err = (int)e;
                 work(j);
