@@ -47,3 +47,30 @@ def test_a_relaxed_thread_downloads_during_a_capture(n, mode):
     hip.hipGraphDestroy(graph)
     hip.hipStreamDestroy(s)
     g.close()
+
+
+@pytest.mark.parametrize("n", [64, 130])
+def test_a_refused_download_leaves_the_ring_sound(n):
+    """In global mode the wait is refused, as it is without the ring; the
+    copies that were sent end before another download has their slots."""
+    print("case", n, flush=True)
+    a, b = (configs.three_layer_skin(n=(n, n, n), ext=(2.0, 2.0, 1.0), packets=1, steps=1).grid() for _ in range(2))
+    for q, g in enumerate((a, b)):
+        g.upload(lib.FIELD_JMEAN, np.random.default_rng(q).random((n, n, n)))
+    want = b.download(lib.FIELD_JMEAN)
+    hip = _hip()
+    s, graph = C.c_void_p(), C.c_void_p()
+    assert hip.hipStreamCreateWithFlags(C.byref(s), 1) == 0
+    assert hip.hipStreamBeginCapture(s, GLOBAL) == 0
+    try:
+        with pytest.raises(lib.TamError):
+            a.download(lib.FIELD_JMEAN)
+    finally:
+        hip.hipStreamEndCapture(s, C.byref(graph))                            # the refusal has ended it
+    hip.hipGetLastError()
+    for _ in range(3):
+        assert np.array_equal(b.download(lib.FIELD_JMEAN), want)
+    assert np.array_equal(a.download(lib.FIELD_JMEAN), np.random.default_rng(0).random((n, n, n)))
+    hip.hipStreamDestroy(s)
+    a.close()
+    b.close()

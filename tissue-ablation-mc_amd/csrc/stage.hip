@@ -256,8 +256,15 @@ hipError_t stage_download(int dev, hipStream_t s, const void* src, StageKind kin
     }
     work(j);
     for (int t = 0; t < started; ++t) extra[t].join();
-    const hipError_t done = hipStreamSynchronize(s);   // also before the slots go to another download
+    // before the slots go to another download no copy to them may be on its way,
+    // also where the caller's wait is refused (its capture mode) or a thread gave up
+    const hipError_t done = hipStreamSynchronize(s);
+    hipError_t settled = done;
+    if (settled != hipSuccess) {
+        const CaptureMode relaxed(hipStreamCaptureModeRelaxed);
+        settled = hipStreamSynchronize(s);
+    }
     const hipError_t e = (hipError_t)j.err.load();
-    ring_give(r);
+    if (settled == hipSuccess) ring_give(r);            // else lost with its device
     return e != hipSuccess ? e : done;
 }
