@@ -46,8 +46,6 @@ constexpr int kMaxDevices = 64;
 // tam_tune_mc keeps the CU-wide LDS tally box when it times within this
 // fraction of the fastest candidate
 constexpr double kWideBoxMargin = 0.10;
-// ... and a random-phase batch of 32 when it times within this fraction of the fastest batch
-constexpr double kBatchMargin = 0.03;
 std::mutex scratch_mu;
 double* scratch_dev[kMaxDevices] = {};
 
@@ -1370,8 +1368,11 @@ int tam_tune_mc(tam_ctx* c, int64_t sample, int32_t* blocks_per_cu, int32_t* rng
     // Ties go to the single CU-wide box (box on, 1024-lane blocks, one per
     // CU): candidates are timed on the tissue as it is, and once a crater
     // forms and the deposition moves below it, the largest box holds its lead
-    // (c1 crater phase: 360 ms per 1e8 packets against 465 ms for three
-    // boxes per CU, which can be a few percent ahead on fresh tissue).
+    // (three-layer skin at 200^3 after 3 cycles: 299 ms per 1e8 packets, 355 and
+    // 358 with two boxes per CU, 404 with three; on the fresh tissue the sample
+    // of 5e6 has one and two within 1 %).  The batch is the fastest one's: after
+    // 3 and after 15 cycles 8 to 48 are within 0.2 %, and the fresh tissue is
+    // fastest at 40 and 48 (57 ms per 1e8, 59 at 32, 60 at 8).
     if (!(bx && bb == 4)) {
         double wide = 0.0;
         int wt = bt;
@@ -1383,18 +1384,6 @@ int tam_tune_mc(tam_ctx* c, int64_t sample, int32_t* blocks_per_cu, int32_t* rng
             bx = box_on;
             best = wide;
         }
-    }
-    // With the CU-wide box, a random-phase batch of 32 is kept when it times
-    // within kBatchMargin of the fastest batch: on fresh tissue the batches
-    // 8-48 tie within the timing noise, while in the c1 crater phase 24-32
-    // run fastest (318 ms per 1e8 packets against 348 ms at 8 and 353 at 48).
-    if (bx && bb == 4 && bt != 32) {
-        for (size_t q = 0; q < rates.size(); ++q)
-            if (rates[q].box && rates[q].bpc == 4 && rates[q].batch == 32 &&
-                rates[q].rate >= (1.0 - kBatchMargin) * best) {
-                bt = 32;
-                best = rates[q].rate;
-            }
     }
     c->mc_bpc = bb;
     c->mc_batch = bt;
