@@ -361,8 +361,15 @@ def transport_state_leg(args, log):
     prob = configs.config1(n=(n, n, n), packets=int(args.packets), steps=10000, cycles=3)
     d = np.load(args.state[1])
     g = lib.TissueGrid(prob.params)
-    g.set_optics(prob.mat, prob.table, d["rhokap"])              # removed voxels: rhokap 0
-    g.set_thermal(d["temp"], d["kappa"], d["density"], d["heatcap"])
+    g.set_optics(prob.mat, prob.table)
+    # the state's removed voxels go as in a run, by a rebuild that finds them too
+    # hot, so that the transport finds mu_t as it does there (by the material)
+    gone = np.zeros(d["temp"].shape, bool)
+    gone[1:-1, 1:-1, 1:-1] = d["rhokap"].reshape(gone.shape)[1:-1, 1:-1, 1:-1] == 0.0
+    g.set_thermal(np.where(gone, prob.params.ablate_K + 10.0, np.minimum(d["temp"], prob.params.ablate_K - 1.0)),
+                  prob.kappa, prob.density, prob.heatcap)
+    g.rebuild()
+    assert np.array_equal(g.download(lib.FIELD_RHOKAP).reshape(gone.shape) == 0.0, d["rhokap"].reshape(gone.shape) == 0.0)
     bpc, batch = (int(x) for x in args.mc_launch.split(":"))
     g.set_mc_launch(bpc, batch)
     g.set_mc_box(True)
