@@ -603,9 +603,9 @@ __device__ __forceinline__ T* uni(T* q)
 //   smaller dT; the exact tests follow inside.  Loads of the next plane go out
 //   after the class loads of mixed waves, which would otherwise wait for them
 //   (loads return in order).
-// us a step, before and after: 200^3 skin, late state, 32x16 kz 8: 39.4, 34.3
-// (without damage 31.0, 25.7); 256^3 kz 16: 80.3, 69.6; 113x97x101 kz 4: 7.6,
-// 6.7.  VALU instructions per wave and plane 157, 110; L1 accesses 12.8e6,
+// us a step, before and after: 200^3 skin with a crater, kz 8: 39.4, 34.9
+// (without damage 31.0, 25.7); 256^3 kz 16: 80.0, 70.1; 113x97x101 kz 4: 7.3,
+// 6.5.  VALU instructions per wave and plane 157, 110; L1 accesses 12.8e6,
 // 8.4e6 a launch at 200^3.  At most 64 VGPRs (8 waves a SIMD) gave 66.9 at 256^3
 // but 35.6 and 7.2 at the other two; two copies of the loop body with the
 // registers renamed instead of moved gave nothing.

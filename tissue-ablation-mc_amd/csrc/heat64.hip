@@ -25,8 +25,8 @@ __device__ __forceinline__ double wave_sum_d(double v)
     return v;
 }
 
-// One thread per voxel; bound by the FP64 fields it streams (dT, three face
-// coefficients, coeff, jmean: about 40 MB at 80^3).  The energy through the
+// One thread per voxel; bound by the FP64 fields it streams (T in and out, three
+// face coefficients, coeff, jmean: 56 bytes a voxel, 29 MB at 80^3).  The energy through the
 // grid's faces goes to the block's own slot, which only this block writes in a
 // launch: on a grid of 80^3 nearly every wave holds a boundary voxel, and 8000
 // FP64 adds to one address took 95 us of the step's 102 us at 12 ns each.

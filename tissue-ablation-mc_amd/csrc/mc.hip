@@ -33,14 +33,17 @@
 //    crossing loads the material's byte and takes mu_t from the table in LDS,
 //    and an event loads nothing: 8 MB instead of 40 MB of grid at 200^3, of
 //    which each XCD's 4 MB L2 holds the part under the beam.
-//  * What bounds it: issue and latency of the loop itself (with its device
-//    adds left out it takes 6-7% less); a short run, the chain of events of
+//  * What bounds it: on fresh tissue, whose deposits the LDS box takes, issue
+//    and latency of the loop (1e8 packets on the 200^3 skin, 3.4 device adds a
+//    packet: 59.5 ms, 57.0 with the device adds left out); past a crater or in
+//    a wide beam, the device adds (the same skin after 3 cycles, 52.9 a packet:
+//    271 ms at 2.0e10 adds/s, 162 without them); a short run, the chain of events of
 //    its longest packets.  The pass as straight code with selects, the
 //    absorbed packets' tally merged into the pass, LDS counts of rare ends,
 //    the byte loads, and no draws from a drained queue took 1e8 packets on the
-//    cratered 200^3 skin from 187 to 164-173 ms (31 device adds a packet,
-//    1.9e10/s), 3e7 on the fresh skin from 27.5 to 19.8, 1e6 at 100^3 from 7.1
-//    to 5.4 (one 1024-lane block a CU, random-phase batch 32).
+//    fresh skin from 82 to 59.5 ms, on the crater with 31 device adds a packet from
+//    187 to 160, with 54 from 306.6 to 304.8 (one card; another 271), 1e6 at
+//    100^3 from 7.0 to 4.6 (one 1024-lane block a CU).
 //  * Tally: path length is summed in a register while the packet stays in a
 //    voxel and written with one FP64 atomic add per voxel visit (at exit or
 //    absorption).  The absorbed fraction per voxel is mu_a * L.  Voxels with
@@ -117,7 +120,10 @@ constexpr int kBoxUnitBits = 13;            // fixed-point box unit: 2^-13 of dx
 constexpr long kLdsOwn = 1024;              // LDS per block kept for the kernel's own use (counts, material table)
 constexpr long kCountLds = sizeof(unsigned long long) * TAM_CNT_N;     // a block's counts, static
 constexpr int kTabMax = 64;                 // materials in the LDS of a kernel without the box
-constexpr int kBatchTab = 4;                // materials per wave in a batched block's own LDS
+// Entries per wave in a batched block's own LDS: what kLdsOwn holds beside the
+// counts.  Tissues of more entries take mu_t from the array as before (eight of
+// four materials and air, 4 blocks a CU: 44.5 ms; with one material 43.8).
+constexpr int kBatchTab = 4;
 constexpr long kBatchLds = 4 * (kCountLds + kBatchTab * (long)sizeof(MatEntry));   // a batched block's static LDS
 static_assert(kCountLds <= kLdsOwn && kBatchLds <= kLdsOwn, "the boxes leave kLdsOwn bytes of a block's LDS");
 
@@ -278,7 +284,7 @@ __device__ __forceinline__ void transport(const McArgs& a, BT* box, const BoxGeo
     float t = 0.f;                             // distance travelled from the origin
     float Tx = 0.f, Ty = 0.f, Tz = 0.f;        // distance from the origin to the next face per axis
     float ux = 0.f, uy = 0.f, uz = -1.f;
-    float sx = 0.f, sy = 0.f, sz = 0.f;        // path across one voxel per axis (0 where u == 0)
+    float sx = 0.f, sy = 0.f, sz = 0.f;        // path across one voxel per axis (unused where u == 0)
     float tau = 0.f, lacc = 0.f;               // optical depth left; path in this voxel
     float nin = 1.f, nout = 1.f;               // indices at a pending Fresnel test
 
@@ -472,8 +478,7 @@ __device__ __forceinline__ void transport(const McArgs& a, BT* box, const BoxGeo
                         // crossing (or a dead packet's last tally)
                         ++nev;
                         lacc += s;
-                        // mu_t = 0 (ablated): nothing is absorbed, and the atomic
-                        // unit's throughput is what bounds this kernel
+                        // mu_t = 0 (ablated): nothing is absorbed, and an add costs
                         if (mu > 0.f) {
                             c_box += tally_add<BOX, BT>(a, box, g, v, ci, cj, ck, lacc, pa);
                             ++c_tally;
