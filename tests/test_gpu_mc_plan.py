@@ -1,6 +1,6 @@
-"""The LDS box of a transport run on the device: a run whose packets justify
-fewer blocks a CU than its launch shape names gets the larger box that those
-leave room for, and the tuner launches a shape's own blocks on its samples."""
+"""The LDS box of a transport run on the device: it is its launch shape's, whether
+the packets justify all of the shape's blocks or fewer, in the runs and in the
+tuner's samples; and the material tables beside it."""
 import numpy as np
 import pytest
 
@@ -8,16 +8,17 @@ from tam_amd import configs, lib
 
 pytestmark = pytest.mark.gpu
 
-ONE, TWO, THREE = (42, 42, 46), (34, 34, 34), (28, 28, 34)          # boxes of one, two, three blocks a CU
+ONE, TWO, THREE, SIX = (42, 42, 46), (34, 34, 34), (28, 28, 34), (22, 22, 27)     # boxes by blocks a CU
 
 
 def _grid():
     return configs.three_layer_skin(n=(64, 64, 64), ext=(0.5, 0.5, 0.25), packets=1, steps=1).grid()
 
 
-@pytest.mark.parametrize("shape,packets,box", [(8, 1_000_000, ONE), (6, 1_000_000, ONE), (4, 1_000_000, ONE),
-                                               (3, 1_000_000, THREE), (2, 1_000_000, TWO), (8, 8_388_608, TWO)])
-def test_box_of_the_blocks_that_run(shape, packets, box):
+@pytest.mark.parametrize("shape,packets,box", [(8, 200_000, TWO), (8, 1_000_000, TWO), (6, 1_000_000, SIX),
+                                               (4, 1_000_000, ONE), (3, 1_000_000, THREE), (2, 1_000_000, TWO),
+                                               (8, 8_388_608, TWO)])
+def test_box_of_the_shape(shape, packets, box):
     print("case", shape, packets, box, flush=True)
     g = _grid()
     g.set_mc_box(False)

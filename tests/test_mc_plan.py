@@ -1,6 +1,6 @@
 """The transport's launch plan (host arithmetic, CPU only): a run's blocks are
-chosen in waves per CU whatever the block size, and the LDS box is sized for
-the blocks that are launched."""
+chosen in waves per CU whatever the block size, and the LDS box is the launch
+shape's whatever the packets."""
 import ctypes as C
 import random
 
@@ -37,8 +37,9 @@ def test_short_box_runs_keep_sixteen_waves_a_cu(shape, packets):
     if packets >= 4096 * NCU * shape:                           # 1024 packets for each wave of the shape
         assert waves(p) == 4 * shape
     assert waves(p) <= max(16, packets / (1024 * NCU))
-    # the box is sized for the blocks that run
-    assert p["blocks"] == NCU * p["per_cu"]
+    # the box is the shape's, and so is what is rounded to its units
+    assert {k: p[k] for k in ("lanes", "per_cu", "sd", "d", "ntab", "lds")} == \
+        {k: plan(10 ** 9, shape=shape)[k] for k in ("lanes", "per_cu", "sd", "d", "ntab", "lds")}
     share = LDS // p["per_cu"] - 1024
     assert p["sd"] == int((share // 2) ** (1 / 3)) & ~1
     assert 2 * p["sd"] ** 2 * (p["d"] + 1) > share >= 2 * p["sd"] ** 2 * p["d"]

@@ -881,8 +881,8 @@ hipError_t mc_prepare(int dev)
                                lds_blk - (int)kBatchLds);
 }
 
-// The launch of a transport run: its blocks first, then the LDS box and table
-// that so many blocks a CU leave room for.
+// The launch of a transport run: box or not, how many blocks, and where the
+// material table lies.
 McPlan mc_plan(const McArgs& a, const McDevice& dev)
 {
     McPlan p{};
@@ -893,26 +893,27 @@ McPlan mc_plan(const McArgs& a, const McDevice& dev)
     // the box: clearing and flushing the box would cost more than it saves.
     const bool few = (double)a.npk < 64.0 * (double)dev.ncu * shape;
     if (a.box_enable && !few) {
+        // a multiple of 4 runs as bpc / 4 blocks of 1024 lanes: the same waves
+        // per CU, one box per 16 waves
+        const bool wide = shape % 4 == 0;
+        p.lanes = wide ? 1024 : 256;
+        p.per_cu = wide ? shape / 4 : shape;
         // A block's box costs a clearing and a device add per touched voxel,
         // and waves that share a SIMD slow each other's longest packets: 16
         // waves a CU (all of a smaller shape's), further ones where each has
         // 1024 packets (8 blocks of 256 lanes a CU at 100^3: 3e6 packets 12.7
         // ms on 256 blocks of 1024 lanes, 13.9 on 512; 1e7 39.3 on both).  In
         // waves, so that 256-lane blocks fill a CU too: 1e6 packets at 100^3,
-        // shapes 2, 3, 6, 8: 5.0, 5.7, 4.6, 4.6 ms; with one block a CU of
-        // whatever size, its box that of the shape, 6.7, 6.8, 6.7, 5.3.
-        int bpc = shape;
-        const int64_t justified = (int64_t)(a.npk / ((uint64_t)dev.ncu * 4096u));
-        if (!a.full_grid && justified < shape) bpc = std::min(shape, std::max(4, (int)justified & ~3));
-        // a multiple of 4 runs as bpc / 4 blocks of 1024 lanes: the same waves
-        // per CU, one box per 16 waves
-        const bool wide = bpc % 4 == 0;
-        p.lanes = wide ? 1024 : 256;
-        p.per_cu = wide ? bpc / 4 : bpc;
-        p.blocks = (int64_t)dev.ncu * p.per_cu;
-        // LDS tally box: the blocks of a CU share its LDS (160 KiB on
-        // MI355X, also the most one block may take), 1 KiB per block kept for
-        // the kernel's own use: with 16-bit sums 42^2 x 46 voxels at 1 block per CU
+        // shapes 2, 3, 6: 5.0, 5.6, 6.3 ms; with one block a CU of whatever size
+        // 6.7, 6.8, 6.7.
+        const int64_t all = (int64_t)dev.ncu * p.per_cu, wave_blocks = p.lanes / 64;
+        const int64_t justified = (int64_t)(a.npk / (uint64_t)(wave_blocks * 1024));
+        const int64_t least = (int64_t)dev.ncu * (16 / wave_blocks);
+        p.blocks = a.full_grid ? all : std::min(all, std::max(least, justified));
+        // LDS tally box: the shape's blocks of a CU share its LDS (160 KiB on
+        // MI355X, also the most one block may take; a run of fewer blocks keeps
+        // the shape's box, since the deposits that are rounded to its units are
+        // part of the result), 1 KiB per block kept for the kernel's own use: with 16-bit sums 42^2 x 46 voxels at 1 block per CU
         // (1 or 4 blocks_per_cu), 34^2 x 34 at 2 (2 or 8), 28^2 x 34 at 3; with
         // FP64 27^3, 21^3, 18^2 x 20.  The cube sits on the beam axis (its x edge
         // even with 16-bit sums, so the two voxels of a word share a row).  Its z range is where
