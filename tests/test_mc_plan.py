@@ -94,15 +94,38 @@ def test_no_plan_asks_for_more_lds_than_is_allowed():
             assert -(-(p["lds"] + COUNTS) // step) * step * p["per_cu"] <= LDS, q
 
 
+def batch_slots(grids, shape):
+    """(slots a wave asks for, each grid's cube)"""
+    n = len(grids)
+    edges, cube = (C.c_int32 * (3 * n))(*[e for g in grids for e in g]), (C.c_int32 * (2 * n))()
+    slots = lib.load().tam_internal_batch_slots(edges, n, NCU, LDS, LDS, shape, cube)
+    return slots, [tuple(cube[2 * i:2 * i + 2]) for i in range(n)]
+
+
 @pytest.mark.parametrize("shape", range(1, 65))
+def test_batched_cubes_fit_their_slices(shape):
+    rng = random.Random(shape)
+    most = min(LDS - 1024, LDS // shape - 1024) // 8 & ~7 if LDS // shape > 1024 else 0
+    for _ in range(50):
+        grids = [tuple(rng.randint(1, 200) for _ in range(3)) for _ in range(rng.randint(1, 6))]
+        slots, cubes = batch_slots(grids, shape)
+        assert slots % 8 == 0 and slots <= most
+        for (nx, ny, nz), (sd, d) in zip(grids, cubes):
+            assert sd * sd * d <= slots and sd <= min(nx, ny) and d <= nz
+            assert sd < 2 or sd % 2 == 0
+            # the largest: neither edge could be longer
+            assert d == nz or sd * sd * (d + 1) > most
+            assert sd >= min(nx, ny) - 1 or (sd + 2) ** 3 > most
+        assert slots == -(-max(sd * sd * d for sd, d in cubes) // 8) * 8
+
+
+@pytest.mark.parametrize("shape", [1, 2, 3, 4, 8])
 def test_batched_blocks_of_a_cu_find_their_lds(shape):
-    slots = lib.load().tam_internal_batch_slots(NCU, LDS, LDS, shape)
-    assert slots % 8 == 0 and slots >= 0
+    """Cubes of ordinary tissues leave the counts and tables of every block of a CU their LDS."""
+    slots, _ = batch_slots([(64, 64, 64), (96, 96, 96), (160, 160, 160)], shape)
     static, step = 4 * (COUNTS + 4 * 32), LDS // 128            # a wave's counts and four materials, four times
     block = static + 4 * 2 * slots
     assert block <= LDS and -(-block // step) * step * shape <= LDS
-    # and little of it stays idle: a step, the 1 KiB left beside the box, the rounding to 8 slots a wave
-    assert block > LDS // shape - step - 1024 - 64
 
 
 @pytest.mark.parametrize("w", [4, 1024, 4096, 8192])

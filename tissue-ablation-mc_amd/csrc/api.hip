@@ -1562,7 +1562,7 @@ int batch_mc(tam_batch* b, const int64_t* npk, uint64_t seed, uint32_t stream0, 
     }
     BCHK(b, hipMemcpyAsync(b->dmc, tab.data(), sizeof(McArgs) * (size_t)n, hipMemcpyHostToDevice, b->stream));
     BCHK(b, hipEventRecord(b->ev0, b->stream));
-    BCHK(b, launch_mc_batch(b->dmc, n, total, b->bpc, b->stream));
+    BCHK(b, launch_mc_batch(tab.data(), b->dmc, n, total, b->bpc, b->stream));
     BCHK(b, hipEventRecord(b->ev1, b->stream));
     BCHK(b, hipStreamSynchronize(b->stream));
     b->last_ms = bms(b);

@@ -701,22 +701,39 @@ __global__ __launch_bounds__(256) void box_window_kernel(const double* __restric
     }
 }
 
+// The cube of at most wbox voxels that a batched wave sums in LDS: inside the grid
+// (sd <= nx, ny; d <= nz)
+struct BatchCube {
+    int sd, d;
+};
+__host__ __device__ inline BatchCube batch_cube(int nx, int ny, int nz, int wbox)
+{
+    int sd = (int)cbrtf((float)wbox);
+    while ((long)(sd + 1) * (sd + 1) * (sd + 1) <= wbox) ++sd;
+    while (sd > 1 && (long)sd * sd * sd > wbox) --sd;
+    sd = sd < nx ? sd : nx;
+    sd = sd < ny ? sd : ny;
+    if (sd > 1) sd &= ~1;                                  // the two voxels of a word share a row
+    const int d = wbox / (sd * sd);
+    return BatchCube{sd, d < nz ? d : nz};
+}
+
 // Many instances in one launch: a wave takes packets from one instance's
 // queue until it drains, then moves on to the next instance (starting at its
 // own index, so the waves spread over the instances); each instance keeps its
 // own queue, tally and counters, and the instance's arguments stay uniform
-// over the wave.  With wbox > 0 each wave owns an LDS slice of wbox 16-bit
-// fixed-point voxels: for every instance it works on (with the box enabled,
+// over the wave.  With wbox > 0 each wave owns an LDS slice of 16-bit
+// fixed-point voxels (slots: the largest cube of the instances): for every instance it works on (with the box enabled,
 // of either kind) it sums its
 // visits to a cube under the top face on that instance's beam axis there,
 // and adds the cube to the instance's tally when it moves on.  The waves of
 // a block work on different instances, so the slices are per wave and only
 // wave-level ordering is needed.
-__global__ __launch_bounds__(256) void mc_batch_kernel(const McArgs* __restrict__ tab, int n, int wbox)
+__global__ __launch_bounds__(256) void mc_batch_kernel(const McArgs* __restrict__ tab, int n, int wbox, int slots)
 {
     extern __shared__ __attribute__((aligned(16))) unsigned char lds_slices[];
-    // wbox is a multiple of 8, so every slice starts on a 16-byte boundary
-    uint16_t* box = reinterpret_cast<uint16_t*>(lds_slices) + (size_t)(threadIdx.x >> 6) * (size_t)wbox;
+    // slots is a multiple of 8, so every slice starts on a 16-byte boundary
+    uint16_t* box = reinterpret_cast<uint16_t*>(lds_slices) + (size_t)(threadIdx.x >> 6) * (size_t)slots;
     // per wave: counts of the current instance and its material table
     __shared__ unsigned long long wsums[4][TAM_CNT_N];
     __shared__ __attribute__((aligned(16))) MatEntry wtab[4][kBatchTab];
@@ -734,13 +751,8 @@ __global__ __launch_bounds__(256) void mc_batch_kernel(const McArgs* __restrict_
             continue;
         BoxGeom g{};
         if (wbox > 0 && a.box_enable) {
-            // a cube of at most wbox voxels inside the grid (sd <= nx, ny; d <= nz)
-            int sd = (int)cbrtf((float)wbox);
-            while ((long)(sd + 1) * (sd + 1) * (sd + 1) <= wbox) ++sd;
-            while (sd > 1 && (long)sd * sd * sd > wbox) --sd;
-            sd = min(sd, min(a.nx, a.ny));
-            if (sd > 1) sd &= ~1;                          // the two voxels of a word share a row
-            const int d = min(a.nz, wbox / (sd * sd));
+            const BatchCube q = batch_cube(a.nx, a.ny, a.nz, wbox);
+            const int sd = q.sd, d = q.d;
             g.n[0] = g.n[1] = sd;
             g.n[2] = d;
             g.o[0] = max(0, min((int)lroundf(a.cx / a.dx) - sd / 2, a.nx - sd));
@@ -820,24 +832,50 @@ McDevice mc_device()
     return d;
 }
 
-// 16-bit slots of a batched wave's LDS tally box: a quarter of its block's share
-// of the CU's LDS, less 1 KiB for the kernel's own use, in whole steps in which
-// LDS is given out (a share of lds_cu / 3 or / 5 is not: with the counts and
-// tables in it 2 blocks a CU were resident instead of 3, 4 instead of 5: eight
-// tissues of four materials 46.3 ms at 3 a CU, 42.2 now; of one 41.5, 40.9)
+// 16-bit slots that a batched wave's cube may have: a quarter of its block's share
+// of the CU's LDS, less 1 KiB for the kernel's own use, a multiple of 8
 int mc_batch_slots(const McDevice& dev, int bpc)
 {
-    const long step = dev.lds_cu / 128, whole = 128 / bpc * step;
-    const long box = std::min({(long)dev.lds_blk - kLdsOwn, (long)dev.lds_cu / bpc - kLdsOwn, whole - kBatchLds});
-    return box > 0 ? (int)(box / 4 / 2) & ~7 : 0;              // a multiple of 8 per wave
+    const long per_block = std::min((long)dev.lds_blk - kLdsOwn, (long)dev.lds_cu / bpc - kLdsOwn);
+    return per_block > 0 ? (int)(per_block / 4 / 2) & ~7 : 0;
 }
 
-extern "C" int tam_internal_batch_slots(int ncu, int lds_cu, int lds_blk, int bpc)
+// The slots of a launch's largest cube, a multiple of 8: what the launch asks for,
+// so that the counts and tables of a block (960 bytes) come in beside it.  LDS is
+// given out in steps of 1280 bytes; with all of a third of a CU's LDS but 1 KiB asked for,
+// 2 blocks a CU were resident instead of 3 (eight tissues of four materials
+// 46.3 ms at 3 a CU, 42.2 so; of one 41.5, 40.9).
+int mc_batch_cube(const McArgs* tab, int n, int wbox)
 {
-    return mc_batch_slots(McDevice{ncu, lds_cu, lds_blk}, bpc);
+    long most = 0;
+    for (int i = 0; i < n; ++i)
+        if (wbox > 0 && tab[i].npk > 0 && tab[i].box_enable) {
+            const BatchCube q = batch_cube(tab[i].nx, tab[i].ny, tab[i].nz, wbox);
+            most = std::max(most, (long)q.sd * q.sd * q.d);
+        }
+    return (int)((most + 7) & ~7L);
 }
 
-hipError_t launch_mc_batch(const McArgs* dtab, int n, long total_npk, int blocks_per_cu, hipStream_t s)
+extern "C" int tam_internal_batch_slots(const int32_t* edges, int n, int ncu, int lds_cu, int lds_blk, int bpc,
+                                        int32_t* cube)
+{
+    std::vector<McArgs> tab((size_t)n);
+    const int wbox = mc_batch_slots(McDevice{ncu, lds_cu, lds_blk}, bpc);
+    for (int i = 0; i < n; ++i) {
+        McArgs& a = tab[(size_t)i];
+        a = McArgs{};
+        a.npk = 1;
+        a.box_enable = 1;
+        a.nx = edges[3 * i]; a.ny = edges[3 * i + 1]; a.nz = edges[3 * i + 2];
+        const BatchCube q = wbox > 0 ? batch_cube(a.nx, a.ny, a.nz, wbox) : BatchCube{0, 0};
+        cube[2 * i] = q.sd;
+        cube[2 * i + 1] = q.d;
+    }
+    return mc_batch_cube(tab.data(), n, wbox);
+}
+
+hipError_t launch_mc_batch(const McArgs* tab, const McArgs* dtab, int n, long total_npk, int blocks_per_cu,
+                           hipStream_t s)
 {
     if (n <= 0 || total_npk <= 0) return hipSuccess;
     const McDevice dev = mc_device();
@@ -845,9 +883,9 @@ hipError_t launch_mc_batch(const McArgs* dtab, int n, long total_npk, int blocks
     long blocks = (long)dev.ncu * bpc;
     const long need = (total_npk + 255) / 256;
     if (need < blocks) blocks = need;
-    const int wbox = mc_batch_slots(dev, bpc);
-    const size_t lds = sizeof(uint16_t) * 4 * (size_t)wbox;
-    hipLaunchKernelGGL(mc_batch_kernel, dim3((unsigned)blocks), dim3(256), lds, s, dtab, n, wbox);
+    const int wbox = mc_batch_slots(dev, bpc), slots = mc_batch_cube(tab, n, wbox);
+    const size_t lds = sizeof(uint16_t) * 4 * (size_t)slots;
+    hipLaunchKernelGGL(mc_batch_kernel, dim3((unsigned)blocks), dim3(256), lds, s, dtab, n, wbox, slots);
     return hipGetLastError();
 }
 

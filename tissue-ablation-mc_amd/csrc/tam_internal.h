@@ -379,9 +379,12 @@ hipError_t mc_prepare(int dev);
 // the fixed-point LDS box's unit for a's voxel size (box_scale, box_quantum)
 void mc_box_units(McArgs& a);
 int mc_batch_slots(const McDevice& dev, int bpc);
-extern "C" int tam_internal_batch_slots(int ncu, int lds_cu, int lds_blk, int bpc);     // host only
-// all instances of a device table in one launch (see mc_batch_kernel)
-hipError_t launch_mc_batch(const McArgs* dtab, int n, long total_npk, int blocks_per_cu, hipStream_t s);
+// slots of a batch of grids (edges: nx, ny, nz each); cube: (sd, d) of each; host only
+extern "C" int tam_internal_batch_slots(const int32_t* edges, int n, int ncu, int lds_cu, int lds_blk, int bpc,
+                                        int32_t* cube);
+// all instances of a table (host and device copy) in one launch (see mc_batch_kernel)
+hipError_t launch_mc_batch(const McArgs* tab, const McArgs* dtab, int n, long total_npk, int blocks_per_cu,
+                           hipStream_t s);
 // `count` FP64 atomic adds (whole waves) to pseudo-random slots of t[0, slots)
 hipError_t launch_atomic_rate(double* t, long slots, long count, hipStream_t s);
 hipError_t launch_heat_step(const HeatArgs& a, const float* Tin, float* Tout, float lon, double time_after,
