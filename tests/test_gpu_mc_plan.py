@@ -105,3 +105,31 @@ def test_batched_tissues_of_several_materials(materials, shape):
         unit = 2.0 * (p.xmax / p.nx + p.ymax / p.ny + p.zmax / p.nz) / 2 ** 13
         np.testing.assert_allclose(tb[i], t1, rtol=1e-4, atol=16 * unit)
         g.close()
+
+
+def test_batched_grids_one_voxel_wide():
+    """Without a box: a word of the 16-bit box holds two x neighbours, and its
+    carry goes to the second."""
+    sizes = [(1, 20, 33), (24, 1, 40), (1, 1, 61), (30, 30, 30)]
+    print("case: batch of", sizes, flush=True)
+    probs = []
+    for n in sizes:
+        prob = configs.three_layer_skin(n=n, ext=(0.2, 0.2, 0.5), packets=1, steps=1)
+        prob.params.damage_every_step = 0
+        probs.append(prob)
+    gs = [p.grid() for p in probs]
+    b = lib.Batch(gs)
+    npk = [40_000, 30_000, 50_000, 20_000]
+    st = b.mc_run(npk, seed=6, stream0=2)
+    tb = [g.download(lib.FIELD_TALLY) for g in gs]
+    b.close()
+    for i, g in enumerate(gs):
+        assert (st[i].box_adds > 0) == (min(sizes[i][:2]) > 1)
+        g.set_mc_box(False)
+        s1 = g.mc_run(npk[i], seed=6, stream=2 + i)
+        t1 = g.download(lib.FIELD_TALLY)
+        for k in ("absorbed", "specular", "missed", "killed", "crossings", "interactions", "tally_adds"):
+            assert getattr(st[i], k) == getattr(s1, k), (i, k)
+        if min(sizes[i][:2]) == 1:
+            np.testing.assert_allclose(tb[i], t1, rtol=1e-9, atol=1e-9 * t1.max())
+        g.close()

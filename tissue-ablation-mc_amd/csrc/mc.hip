@@ -702,7 +702,7 @@ __global__ __launch_bounds__(256) void box_window_kernel(const double* __restric
 }
 
 // The cube of at most wbox voxels that a batched wave sums in LDS: inside the grid
-// (sd <= nx, ny; d <= nz)
+// (sd <= nx, ny; d <= nz); none on a grid one voxel wide
 struct BatchCube {
     int sd, d;
 };
@@ -713,7 +713,10 @@ __host__ __device__ inline BatchCube batch_cube(int nx, int ny, int nz, int wbox
     while (sd > 1 && (long)sd * sd * sd > wbox) --sd;
     sd = sd < nx ? sd : nx;
     sd = sd < ny ? sd : ny;
-    if (sd > 1) sd &= ~1;                                  // the two voxels of a word share a row
+    // the two voxels of a word share a row; a grid one voxel wide has no such
+    // pair (a carry would go past its column, and past its tally at the top)
+    sd &= ~1;
+    if (sd < 2) return BatchCube{0, 0};
     const int d = wbox / (sd * sd);
     return BatchCube{sd, d < nz ? d : nz};
 }
