@@ -42,8 +42,8 @@
 //    absorbed packets' tally merged into the pass, LDS counts of rare ends,
 //    the byte loads, and no draws from a drained queue took 1e8 packets on the
 //    fresh skin from 82 to 59.5 ms, on the crater with 31 device adds a packet from
-//    187 to 160, with 54 from 306.6 to 304.8 (one card; another 271), 1e6 at
-//    100^3 from 7.0 to 4.6 (one 1024-lane block a CU).
+//    187 to 160, with 54 from 306.6 to 304.8 (another card 10 % less), 1e6 at
+//    100^3 from 6.5 to 4.6 (one 1024-lane block a CU).
 //  * Tally: path length is summed in a register while the packet stays in a
 //    voxel and written with one FP64 atomic add per voxel visit (at exit or
 //    absorption).  The absorbed fraction per voxel is mu_a * L.  Voxels with
