@@ -52,6 +52,18 @@ def test_tuner_samples_run_the_whole_shape(shape):
         assert plan(packets, shape=shape, full=1) == long_run
 
 
+@pytest.mark.parametrize("shape", [1, 2, 3, 4, 6, 8, 16])
+@pytest.mark.parametrize("packets", [1, 4097, 20_000, 140_000, 400_000, 1_000_000, 3_000_000, 8_400_000, 20_000_000, 10 ** 8])
+def test_runs_without_the_box_keep_sixteen_waves_a_cu(shape, packets):
+    p = plan(packets, shape=shape, box=0)
+    assert (p["box"], p["lanes"]) == (0, 256)
+    most = 4 * shape
+    assert waves(p) <= min(most, max(16, packets / (1024 * NCU))) + 4 / NCU
+    assert waves(p) >= min(most, max(min(16, packets / (64 * NCU)), min(8, packets / (4 * NCU)), packets // 1024 / NCU))
+    # the tuner's samples stand for longer runs
+    assert plan(packets, shape=shape, box=0, full=1)["blocks"] == NCU * shape
+
+
 def test_box_leaves_the_lds_that_its_blocks_need():
     rng = random.Random(5)
     for _ in range(4000):

@@ -994,13 +994,19 @@ McPlan mc_plan(const McArgs& a, const McDevice& dev)
     // 4; past that every wave starts with a full set of lanes.  20 000
     // packets at 64^3: 1.35 ms, against 2.7 ms on full waves alone
     // (1.6 at 4 waves a CU, 1.35 at 16); 125 000 packets of a pure
-    // absorber: 40 us, against 68 (44 at 16 waves a CU).
+    // absorber: 40 us, against 68 (44 at 16 waves a CU).  Past 16 waves a CU
+    // each has 1024 packets, as with the box: 400 000 packets at shape 8 on a
+    // 37x51x45 and a 100^3 cube and on the 200^3 skin 3.4, 4.8 and 2.8 ms,
+    // against 4.1, 5.4 and 2.9 on a wave per 64 packets; of the pure absorber,
+    // whose packets are then drawn, 0.15 against 0.11.
     p = McPlan{};
     p.lanes = 256;
     p.per_cu = shape;
-    const int64_t waves = std::max((int64_t)((a.npk + 63) / 64),
-                                   std::min((int64_t)8 * dev.ncu, (int64_t)((a.npk + 3) / 4)));
-    p.blocks = std::min((int64_t)dev.ncu * shape, (waves + 3) / 4);
+    auto up = [](uint64_t n, uint64_t d) { return (int64_t)(n / d + (n % d != 0)); };
+    const int64_t all = (int64_t)dev.ncu * shape;
+    const int64_t waves = std::max({std::min(up(a.npk, 4), (int64_t)8 * dev.ncu),
+                                    std::min(up(a.npk, 64), (int64_t)16 * dev.ncu), up(a.npk, 1024)});
+    p.blocks = a.full_grid ? all : std::min(all, up((uint64_t)waves, 4));
     p.ntab = a.mut_by_mat && a.nmat <= kTabMax ? a.nmat : 0;
     p.lds = (int64_t)sizeof(MatEntry) * p.ntab;
     return p;
