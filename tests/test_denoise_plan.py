@@ -1,5 +1,7 @@
 """The denoiser's weight-gradient launch (host arithmetic, CPU only): one round
 of the blocks that the device holds at once, each with as many bricks."""
+import ctypes as C
+
 import pytest
 
 from tam_amd import lib
@@ -17,3 +19,10 @@ def test_one_round_of_resident_blocks(ncu, n, cin, cout, rows):
     per = blocks // rows
     each = -(-bricks // per)
     assert per <= bricks and each <= -(-bricks // max(1, held // rows))     # no block has more than its share
+
+
+def test_host_functions_start_a_cache_line():
+    """Where they fall in one sets how fast the weights are drawn."""
+    L = lib.load()
+    for name in lib.EXPORTED + ("tam_dn_create",):
+        assert C.cast(getattr(L, name), C.c_void_p).value % 64 == 0, name
